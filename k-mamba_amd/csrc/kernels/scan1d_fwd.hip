@@ -28,6 +28,7 @@
 //    follow the per-step clamp exactly.
 #include <algorithm>
 #include <cstdlib>
+#include <mutex>
 #include <type_traits>
 
 #include "km_device.hpp"
@@ -54,14 +55,23 @@ struct Scan1DFwdArgs {
     long B, L, D, N;
     long sb, st, sd;
     int clamp;
-    // Segmented launches (the sequence split over workgroups): a workgroup
-    // whose states leave [-1000, 1000] sets clamp_flag[b / nseg * groups +
-    // group] and leaves the sequential re-run to scan1d_clamp_repair, or
-    // null for the workgroup's own fallback.
+    // Segmented launches (the sequence split over workgroups): the grid holds
+    // nseg workgroups per (batch, group), workgroup sg on steps [sg * Ls,
+    // min(L, (sg + 1) * Ls)). nseg = 1 with Ls = L otherwise.
+    int nseg, Ls;
+    // A workgroup of a segmented launch whose states leave [-1000, 1000] sets
+    // clamp_flag[b * groups + group] and leaves the sequential re-run to
+    // scan1d_clamp_repair; null: the workgroup's own fallback.
     int *clamp_flag;
-    long nseg;
-    // [B, D] sum of delta over the sequence (kernels built with DSUM).
-    float *dsum_out;
+    // Segment maps [B, S - 1, D, N] and [B, S - 1, D] of all S segments but
+    // the last: the end state from zero and the sum of delta. Written by the
+    // map pass (DSUM), read by the replay (seg_in).
+    float *seg_h, *seg_dsum;
+    int seg_in;
+    // [B, D, N] copy of h0 the map pass leaves for the replay where h_final
+    // shares h0's memory (the replay's last segment writes it while earlier
+    // segments may not have started), or null.
+    float *h0_copy;
 };
 
 // Output of one step: the readout, plus Dskip*x and times SiLU(z) when
@@ -163,18 +173,22 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
     const int dl = lane % DL;
     const int ns = lane / DL;
     const int n0 = ns * NPL;
-    const long ngroups = (p.D + DL - 1) / DL;
+    const unsigned ngroups = static_cast<unsigned>((p.D + DL - 1) / DL);
     // Workgroups numbered XCD-major: the channel groups of a batch element
     // run on as few XCDs as possible, so its shared B/C rows and (bf16: a
     // group's 32 channels are half of a 128-byte line) its x / delta lines
-    // are fetched into one L2.
-    const long wg = xcd_remap(blockIdx.x, gridDim.x);
-    const long b = wg / ngroups;
-    const long grp = wg - b * ngroups;
-    const long d = grp * DL + dl;
+    // are fetched into one L2. The grid is below 2^31, so 32-bit divisions.
+    const unsigned wg = static_cast<unsigned>(xcd_remap(blockIdx.x, gridDim.x));
+    const unsigned bs = wg / ngroups;                       // (batch element, segment)
+    const unsigned grp = wg - bs * ngroups;
+    const unsigned nseg = static_cast<unsigned>(p.nseg);
+    const long b = bs / nseg;
+    const int seg = static_cast<int>(bs - static_cast<unsigned>(b) * nseg);
+    const long t00 = static_cast<long>(seg) * p.Ls;         // the workgroup's first step
+    const long d = static_cast<long>(grp) * DL + dl;
     const bool dvalid = d < p.D;
     const int dc = static_cast<int>(dvalid ? d : p.D - 1);
-    const int L = static_cast<int>(p.L);
+    const int L = static_cast<int>(min(static_cast<long>(p.Ls), p.L - t00));
     const int Dm = static_cast<int>(p.D);
     const int nit = (L + SC - 1) / SC;
     const bool store_y = dvalid && ns == 0;
@@ -192,17 +206,19 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
     // launcher keeps every window and offset below 1 GiB). Every variable
     // offset goes in the VGPR offset so the hardware range check applies:
     // rows past L load as 0 and their stores are dropped.
-    const long xoff = b * p.L * p.D;
-    const auto rx = make_rsrc(static_cast<const char *>(p.x) + xoff * TS, p.L * p.D * TS);
-    const auto rdt = make_rsrc(static_cast<const char *>(p.dt) + xoff * TS, p.L * p.D * TS);
+    const long xoff = (b * p.L + t00) * p.D;
+    const long xbytes = static_cast<long>(L) * p.D * TS;
+    const auto rx = make_rsrc(static_cast<const char *>(p.x) + xoff * TS, xbytes);
+    const auto rdt = make_rsrc(static_cast<const char *>(p.dt) + xoff * TS, xbytes);
     // y may be null (checkpoint-only forward): a zero-sized window drops the stores.
-    const auto ry = make_rsrc(p.y ? static_cast<char *>(p.y) + xoff * TS : nullptr,
-                              p.y ? p.L * p.D * TS : 0);
+    const auto ry = make_rsrc(p.y ? static_cast<char *>(p.y) + xoff * TS : nullptr, p.y ? xbytes : 0);
     const auto rz = make_rsrc(GATE && p.z ? static_cast<const char *>(p.z) + xoff * TS : nullptr,
-                              GATE && p.z ? p.L * p.D * TS : 0);
-    const auto rB = make_rsrc(static_cast<const char *>(p.Bm) + b * p.sb * TS, p.L * p.st * TS);
-    const auto rC = make_rsrc(static_cast<const char *>(p.Cm) + b * p.sb * TS, p.L * p.st * TS);
-    const auto rh = make_rsrc(p.hist ? p.hist + xoff * p.N : nullptr, HIST ? p.L * p.D * p.N * 4 : 0);
+                              GATE && p.z ? xbytes : 0);
+    const long bcoff = (b * p.sb + t00 * p.st) * TS, bcbytes = static_cast<long>(L) * p.st * TS;
+    const auto rB = make_rsrc(static_cast<const char *>(p.Bm) + bcoff, bcbytes);
+    const auto rC = make_rsrc(static_cast<const char *>(p.Cm) + bcoff, bcbytes);
+    const auto rh = make_rsrc(p.hist ? p.hist + xoff * p.N : nullptr,
+                              HIST ? static_cast<long>(L) * p.D * p.N * 4 : 0);
     const int vx = dc * TS;                             // lane byte offset in an x row
     const int rowx = Dm * TS;                           // bytes per x row
     const int rowbc = static_cast<int>(p.st) * TS;      // bytes per B/C row
@@ -228,6 +244,10 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
         IO::st(r, static_cast<int>(v + static_cast<unsigned>(t * rb)), 0, val);
     };
     const unsigned vhs = dvalid ? static_cast<unsigned>(vh) : kDrop;
+    // The lane's checkpoint of the workgroup's first kCkptSteps steps, and
+    // how many checkpoints its steps have.
+    float *const ckpt0 = p.ckpt ? p.ckpt + ((b * p.nck + t00 / kCkptSteps) * Dm + dc) * N + ns : nullptr;
+    const int nckw = (L + kCkptSteps - 1) / kCkptSteps;
 
     __shared__ float sB[SHARED ? 3 : 1][SHARED ? TILE : 1];
     __shared__ float sC[SHARED ? 3 : 1][SHARED ? TILE : 1];
@@ -254,10 +274,38 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
                      (p.A[dc * N + NS * j + ns] == static_cast<float>(NS * j + ns + 1) * p.A[dc * N]);
     const bool fast = __builtin_amdgcn_readfirstlane(__syncthreads_and(structured)) != 0;
 
-    if (w == 0) {
+    // The state entering the workgroup's steps, state j by wave j (mod W): h0
+    // or, in a replay of segment seg > 0, h0 carried through the maps of the
+    // segments before it, h <- exp(A * sum delta) h + h_end, in order. The
+    // map loads of kFoldRun segments are in flight together.
+    for (int j = w; j < NPL; j += W) {
+        const long hi = (b * Dm + dc) * N + NS * j + ns;
+        float run = (p.h0 && !DSUM) ? p.h0[hi] : 0.f;
+        if constexpr (!DSUM) {
+            if (p.seg_in && seg > 0) {
+                constexpr int kFoldRun = 8;
+                const float a2 = p.A[dc * N + NS * j + ns] * kLog2e;
+                const long m0 = b * (nseg - 1) * Dm + dc;
+                for (int s0 = 0; s0 < seg; s0 += kFoldRun) {
+                    float ds[kFoldRun], hv[kFoldRun];
 #pragma unroll
-        for (int j = 0; j < NPL; ++j)
-            carry[0][j][lane] = p.h0 ? p.h0[(b * Dm + dc) * N + NS * j + ns] : 0.f;
+                    for (int i = 0; i < kFoldRun; ++i) {
+                        const long m = m0 + static_cast<long>(min(s0 + i, seg - 1)) * Dm;
+                        ds[i] = p.seg_dsum[m];
+                        hv[i] = p.seg_h[m * N + NS * j + ns];
+                    }
+#pragma unroll
+                    for (int i = 0; i < kFoldRun; ++i)
+                        if (s0 + i < seg) run = fmaf(exp2_fast(ds[i] * a2), run, hv[i]);
+                }
+            }
+        } else {
+            if (p.h0_copy && seg == 0 && dvalid) p.h0_copy[hi] = p.h0[hi];
+        }
+        carry[0][j][lane] = run;
+    }
+    if constexpr (DSUM) {
+        if (p.clamp_flag && seg == 0 && tid == 0) p.clamp_flag[b * ngroups + grp] = 0;
     }
 
     // B/C tile of super-chunk s: element e = (step, state) at row s*SC + e/N.
@@ -413,9 +461,9 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
                 // final state). Launches with checkpoints use super-chunks
                 // that are multiples of kCkptSteps.
                 if (((v + 1) * TC) % kCkptSteps == 0) {   // folded after unrolling
-                    const long c = (static_cast<long>(s) * SC + (v + 1) * TC) / kCkptSteps - 1;
-                    if (p.ckpt && dvalid && c < p.nck)
-                        p.ckpt[((b * p.nck + c) * Dm + d) * N + NS * j + ns] = run;
+                    const int c = (s * SC + (v + 1) * TC) / kCkptSteps - 1;
+                    if (ckpt0 && dvalid && c < nckw)
+                        ckpt0[static_cast<long>(c) * Dm * N + NS * j] = run;
                 }
             }
             carry[cur ^ 1][j][lane] = run;
@@ -511,15 +559,16 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
                 for (int i = 1; i < W; ++i) dtot += aggP[i][0][lane];
             }
         }
-        if (w == 0 && dvalid && ns == 0) p.dsum_out[b * Dm + d] = dtot;
+        if (w == 0 && dvalid && ns == 0) p.seg_dsum[static_cast<long>(bs) * Dm + d] = dtot;
     }
 
     if constexpr (DSUM) {
         // The segment's local end state is the last super-chunk's outgoing
         // carry (the segment-map pass runs without the clamp).
-        if (w == W - 1 && p.hfin && dvalid) {
+        if (w == W - 1 && dvalid) {
 #pragma unroll
-            for (int j = 0; j < NPL; ++j) p.hfin[(b * Dm + d) * N + NS * j + ns] = carry[nit & 1][j][lane];
+            for (int j = 0; j < NPL; ++j)
+                p.seg_h[(static_cast<long>(bs) * Dm + d) * N + NS * j + ns] = carry[nit & 1][j][lane];
         }
         return;
     }
@@ -533,7 +582,7 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
         if (p.clamp_flag) {
             // A segment of a split sequence: states entering later segments
             // are also off, so the whole sequence is re-run by the repair.
-            if (tid == 0) p.clamp_flag[(b / p.nseg) * ngroups + grp] = 1;
+            if (tid == 0) p.clamp_flag[b * ngroups + grp] = 1;
             return;
         }
         // The sequential pass keeps each lane's states contiguous
@@ -546,7 +595,7 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
         }
         return;
     }
-    if (w == W - 1 && p.hfin && dvalid) {
+    if (w == W - 1 && p.hfin && dvalid && seg == p.nseg - 1) {
 #pragma unroll
         for (int j = 0; j < NPL; ++j) p.hfin[(b * Dm + d) * N + NS * j + ns] = h[j];
     }
@@ -638,55 +687,15 @@ static int launch_n16(const Scan1DFwdArgs &a, bool shared, bool hist, hipStream_
 }
 
 // ---------------------------------------------------------------------------
-// Sequences split over workgroups (few (batch, channel group) pairs, long L):
-// segment s of batch element b is "batch element" b*S + s of a [B*S, Ls, .]
-// view of the same buffers. (1) the chunked kernel runs every segment from a
-// zero state, writing its local end state hl and its sum of delta; (2)
-// scan1d_segment_fold forms each segment's incoming state
-// h_in[s+1] = exp(A * sum delta over s) h_in[s] + hl[s] (and the final
-// state); (3) the chunked kernel replays every segment from its incoming
-// state, writing y. With the per-step clamp, a
-// segment whose states leave [-1000, 1000] flags its (batch, group) and
-// scan1d_clamp_repair re-runs that whole sequence with the sequential
-// clamped recurrence.
+// Sequences split over workgroups (few (batch, channel group) pairs, long L)
+// in segments of Ls steps: (1) the map pass runs every segment but the last
+// from a zero state, writing its end state and its sum of delta; (2) the
+// replay runs every segment from its incoming state, which each workgroup
+// folds from the maps before it (h <- exp(A * sum delta) h + h_end), writing
+// every output. With the per-step clamp, a segment whose states leave
+// [-1000, 1000] flags its (batch, group) and (3) scan1d_clamp_repair re-runs
+// that whole sequence with the sequential clamped recurrence.
 // ---------------------------------------------------------------------------
-
-// One thread per (batch, channel, state) of N = 16 states: the fold over
-// at most kMaxSegments segments, h_in[s+1] = exp(A * dsum[s]) h_in[s] + hl[s].
-// Every segment's operands are loaded before the arithmetic (they do not
-// depend on the state), so the kernel waits for memory once, not once per
-// segment. Also zeroes the clamp flags.
-constexpr int kMaxSegments = 64;
-__global__ void __launch_bounds__(256) scan1d_segment_fold(const float *A, const float *h0,
-                                                           const float *hl, const float *dsum,
-                                                           float *hin, float *hfin, int *flags,
-                                                           long nflags, long B, long D, int nseg) {
-    constexpr int N = 16;
-    const long gid = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (gid < nflags) flags[gid] = 0;
-    if (gid >= B * D * N) return;
-    const long bd = gid / N, n = gid - bd * N;
-    const long b = bd / D, d = bd - b * D;
-    const long base = b * nseg;                      // segment sg is row base + sg of [B*S, D, N]
-    float ds[kMaxSegments], hv[kMaxSegments];
-#pragma unroll
-    for (int sg = 0; sg < kMaxSegments; ++sg) {
-        if (sg < nseg) {
-            ds[sg] = dsum[(base + sg) * D + d];
-            hv[sg] = hl[((base + sg) * D + d) * N + n];
-        }
-    }
-    const float a2 = A[d * N + n] * kLog2e;
-    float h = h0 ? h0[gid] : 0.f;                    // h0 is [B, D, N]: index gid
-#pragma unroll
-    for (int sg = 0; sg < kMaxSegments; ++sg) {
-        if (sg < nseg) {
-            hin[((base + sg) * D + d) * N + n] = h;
-            h = fmaf(exp2_fast(ds[sg] * a2), h, hv[sg]);
-        }
-    }
-    if (hfin) hfin[gid] = h;
-}
 
 // Re-runs every flagged (batch, channel group) sequence from its start with
 // the sequential clamped recurrence (wave 0 of a one-wave workgroup per
@@ -720,83 +729,111 @@ static long scan1d_split_override() {
     return v;
 }
 
-// Segment length for a split launch, or 0 to run unsplit. Only N = 16 and
-// layouts whose batch stride is the sequence's (the [B*S, Ls, .] view),
-// without checkpoints, when the unsplit grid leaves CUs idle. The model,
-// from gfx950 timings of the 8-wave kernel with one workgroup per CU: a
-// launch of n workgroups over Ls steps takes (4 + 2.1 ceil(Ls/64))
-// ceil(n/256) us; a split runs two such launches over S = L/Ls segments of
-// B*groups*S workgroups, plus ~6 us for the fold and the clamp check. The
-// split is taken when the best segment length beats the unsplit launch by
-// 15 %.
+constexpr int kMaxSegments = 64;
+
+// Segment length (a multiple of 64; the last segment may be shorter) for a
+// split launch, or 0 to run unsplit. Only N = 16, and only when the unsplit
+// grid leaves CUs idle. The model, from gfx950 timings of the 8-wave kernel
+// with one workgroup per CU: a launch of n workgroups over c 64-step chunks
+// takes (4 + 2.1 c) ceil(n / 256) us, and a split runs two of them, plus
+// ~6 us for the clamp check and the launches; it is taken when it wins 15 %.
+// B1 L5003 D1536 bf16 gated (48 groups): 79.2 us in 5 segments, 195.7 us
+// unsplit; B1 L1920 D768 fp32 (24): 29.5 in 10, 68.8; B2 L1920 D1536 fp32
+// (96): 71.7 in 5 against 69.6 unsplit, which the model keeps.
 static long segment_length(const KMScan1DFwd *k, long groups_total) {
-    if (k->N != 16 || k->h_ckpt || groups_total >= 128 || k->L % 64 != 0 || k->L < 128) return 0;
-    if (k->B > 1 && k->bc_sb != k->L * k->bc_st) return 0;
+    if (k->N != 16 || groups_total >= 128 || k->L < 128) return 0;
     const long ov = scan1d_split_override();
     if (ov == 0) return 0;
-    if (ov > 0)
-        return (ov % 64 == 0 && ov < k->L && k->L % ov == 0 && k->L / ov <= kMaxSegments) ? ov : 0;
-    auto launch_us = [](long steps, long wgs) {
-        return (4.0 + 2.1 * static_cast<double>((steps + 63) / 64)) *
-               static_cast<double>((wgs + 255) / 256);
+    if (ov > 0 && ov % 64 == 0 && ov < k->L && k->L % ov == 0 && k->L / ov <= kMaxSegments) return ov;
+    auto launch_us = [](long chunks, long wgs) {
+        return (4.0 + 2.1 * static_cast<double>(chunks)) * static_cast<double>((wgs + 255) / 256);
     };
-    const double unsplit = launch_us(k->L, groups_total);
+    const long nc = (k->L + 63) / 64;
+    const double unsplit = launch_us(nc, groups_total);
     double best_t = 0.85 * unsplit;
     long best = 0;
-    for (long ls = 64; ls < k->L; ls += 64) {
-        if (k->L % ls != 0 || k->L / ls > kMaxSegments) continue;
-        const double t = 2.0 * launch_us(ls, groups_total * (k->L / ls)) + 6.0;
+    for (long c = 1; c < nc; ++c) {
+        const long S = (nc + c - 1) / c;
+        if (S > kMaxSegments) continue;
+        const double t = 2.0 * launch_us(c, groups_total * S) + 6.0;
         if (t < best_t) {
             best_t = t;
-            best = ls;
+            best = 64 * c;
         }
     }
     return best;
 }
 
+// Whether the split may use the library's scratch for this call. Sequences
+// of whole 64-step blocks without checkpoints, whose batch stride is the
+// sequence's, always have; every other call needs scratch only to run
+// faster, so it is split only where taking scratch cannot disturb the
+// caller: not while the stream is captured (a graph would keep the block's
+// address), not on the per-thread stream (one handle, several streams).
+static bool split_always(const KMScan1DFwd *k) {
+    return k->L % 64 == 0 && !k->h_ckpt && (k->B == 1 || k->bc_sb == k->L * k->bc_st);
+}
+
+// Launches of one split call on a stream stay together when several host
+// threads enqueue on it (they share the stream's scratch block).
+static std::mutex g_split_mu;
+
 // Segment workgroups have the unsplit kernel's shape: 8 waves of 8 steps
-// (64-step super-chunks).
+// (64-step super-chunks). Returns 1 when the scratch is not to be had and
+// the call can run unsplit.
 template <typename T>
-static int launch_segmented(const KMScan1DFwd *k, long Ls, hipStream_t s) {
+static int launch_segmented(const KMScan1DFwd *k, const Scan1DFwdArgs &base, long Ls, hipStream_t s) {
     constexpr int NPL = 8, NS = 2, DL = 32, WS = 8;
-    const long S = k->L / Ls;
+    const long S = (k->L + Ls - 1) / Ls;
     const long groups = (k->D + DL - 1) / DL;
-    const long BS = k->B * S;
-    const size_t st = align_up(sizeof(float) * BS * k->D * k->N, 256);
-    const size_t sd = align_up(sizeof(float) * BS * k->D, 256);
-    char *ws = static_cast<char *>(Workspace::reserve(2 * st + sd + align_up(4 * k->B * groups, 256), s, WsUse::Scan1DSplit));
-    if (!ws) return -1;
-    float *hl = reinterpret_cast<float *>(ws);
-    float *hin = reinterpret_cast<float *>(ws + st);
-    float *dsum = reinterpret_cast<float *>(ws + 2 * st);
-    int *flags = reinterpret_cast<int *>(ws + 2 * st + sd);
-    const long grid = BS * groups;
-    if (grid > 0x7fffffffL) {
-        set_error("km_scan1d_fwd: grid of %ld workgroups out of range", grid);
-        return -1;
+    const long grid = k->B * S * groups, mgrid = k->B * (S - 1) * groups;
+    const size_t nst = static_cast<size_t>(k->B) * k->D * k->N;
+    const size_t st = align_up(sizeof(float) * nst * (S - 1), 256);
+    const size_t sd = align_up(sizeof(float) * k->B * k->D * (S - 1), 256);
+    const size_t sf = align_up(4 * k->B * groups, 256);
+    const char *h0b = reinterpret_cast<const char *>(k->h0), *hfb = reinterpret_cast<const char *>(k->h_final);
+    const bool alias = h0b && hfb && h0b < hfb + 4 * nst && hfb < h0b + 4 * nst;
+    const size_t bytes = st + sd + sf + (alias ? align_up(4 * nst, 256) : 0);
+    std::lock_guard<std::mutex> guard(g_split_mu);
+    char *ws;
+    if (split_always(k)) {
+        ws = static_cast<char *>(Workspace::reserve(bytes, s, WsUse::Scan1DSplit));
+        if (!ws) return -1;
+    } else {
+        ws = static_cast<char *>(Workspace::try_reserve(bytes, s, WsUse::Scan1DSegments));
+        if (!ws) return 1;
     }
     const bool shared = (k->bc_sd == 0), hist = (k->h_hist != nullptr);
     const bool gate = k->z || k->Dskip;
-    // (1) local end states and delta sums of every segment, from zero
-    Scan1DFwdArgs a{k->x, k->delta, k->A, k->Bm, k->Cm, nullptr, nullptr, hl, nullptr, nullptr, 1,
-                    nullptr, nullptr, BS, Ls, k->D, k->N, Ls * k->bc_st, k->bc_st, k->bc_sd, 0,
-                    nullptr, S, dsum};
-#define KM_SEG(SH, HI, GA, BU) \
-    hipLaunchKernelGGL((scan1d_fwd_chunked<T, NPL, NS, WS, 8, SH, HI, BU, 2, GA, true>), dim3(grid), dim3(64 * WS), 0, s, a)
-    if (shared) KM_SEG(true, false, false, true); else KM_SEG(false, false, false, true);
+    int *flags = reinterpret_cast<int *>(ws + st + sd);
+    // (1) map pass: end states from zero and delta sums of every segment but
+    // the last; clamp flags cleared
+    Scan1DFwdArgs a = base;
+    a.nseg = static_cast<int>(S - 1);
+    a.Ls = static_cast<int>(Ls);
+    a.seg_h = reinterpret_cast<float *>(ws);
+    a.seg_dsum = reinterpret_cast<float *>(ws + st);
+    a.clamp_flag = k->clamp ? flags : nullptr;
+    a.h0_copy = alias ? reinterpret_cast<float *>(ws + st + sd + sf) : nullptr;
+    a.y = nullptr; a.hfin = nullptr; a.hist = nullptr; a.ckpt = nullptr; a.z = nullptr; a.Dskip = nullptr;
+#define KM_SEG(SH) \
+    hipLaunchKernelGGL((scan1d_fwd_chunked<T, NPL, NS, WS, 8, SH, false, true, 2, false, true>), \
+                       dim3(static_cast<unsigned>(mgrid)), dim3(64 * WS), 0, s, a)
+    if (shared) KM_SEG(true); else KM_SEG(false);
+#undef KM_SEG
     KM_HIP_TRY(hipGetLastError());
-    // (2) incoming state of every segment, the final state, flags cleared
-    const long nth = k->B * k->D * k->N;      // >= B * groups flags
-    hipLaunchKernelGGL(scan1d_segment_fold, dim3((nth + 255) / 256), dim3(256), 0, s, k->A, k->h0,
-                       static_cast<const float *>(hl), static_cast<const float *>(dsum), hin,
-                       k->h_final, flags, k->B * groups, k->B, k->D, static_cast<int>(S));
-    KM_HIP_TRY(hipGetLastError());
-    // (3) replay every segment from its incoming state
-    Scan1DFwdArgs r{k->x, k->delta, k->A, k->Bm, k->Cm, k->y, hin, nullptr, k->h_hist, nullptr, 1,
-                    k->z, k->Dskip, BS, Ls, k->D, k->N, Ls * k->bc_st, k->bc_st, k->bc_sd, k->clamp,
-                    k->clamp ? flags : nullptr, S};
+    // (2) replay every segment from the state its predecessors' maps give
+    Scan1DFwdArgs r = base;
+    r.nseg = static_cast<int>(S);
+    r.Ls = static_cast<int>(Ls);
+    r.seg_h = a.seg_h;
+    r.seg_dsum = a.seg_dsum;
+    r.seg_in = 1;
+    r.clamp_flag = a.clamp_flag;
+    if (alias) r.h0 = a.h0_copy;
 #define KM_SEGR(SH, HI, GA) \
-    hipLaunchKernelGGL((scan1d_fwd_chunked<T, NPL, NS, WS, 8, SH, HI, !HI && !GA, 2, GA>), dim3(grid), dim3(64 * WS), 0, s, r)
+    hipLaunchKernelGGL((scan1d_fwd_chunked<T, NPL, NS, WS, 8, SH, HI, !HI && !GA, 2, GA>), \
+                       dim3(static_cast<unsigned>(grid)), dim3(64 * WS), 0, s, r)
     if (shared) {
         if (hist) { if (gate) KM_SEGR(true, true, true); else KM_SEGR(true, true, false); }
         else      { if (gate) KM_SEGR(true, false, true); else KM_SEGR(true, false, false); }
@@ -805,13 +842,11 @@ static int launch_segmented(const KMScan1DFwd *k, long Ls, hipStream_t s) {
         else      { if (gate) KM_SEGR(false, false, true); else KM_SEGR(false, false, false); }
     }
 #undef KM_SEGR
-#undef KM_SEG
     KM_HIP_TRY(hipGetLastError());
     if (k->clamp) {
-        // (4) flagged sequences again, sequentially with the clamp
-        Scan1DFwdArgs q{k->x, k->delta, k->A, k->Bm, k->Cm, k->y, k->h0, k->h_final, k->h_hist, nullptr,
-                        1, k->z, k->Dskip, k->B, k->L, k->D, k->N, k->bc_sb, k->bc_st, k->bc_sd, 1,
-                        nullptr, 1};
+        // (3) flagged sequences again, sequentially with the clamp
+        Scan1DFwdArgs q = base;
+        if (alias) q.h0 = a.h0_copy;
         const dim3 g2(static_cast<unsigned>(k->B * groups));
         if (shared) {
             if (hist) hipLaunchKernelGGL((scan1d_clamp_repair<T, NPL, NS, true, true>), g2, dim3(64), 0, s, q, flags);
@@ -872,7 +907,8 @@ int scan1d_fwd_launch(const KMScan1DFwd *k, hipStream_t stream, bool allow_split
     }
     Scan1DFwdArgs a{k->x, k->delta, k->A, k->Bm, k->Cm, k->y, k->h0, k->h_final, k->h_hist,
                     k->h_ckpt, (k->L + kCkptSteps - 1) / kCkptSteps, k->z, k->Dskip,
-                    k->B, k->L, k->D, k->N, k->bc_sb, k->bc_st, k->bc_sd, k->clamp, nullptr, 1};
+                    k->B, k->L, k->D, k->N, k->bc_sb, k->bc_st, k->bc_sd, k->clamp, 1,
+                    static_cast<int>(std::min<long>(k->L, 0x7fffffffL)), nullptr, nullptr, nullptr, 0, nullptr};
     // The register-blocked kernel addresses each batch element's windows with
     // 32-bit byte offsets; larger problems take the sequential kernel.
     const long es = (k->dtype == KM_BF16) ? 2 : 4;
@@ -887,8 +923,10 @@ int scan1d_fwd_launch(const KMScan1DFwd *k, hipStream_t stream, bool allow_split
         return bf ? launch_serial<bf16_t>(a, hist, stream) : launch_serial<f32_t>(a, hist, stream);
     // Few (batch, channel group) pairs and a long sequence: split the
     // sequence over workgroups.
-    if (const long Ls = allow_split ? segment_length(k, k->B * ((k->D + 31) / 32)) : 0)
-        return bf ? launch_segmented<bf16_t>(k, Ls, stream) : launch_segmented<f32_t>(k, Ls, stream);
+    if (const long Ls = allow_split ? segment_length(k, k->B * ((k->D + 31) / 32)) : 0) {
+        const int rc = bf ? launch_segmented<bf16_t>(k, a, Ls, stream) : launch_segmented<f32_t>(k, a, Ls, stream);
+        if (rc <= 0) return rc;
+    }
     switch (k->N) {
     case 16:
         return bf ? launch_n16<bf16_t>(a, shared, hist, stream)

@@ -270,6 +270,35 @@ void *Workspace::reserve(size_t bytes, hipStream_t stream, WsUse use, bool *fres
     return p;
 }
 
+void *Workspace::try_reserve(size_t bytes, hipStream_t stream, WsUse use) {
+    if (stream == hipStreamPerThread) return nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (cap != hipStreamCaptureStatusNone) return nullptr;
+    {
+        std::lock_guard<std::mutex> guard(g_ws_mu);
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0) return nullptr;
+        bool have = false;
+        for (int i = 0; i < g_ws_n; ++i)
+            have = have || (g_ws[i].dev == dev && g_ws[i].stream == stream && g_ws[i].use == use);
+        if (!have && g_ws_n == kMaxWs) return nullptr;
+    }
+    // An allocation must not end a capture that some other stream is in.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    void *p = reserve(bytes, stream, use);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!p) clear_error();
+    return p;
+}
+
 size_t Workspace::release(hipStream_t stream) {
     std::lock_guard<std::mutex> guard(g_ws_mu);
     int dev = 0;

@@ -45,7 +45,8 @@ struct PinnedStaging {
 // another that reserves scratch (the Scan1D split's segment states) on the
 // same stream without the two aliasing.
 enum class WsUse : int {
-    Scan1DSplit = 0,   // segment end states, incoming states, flags
+    Scan1DSplit = 0,   // segment end states and delta sums, flags
+    Scan1DSegments,    // the same, where only try_reserve may provide it
     Scan1DBwd,         // checkpoints and per-workgroup partial sums
     Scan1DM1,          // M = 1 backward's per-workgroup ddelta partials
     ScanNDPlan,        // per-level fallback's plan offsets
@@ -71,6 +72,12 @@ enum class WsUse : int {
 struct Workspace {
     static void *reserve(size_t bytes, hipStream_t stream, WsUse use, bool *fresh = nullptr,
                          size_t *got = nullptr);   // nullptr on failure (error set)
+    // reserve() for scratch that only makes a call faster, so that taking it
+    // disturbs nothing: nullptr without an error (the caller runs without)
+    // while the stream is captured, on the per-thread stream (one handle,
+    // several streams), where a full table would cost another stream its
+    // block, and when the device has no room.
+    static void *try_reserve(size_t bytes, hipStream_t stream, WsUse use);
     // Frees every block of (current device, stream) after draining the
     // stream. Returns the bytes freed.
     static size_t release(hipStream_t stream);

@@ -1,0 +1,95 @@
+"""GPU parity of the segmented Scan1D forward on sequences that are not whole
+64-step blocks, with checkpoints, with the state updated in place, and under
+stream capture, against the CPU oracle (condition-scaled error <= 1e-4 fp32)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import kmamba as K
+import oracle as O
+from kmtest import TOL_F32, assert_close, rel_err_cond, rng_for, scan1d_inputs, scan1d_kappa
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+N = 16
+
+
+def T(a, dtype=torch.float32):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV, dtype)
+
+
+# Few channel groups and a last segment of 1, 41, 63, 9 and 64 steps; D not a
+# multiple of 32 leaves lanes without a channel.
+RAGGED = [(1, 1025, 64), (2, 1001, 40), (3, 1023, 100), (1, 777, 32), (1, 4160, 96)]
+
+
+@pytest.mark.parametrize("Bsz,L,D", RAGGED)
+@pytest.mark.parametrize("layout", ["shared", "per_channel"])
+def test_ragged_segments_with_checkpoints(Bsz, L, D, layout):
+    x, dt, A, _, _ = scan1d_inputs(Bsz, L, D, N, seed=31)
+    g = rng_for("segments", Bsz, L, D)
+    h0 = g.standard_normal((Bsz, D, N)).astype(np.float32)
+    shape = (Bsz, L, N) if layout == "shared" else (Bsz, L, D, N)
+    strides = (L * N, N, 0) if layout == "shared" else (L * D * N, D * N, N)
+    Bm, Cm = ((g.standard_normal(shape) * 0.25).astype(np.float32) for _ in range(2))
+    yr, hr, hhr = O.scan1d_batched(x, dt, A, Bm, Cm, h0=h0, bc_strides=strides, hist=True)
+    ky, kh, khh = scan1d_kappa(x, dt, A, Bm, Cm, h0=h0, bc_strides=strides)
+    # The checkpoint after every 32 steps and after the last one.
+    at = np.minimum(np.arange(31, L + 31, 32), L - 1)
+    ck = torch.full((Bsz, len(at), D, N), float("nan"), device=DEV)
+    y = torch.full((Bsz, L, D), float("nan"), device=DEV)
+    hf = torch.empty((Bsz, D, N), device=DEV)
+    hh = torch.full((Bsz, L, D, N), float("nan"), device=DEV)
+    ins = [T(a) for a in (x, dt, A, Bm, Cm)]
+    for hist in (None, hh):
+        K.scan1d_fwd(*ins, y, h0=T(h0), h_final=hf, h_hist=hist, h_ckpt=ck, bc_strides=strides)
+        assert_close(y.cpu().numpy(), yr, TOL_F32, "y", ky)
+        assert_close(hf.cpu().numpy(), hr, TOL_F32, "h_final", kh)
+        assert_close(ck.cpu().numpy(), hhr[:, at], TOL_F32, "checkpoints", khh[:, at])
+    assert_close(hh.cpu().numpy(), hhr, TOL_F32, "history", khh)
+
+
+@pytest.mark.parametrize("L", [1024, 1001])
+@pytest.mark.parametrize("peak", [1.0, 4000.0])
+def test_state_updated_in_place(L, peak):
+    # h_final is h0's own memory; with peak = 4000 the states of a few steps
+    # leave [-1000, 1000], so the whole sequence is re-run from h0.
+    Bsz, D = 2, 40
+    x, dt, A, Bm, Cm = scan1d_inputs(Bsz, L, D, N, seed=32)
+    Bm = Bm.copy()
+    Bm[:, 500:505] *= peak
+    h0 = rng_for("in-place", L).standard_normal((Bsz, D, N)).astype(np.float32) * 50
+    yr, hr, _ = O.scan1d_batched(x, dt, A, Bm, Cm, h0=h0)
+    ky, kh, _ = scan1d_kappa(x, dt, A, Bm, Cm, h0=h0)
+    h = T(h0)
+    y = torch.empty((Bsz, L, D), device=DEV)
+    K.scan1d_fwd(*(T(a) for a in (x, dt, A, Bm, Cm)), y, h0=h, h_final=h)
+    assert_close(y.cpu().numpy(), yr, TOL_F32, "y", ky)
+    assert_close(h.cpu().numpy(), hr, TOL_F32, "h", kh)
+
+
+def test_captured_call_takes_no_scratch():
+    # A capture of a shape that would be split needs no allocation, and its
+    # replays follow changed inputs.
+    Bsz, L, D = 1, 1001, 64
+    x, dt, A, Bm, Cm = (T(a) for a in scan1d_inputs(Bsz, L, D, N, seed=33))
+    y, hf = torch.empty_like(x), torch.empty((Bsz, D, N), device=DEV)
+    s = torch.cuda.Stream()
+    args = K.scan1d_fwd_args(x, dt, A, Bm, Cm, y, h_final=hf)
+    held = K.km_device_bytes_held()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        assert K.km_scan1d_fwd_c(C.byref(args), C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    assert K.km_device_bytes_held() == held
+    for i in range(3):
+        xi = rng_for("graph", i).standard_normal((Bsz, L, D)).astype(np.float32)
+        x.copy_(T(xi))
+        g.replay()
+        torch.cuda.synchronize()
+        yr, hr, _ = O.scan1d_batched(xi, *(a.cpu().numpy() for a in (dt, A, Bm, Cm)))
+        ky, kh, _ = scan1d_kappa(xi, *(a.cpu().numpy() for a in (dt, A, Bm, Cm)))
+        assert rel_err_cond(y.cpu().numpy(), yr, ky) <= TOL_F32
+        assert rel_err_cond(hf.cpu().numpy(), hr, kh) <= TOL_F32
