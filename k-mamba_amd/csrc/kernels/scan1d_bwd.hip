@@ -42,6 +42,7 @@
 #include <type_traits>
 
 #include "km_device.hpp"
+#include "scan1d_maps.hpp"
 #include "../km_runtime.hpp"
 #include "kmamba_km.h"
 #include "scan.h"
@@ -61,12 +62,19 @@ struct Scan1DBwdArgs {
     const float *ckpt;     // [B, nck, D, N] state after each 32-step block, or null
     long nck;
     void *dx, *ddt;        // [B, L, D]
-    float *dApart;         // [B, D, N] per-batch dA partials (every element written)
+    float *dApart;         // [B * nseg, D, N] dA partials (every element written)
     float *slot;           // shared B/C: [B, G, L, 2, N] per-channel-group partials (dB, dC)
     long G;                // channel groups per batch element (shared B/C slots)
     void *dB, *dC;         // per-channel B/C: written at the B/C strides
     long B, L, D, N, sb, st, sd;
     int clamp;
+    // A sequence split over nseg workgroups (per channel group), each on sps
+    // super-chunks: its incoming adjoint is folded from the maps of the parts
+    // after it (scan1d_maps.hpp, map_per parts a segment, nmap in all), and
+    // dApart holds [B, nseg, D, N]. nseg = 1 otherwise.
+    int nseg, sps;
+    const float *seg_g, *seg_dsum;
+    int nmap, map_per;
 };
 
 // v from the lane whose id differs in bit MASK: ds_swizzle inside 32-lane
@@ -158,7 +166,9 @@ __device__ __forceinline__ void pow_chain_b(float e1, int n0, float (&e)[NPL]) {
 // the two halves' sums of one round of every wave's steps (half 0's first)
 // and stores them to the slot. The LDS then holds one workgroup per CU
 // (16 waves, as two 8-wave workgroups did).
-template <typename T, int NPL, int NS, bool SHARED, bool HIN, int HWT>
+// SEG: the workgroup owns a segment of the sequence and starts from the
+// adjoint it folds from the maps after it.
+template <typename T, int NPL, int NS, bool SHARED, bool HIN, int HWT, bool SEG>
 __global__ void __launch_bounds__(HWT == 2 ? 1024 : 512, 4) scan1d_bwd_chunked(Scan1DBwdArgs p) {
     using IO = bio<T>;
     constexpr int W = 8, TC = 4;
@@ -206,20 +216,25 @@ __global__ void __launch_bounds__(HWT == 2 ? 1024 : 512, 4) scan1d_bwd_chunked(S
     const int dl = lane % DL;
     const int ns = lane / DL;
     const int n0 = ns * NPL;
-    const long ngroups = (p.D + DL * HW - 1) / (DL * HW);
+    const unsigned ngroups = static_cast<unsigned>((p.D + DL * HW - 1) / (DL * HW));
     // Workgroups numbered so that consecutive channel groups run on one
     // XCD: a group's DL channels are only part of each 128-byte row line
     // of x / delta / dy, and the neighbours that read the rest of the line
     // then find it in the same L2 instead of fetching it again.
-    const long wg = xcd_remap(blockIdx.x, gridDim.x);
-    const long b = wg / ngroups;
-    const long grp = wg - b * ngroups;
-    const long d = grp * DL * HW + hh * DL + dl;
+    // The grid is below 2^31, so the divisions are 32-bit.
+    const unsigned wg = static_cast<unsigned>(xcd_remap(blockIdx.x, gridDim.x));
+    const unsigned bs = wg / ngroups;                       // (batch element, segment)
+    const unsigned grp = wg - bs * ngroups;
+    const long b = SEG ? bs / static_cast<unsigned>(p.nseg) : bs;
+    const int seg = SEG ? static_cast<int>(bs - static_cast<unsigned>(b) * static_cast<unsigned>(p.nseg)) : 0;
+    const long d = static_cast<long>(grp) * DL * HW + hh * DL + dl;
     const bool dvalid = d < p.D;
     const int dc = static_cast<int>(dvalid ? d : p.D - 1);
     const int L = static_cast<int>(p.L);
     const int Dm = static_cast<int>(p.D);
-    const int nit = (L + SC - 1) / SC;
+    // Super-chunks [s0, s1) of the sequence, walked from the last.
+    const int s0 = SEG ? seg * p.sps : 0, s1 = SEG ? min((L + SC - 1) / SC, s0 + p.sps) : (L + SC - 1) / SC;
+    const int nit = s1 - s0;
     const bool own_x = dvalid && ns == 0;
 
     // Per-batch-element windows, 32-bit byte offsets in the VGPR offset (the
@@ -308,7 +323,36 @@ __global__ void __launch_bounds__(HWT == 2 ? 1024 : 512, 4) scan1d_bwd_chunked(S
         }
     };
 
-    if (w == 0) {
+    // The adjoint entering the workgroup's last step, state w by wave w (the
+    // clamped re-run finds it again in the dA partial, which is written
+    // last): zero,
+    // or the fold of the maps after a segment, last first,
+    // g <- exp(A * sum delta) g + g_end. kFoldRun maps' loads are in flight
+    // together.
+    if constexpr (SEG) {
+        if (w < NPL) {
+            float run = 0.f;
+            const int m0 = seg * p.map_per;                           // map 0 follows segment 0
+            if (p.nmap > m0) {
+                constexpr int kFoldRun = 8;
+                const float a2 = p.A[dc * N + n0 + w] * kLog2e;
+                for (int m1 = p.nmap - 1; m1 >= m0; m1 -= kFoldRun) {
+                    float dsv[kFoldRun], gv[kFoldRun];
+#pragma unroll
+                    for (int i = 0; i < kFoldRun; ++i) {
+                        const long m = (b * p.nmap + max(m1 - i, m0)) * Dm + dc;
+                        dsv[i] = p.seg_dsum[m];
+                        gv[i] = p.seg_g[m * N + n0 + w];
+                    }
+#pragma unroll
+                    for (int i = 0; i < kFoldRun; ++i)
+                        if (m1 - i >= m0) run = fmaf(exp2_fast(dsv[i] * a2), run, gv[i]);
+                }
+            }
+            acar[0][w][lh] = run;
+            if (!HIN && dvalid) p.dApart[(static_cast<long>(bs) * Dm + d) * N + n0 + w] = run;
+        }
+    } else if (w == 0) {
 #pragma unroll
         for (int j = 0; j < NPL; ++j) acar[0][j][lh] = 0.f;
     }
@@ -364,13 +408,26 @@ __global__ void __launch_bounds__(HWT == 2 ? 1024 : 512, 4) scan1d_bwd_chunked(S
     };
     // The same for the state this wave folds (wave w < NPL folds state w),
     // as a load prefetched with the super-chunk's x / delta / dy; super-chunk
-    // 0 starts from h0 (zero when null).
+    // 0 starts from h0 (zero when null). In the segment form the row's
+    // base is wave-uniform: the lane keeps one 32-bit offset and no address
+    // (the loop's registers are full, and a spill reload there waits for every
+    // prefetch in flight: 727 against 676 us for the fp32 training step below).
+    // Unsplit, the lane's own address costs less (bf16 503 against 515 us).
     const int jf = w < NPL ? w : NPL - 1;
-    const float *ck0 = HIN ? nullptr : p.ckpt + (b * p.nck * Dm + dc) * N + n0 + jf;
-    const float h0v = p.h0 ? p.h0[(b * Dm + dc) * N + n0 + jf] : 0.f;
+    const unsigned vck = static_cast<unsigned>(dc * N + n0 + jf);
+    const float *const ckb = HIN ? nullptr : p.ckpt + b * p.nck * Dm * N;
+    const float *const h0b = p.h0 ? p.h0 + b * Dm * N : ckb;
+    const float *const ck0 = HIN ? nullptr : ckb + vck;
+    const float h0v = p.h0 ? h0b[vck] : 0.f;
     auto load_ck = [&](int s) -> float {
-        const float cv = ck0[static_cast<long>(max(s - 1, 0)) * Dm * N];
-        return (s == 0) ? h0v : cv;
+        if constexpr (SEG) {
+            const float *base = s > 0 ? ckb + static_cast<unsigned>(s - 1) * static_cast<unsigned>(Dm * N) : h0b;
+            const float cv = base[vck];
+            return (s == 0 && !p.h0) ? 0.f : cv;
+        } else {
+            const float cv = ck0[static_cast<long>(max(s - 1, 0)) * Dm * N];
+            return (s == 0) ? h0v : cv;
+        }
     };
 
     // Prefetches are issued unconditionally (clamped to super-chunk 0, or
@@ -378,14 +435,14 @@ __global__ void __launch_bounds__(HWT == 2 ? 1024 : 512, 4) scan1d_bwd_chunked(S
     // would make the compiler's wait-count merge at the join wait for it
     // before the current data is used.
     if constexpr (SHARED) {
-        load_tile(nit - 1);
+        load_tile(s1 - 1);
         store_tile(0);
-        load_tile(max(nit - 2, 0));
+        load_tile(max(s1 - 2, 0));
     }
     float X0[TC], D0[TC], G0[TC], X1[TC], D1[TC], G1[TC];
     float K0 = 0.f, K1 = 0.f;
-    load_xd(nit - 1, X0, D0, G0);
-    if constexpr (!HIN) K0 = load_ck(nit - 1);
+    load_xd(s1 - 1, X0, D0, G0);
+    if constexpr (!HIN) K0 = load_ck(s1 - 1);
     __syncthreads();
 
     float dAacc[NPL];
@@ -639,7 +696,7 @@ __global__ void __launch_bounds__(HWT == 2 ? 1024 : 512, 4) scan1d_bwd_chunked(S
     auto body = [&](int it, float (&xs)[TC], float (&ds)[TC], float (&gs)[TC],
                     float ks, float (&xn)[TC], float (&dn)[TC], float (&gn)[TC],
                     float &kn) __attribute__((always_inline)) {
-        const int s = nit - 1 - it;
+        const int s = s1 - 1 - it;
         const int cur = it & 1;
         const int slot = it % 3;
         if constexpr (SHARED) {
@@ -689,7 +746,7 @@ __global__ void __launch_bounds__(HWT == 2 ? 1024 : 512, 4) scan1d_bwd_chunked(S
     // from the checkpoint with the sequential clamped recurrence in the
     // forward fallback's arithmetic order.
     auto body_rerun = [&](int it) __attribute__((always_inline)) {
-        const int s = nit - 1 - it;
+        const int s = s1 - 1 - it;
         const int cur = it & 1;
         __syncthreads();                 // the previous super-chunk's tile reads are done
         if (it > 0) comb_flush(s + 1);
@@ -746,20 +803,23 @@ __global__ void __launch_bounds__(HWT == 2 ? 1024 : 512, 4) scan1d_bwd_chunked(S
         if (it + 1 < nit) body(it + 1, X1, D1, G1, K1, X0, D0, G0, K0);
     }
     __syncthreads();
-    comb_flush(0);
+    comb_flush(s0);
     if constexpr (!HIN) {
         // Some super-chunk's states may have left [-1000, 1000]: every
         // output of this workgroup again, with the clamped states.
         if (__builtin_amdgcn_readfirstlane(s_bad) != 0) {
 #pragma unroll
             for (int j = 0; j < NPL; ++j) dAacc[j] = 0.f;
-            if (w == 0) {
+            if constexpr (SEG) {
+                if (w < NPL)
+                    acar[0][w][lh] = dvalid ? p.dApart[(static_cast<long>(bs) * Dm + d) * N + n0 + w] : 0.f;
+            } else if (w == 0) {
 #pragma unroll
                 for (int j = 0; j < NPL; ++j) acar[0][j][lh] = 0.f;
             }
             for (int it = 0; it < nit; ++it) body_rerun(it);
             __syncthreads();
-            comb_flush(0);
+            comb_flush(s0);
         }
     }
 
@@ -775,7 +835,7 @@ __global__ void __launch_bounds__(HWT == 2 ? 1024 : 512, 4) scan1d_bwd_chunked(S
             float acc = aggA[0][j][lh];
 #pragma unroll
             for (int v = 1; v < W; ++v) acc += aggA[v][j][lh];
-            p.dApart[(b * Dm + d) * N + n0 + j] = acc;
+            p.dApart[(static_cast<long>(bs) * Dm + d) * N + n0 + j] = acc;
         }
     }
 }
@@ -864,8 +924,8 @@ __global__ void __launch_bounds__(256) fill_zero_kernel(float *p, long n) {
     for (long i = n4 * 4 + i0; i < n; i += stride) p[i] = 0.f;
 }
 
-// Fixed-order sums of the partials: dA[i] = sum over b of dApart[b, i]
-// (b ascending); with shared B/C, dB / dC at b*sb + t*st + n = sum over the
+// Fixed-order sums of the partials: dA[i] = sum over b < nA of dApart[b, i]
+// (b ascending: batch elements, and their segments in order); with shared B/C, dB / dC at b*sb + t*st + n = sum over the
 // channel groups g (ascending) of slot[b, g, t, 0 / 1, n].
 template <typename T>
 // With q4 (N a multiple of 4) a thread sums four consecutive states with
@@ -874,7 +934,7 @@ template <typename T>
 __global__ void __launch_bounds__(256) scan1d_bwd_finalize(const float *slot, long G, void *dB,
                                                            void *dC, long B, long L, long N,
                                                            long sb, long st, const float *dApart,
-                                                           float *dA, long DN, int q4) {
+                                                           float *dA, long DN, long nA, int q4) {
     using IO = io<T>;
     const long Q = q4 ? 4 : 1;                 // states per thread
     const long Nq = N / Q;
@@ -924,7 +984,7 @@ __global__ void __launch_bounds__(256) scan1d_bwd_finalize(const float *slot, lo
         } else {
             const long k = i - n_bc;
             float acc = 0.f;
-            for (long b = 0; b < B; ++b) acc += dApart[b * DN + k];
+            for (long b = 0; b < nA; ++b) acc += dApart[b * DN + k];
             dA[k] = acc;
         }
     }
@@ -941,8 +1001,13 @@ static int fill_zero(float *p, long n, hipStream_t s) {
 struct BwdPlan {
     bool shared, hist_in, need_ckpt, serial, need_hist;
     bool wide;              // N = 16 shared B/C on 32-channel workgroups (two halves)
+    bool wide_split;        // the same for the split form
     long G;                 // channel groups per batch element (partial slots)
     size_t off_slots, off_dA, off_ckpt, off_hist, bytes;
+    // Split over S segments of sps super-chunks (S = 1: not split), the maps'
+    // parts per segment, and its scratch: maps, delta sums, dA partials.
+    long S, sps, parts;
+    size_t off_g, off_ds, off_dAS, seg_bytes;
 };
 
 // Channels per workgroup of the register-blocked backward for a state size.
@@ -963,6 +1028,57 @@ static bool bwd_wide(long B, long D) {
     if (e && std::strcmp(e, "1") == 0) return true;
     if (e && std::strcmp(e, "0") == 0) return false;
     return B * ((D + 31) / 32) >= kWideMinGroups;
+}
+
+// The split of a sequence over workgroups, for grids that leave the chip
+// partly idle or its last round of workgroups nearly empty. The model, from
+// gfx950 timings (us): per 32-step super-chunk an 8-wave workgroup (16
+// channels) takes 2.65 alone on its CU and 4.05 with a second one beside it, a
+// 16-wave one (32 channels) 4.05; each round of workgroups adds 6 (16 waves:
+// 14) of prologue and uneven ends; the finalize reads the slots at 4.7 TB/s; a
+// split adds the map pass (3.8 VALU instructions per state update) and ~12 of
+// launch, fold and partials. Taken when it wins 10 %. Training step (forward
+// and backward): B1 L4096 D1024 fp32 461 -> 145 us (8 segments), B2 L1999 D768
+// bf16 249 -> 126, B4 L4096 D1024 fp32 479 -> 437, B9 L2000 D1024 fp32 (288
+// workgroups, 1.1 rounds) 656 -> 567.
+constexpr long kMaxBwdSegments = 64;
+static void bwd_segments(const KMScan1DBwd *k, BwdPlan &pl) {
+    pl.S = 1;
+    pl.sps = (k->L + kCkptSteps - 1) / kCkptSteps;
+    pl.parts = 1;
+    if (pl.serial || k->N != 16 || pl.sps < 4) return;
+    const char *we = std::getenv("KM_SCAN1D_BWD_WIDE");
+    const bool forced = we && (std::strcmp(we, "0") == 0 || std::strcmp(we, "1") == 0);
+    auto main_us = [&](bool wide, long S, long sps) {
+        const long gc = wide ? 32 : 16, n = k->B * ((k->D + gc - 1) / gc) * S;
+        const double c = static_cast<double>(sps);
+        const double slots = pl.shared ? 128.0 * static_cast<double>(k->B * ((k->D + gc - 1) / gc) * k->L) / 4.7e6 : 0.0;
+        if (wide) return slots + (14.0 + 4.05 * c) * static_cast<double>((n + 255) / 256);
+        const long rest = n % 512;
+        return slots + (6.0 + 4.05 * c) * static_cast<double>(n / 512) +
+               (rest == 0 ? 0.0 : 6.0 + (rest <= 256 ? 2.65 : 4.05) * c);
+    };
+    const double map_us = 12.0 + static_cast<double>(k->B) * k->D * k->L * 16.0 * 3.8 / 64.0 / 0.5e6;
+    const double base = main_us(pl.wide, 1, pl.sps);
+    double best = 0.9 * base;
+    const long nsc = pl.sps;
+    for (long sps = 2; sps < nsc; sps += 2) {
+        const long S = (nsc + sps - 1) / sps;
+        if (S > kMaxBwdSegments) continue;
+        for (int wide = 0; wide < 2; ++wide) {
+            // Never more slots than the unsplit form's layout holds.
+            if ((wide && !pl.shared) || (!wide && pl.wide)) continue;
+            if (forced && (wide != 0) != pl.wide) continue;
+            const double t = main_us(wide != 0, S, sps) + map_us;
+            if (t < best) {
+                best = t;
+                pl.S = S;
+                pl.sps = sps;
+                pl.wide_split = wide != 0;
+            }
+        }
+    }
+    if (pl.S > 1) pl.parts = map_parts(k->B, k->D, pl.S - 1, pl.sps * kCkptSteps);
 }
 
 static BwdPlan bwd_plan(const KMScan1DBwd *k) {
@@ -991,6 +1107,15 @@ static BwdPlan bwd_plan(const KMScan1DBwd *k) {
     pl.off_hist = off;
     if (pl.need_hist) off += align_up(sizeof(float) * k->B * k->L * k->D * k->N, 256);
     pl.bytes = off;
+    // The split's own scratch (offsets from its start; bytes 0 without one).
+    bwd_segments(k, pl);
+    if (pl.S > 1) {
+        const size_t nst = static_cast<size_t>(k->B) * k->D * k->N, nmap = (pl.S - 1) * pl.parts;
+        pl.off_g = 0;
+        pl.off_ds = align_up(sizeof(float) * nst * nmap, 256);
+        pl.off_dAS = pl.off_ds + align_up(sizeof(float) * k->B * k->D * nmap, 256);
+        pl.seg_bytes = pl.off_dAS + align_up(sizeof(float) * nst * pl.S, 256);
+    }
     return pl;
 }
 
@@ -1026,44 +1151,54 @@ static int bwd_chunked_launch(const Scan1DBwdArgs &a, bool shared, bool hin, boo
     constexpr int W = 8;
     const long DL = bwd_group_channels(a.N, wide);
     const int HW = wide ? 2 : 1;   // the kernel's two halves (LDS sums)
-    const long grid = a.B * ((a.D + DL - 1) / DL);
+    const long grid = a.B * a.nseg * ((a.D + DL - 1) / DL);
     if (grid <= 0 || grid > 0x7fffffffL) {
         set_error("km_scan1d_bwd: grid of %ld workgroups out of range", grid);
         return -1;
     }
     dim3 g(static_cast<unsigned>(grid)), blk(64 * W * HW);
-#define KM_BWD_GO(TT, NPL, NS)                                                                    \
+#define KM_BWD_GO(TT, NPL, NS, SEG)                                                               \
     do {                                                                                          \
         if (shared) {                                                                             \
-            if (hin) hipLaunchKernelGGL((scan1d_bwd_chunked<TT, NPL, NS, true, true, 1>), g, blk, 0, s, a);   \
-            else     hipLaunchKernelGGL((scan1d_bwd_chunked<TT, NPL, NS, true, false, 1>), g, blk, 0, s, a);  \
+            if (hin) hipLaunchKernelGGL((scan1d_bwd_chunked<TT, NPL, NS, true, true, 1, SEG>), g, blk, 0, s, a);   \
+            else     hipLaunchKernelGGL((scan1d_bwd_chunked<TT, NPL, NS, true, false, 1, SEG>), g, blk, 0, s, a);  \
         } else {                                                                                  \
-            if (hin) hipLaunchKernelGGL((scan1d_bwd_chunked<TT, NPL, NS, false, true, 1>), g, blk, 0, s, a);  \
-            else     hipLaunchKernelGGL((scan1d_bwd_chunked<TT, NPL, NS, false, false, 1>), g, blk, 0, s, a); \
+            if (hin) hipLaunchKernelGGL((scan1d_bwd_chunked<TT, NPL, NS, false, true, 1, SEG>), g, blk, 0, s, a);  \
+            else     hipLaunchKernelGGL((scan1d_bwd_chunked<TT, NPL, NS, false, false, 1, SEG>), g, blk, 0, s, a); \
         }                                                                                         \
     } while (0)
-#define KM_BWD_WIDE(TT)                                                                           \
+#define KM_BWD_WIDE(TT, SEG)                                                                      \
     do {                                                                                          \
-        if (hin) hipLaunchKernelGGL((scan1d_bwd_chunked<TT, 4, 4, true, true, 2>), g, blk, 0, s, a);      \
-        else     hipLaunchKernelGGL((scan1d_bwd_chunked<TT, 4, 4, true, false, 2>), g, blk, 0, s, a);     \
+        if (hin) hipLaunchKernelGGL((scan1d_bwd_chunked<TT, 4, 4, true, true, 2, SEG>), g, blk, 0, s, a);      \
+        else     hipLaunchKernelGGL((scan1d_bwd_chunked<TT, 4, 4, true, false, 2, SEG>), g, blk, 0, s, a);     \
     } while (0)
+#define KM_BWD_T(GO, ...)                                                                         \
+    do {                                                                                          \
+        if (bf) GO(bf16_t, __VA_ARGS__);                                                          \
+        else    GO(f32_t, __VA_ARGS__);                                                           \
+    } while (0)
+    const bool seg = a.nseg > 1;
     if (wide) {
-        if (bf) KM_BWD_WIDE(bf16_t);
-        else    KM_BWD_WIDE(f32_t);
+        if (seg) KM_BWD_T(KM_BWD_WIDE, true);
+        else     KM_BWD_T(KM_BWD_WIDE, false);
         KM_HIP_TRY(hipGetLastError());
         return 0;
     }
-#undef KM_BWD_WIDE
     switch (a.N) {
-    case 16: if (bf) KM_BWD_GO(bf16_t, 4, 4); else KM_BWD_GO(f32_t, 4, 4); break;
-    case 8:  if (bf) KM_BWD_GO(bf16_t, 4, 2); else KM_BWD_GO(f32_t, 4, 2); break;
-    case 4:  if (bf) KM_BWD_GO(bf16_t, 4, 1); else KM_BWD_GO(f32_t, 4, 1); break;
-    case 2:  if (bf) KM_BWD_GO(bf16_t, 2, 1); else KM_BWD_GO(f32_t, 2, 1); break;
-    case 1:  if (bf) KM_BWD_GO(bf16_t, 1, 1); else KM_BWD_GO(f32_t, 1, 1); break;
+    case 16:
+        if (seg) KM_BWD_T(KM_BWD_GO, 4, 4, true);
+        else     KM_BWD_T(KM_BWD_GO, 4, 4, false);
+        break;
+    case 8:  KM_BWD_T(KM_BWD_GO, 4, 2, false); break;
+    case 4:  KM_BWD_T(KM_BWD_GO, 4, 1, false); break;
+    case 2:  KM_BWD_T(KM_BWD_GO, 2, 1, false); break;
+    case 1:  KM_BWD_T(KM_BWD_GO, 1, 1, false); break;
     default:
         set_error("km_scan1d_bwd: no register-blocked kernel for N=%ld", a.N);
         return -1;
     }
+#undef KM_BWD_T
+#undef KM_BWD_WIDE
 #undef KM_BWD_GO
     KM_HIP_TRY(hipGetLastError());
     return 0;
@@ -1073,7 +1208,8 @@ static int scan1d_bwd_run(const KMScan1DBwd *k, const BwdPlan &pl, bool bf, hipS
 
 size_t scan1d_bwd_workspace(const KMScan1DBwd *k) {
     if (!bwd_args_ok(k, "km_scan1d_bwd_workspace_bytes")) return 0;
-    return bwd_plan(k).bytes;
+    const BwdPlan pl = bwd_plan(k);
+    return pl.bytes + pl.seg_bytes;
 }
 
 int scan1d_bwd_launch(const KMScan1DBwd *k, hipStream_t stream) {
@@ -1086,7 +1222,7 @@ int scan1d_bwd_launch(const KMScan1DBwd *k, hipStream_t stream) {
 }
 
 static int scan1d_bwd_run(const KMScan1DBwd *k, const BwdPlan &pl, bool bf, hipStream_t stream) {
-    char *ws = nullptr;
+    char *ws = nullptr, *seg_ws = nullptr;
     if (pl.bytes > 0) {
         if (k->workspace) {
             if (k->workspace_bytes < pl.bytes) {
@@ -1095,11 +1231,18 @@ static int scan1d_bwd_run(const KMScan1DBwd *k, const BwdPlan &pl, bool bf, hipS
                 return -1;
             }
             ws = static_cast<char *>(k->workspace);
+            if (pl.seg_bytes > 0 && k->workspace_bytes >= pl.bytes + pl.seg_bytes) seg_ws = ws + pl.bytes;
         } else {
             ws = static_cast<char *>(Workspace::reserve(pl.bytes, stream, WsUse::Scan1DBwd));
             if (!ws) return -1;
+            // Scratch that only makes the call faster: unsplit without it.
+            if (pl.seg_bytes > 0)
+                seg_ws = static_cast<char *>(Workspace::try_reserve(pl.seg_bytes, stream, WsUse::Scan1DBwdSegments));
         }
     }
+    const bool split = seg_ws != nullptr, wide = split ? pl.wide_split : pl.wide;
+    const long gc = pl.serial ? kSerialNB : bwd_group_channels(k->N, wide);
+    const long G = (k->D + gc - 1) / gc;
     Scan1DBwdArgs a{};
     a.x = k->x; a.dt = k->delta; a.dy = k->dy; a.A = k->A; a.Bm = k->Bm; a.Cm = k->Cm;
     a.h0 = k->h0; a.hist = k->h_hist; a.ckpt = k->h_ckpt;
@@ -1109,8 +1252,10 @@ static int scan1d_bwd_run(const KMScan1DBwd *k, const BwdPlan &pl, bool bf, hipS
     a.sb = k->bc_sb; a.st = k->bc_st; a.sd = k->bc_sd; a.clamp = k->clamp;
     // Every partial slot is written by exactly one workgroup: nothing is
     // zeroed first.
-    a.G = pl.G;
-    a.dApart = reinterpret_cast<float *>(ws + pl.off_dA);
+    a.G = G;
+    a.nseg = split ? static_cast<int>(pl.S) : 1;
+    a.sps = static_cast<int>(split ? pl.sps : (k->L + kCkptSteps - 1) / kCkptSteps);
+    a.dApart = reinterpret_cast<float *>(split ? seg_ws + pl.off_dAS : ws + pl.off_dA);
     if (pl.shared) a.slot = reinterpret_cast<float *>(ws + pl.off_slots);
     if (pl.need_ckpt || pl.need_hist) {
         // Forward states from the same inputs (y not written).
@@ -1128,6 +1273,19 @@ static int scan1d_bwd_run(const KMScan1DBwd *k, const BwdPlan &pl, bool bf, hipS
         }
         if (scan1d_fwd_launch(&f, stream, true) != 0) return -1;
     }
+    if (split) {
+        // Adjoint maps of the parts after the first segment.
+        const long Ls = pl.sps * kCkptSteps;
+        MapArgs m{k->dy, k->delta, k->Cm, k->A, k->L, k->D, k->bc_sb, k->bc_st, k->bc_sd,
+                  static_cast<int>((pl.S - 1) * pl.parts), static_cast<int>(Ls / pl.parts), static_cast<int>(Ls),
+                  reinterpret_cast<float *>(seg_ws + pl.off_g), reinterpret_cast<float *>(seg_ws + pl.off_ds),
+                  nullptr, nullptr, nullptr};
+        if ((bf ? launch_maps<bf16_t, true>(m, k->B, stream) : launch_maps<f32_t, true>(m, k->B, stream)) != 0) return -1;
+        a.seg_g = m.seg_h;
+        a.seg_dsum = m.seg_dsum;
+        a.nmap = m.nmap;
+        a.map_per = static_cast<int>(pl.parts);
+    }
     if (pl.serial) {
         const long grid = k->B * pl.G;
         if (grid > 0x7fffffffL) {
@@ -1137,7 +1295,7 @@ static int scan1d_bwd_run(const KMScan1DBwd *k, const BwdPlan &pl, bool bf, hipS
         if (bf) hipLaunchKernelGGL(scan1d_bwd_serial<bf16_t>, dim3(grid), dim3(kSerialNB), 0, stream, a);
         else    hipLaunchKernelGGL(scan1d_bwd_serial<f32_t>, dim3(grid), dim3(kSerialNB), 0, stream, a);
         KM_HIP_TRY(hipGetLastError());
-    } else if (bwd_chunked_launch(a, pl.shared, a.hist != nullptr, bf, pl.wide, stream) != 0) {
+    } else if (bwd_chunked_launch(a, pl.shared, a.hist != nullptr, bf, wide, stream) != 0) {
         return -1;
     }
     // Slots hold whole [L, 2, N] rows from the workspace's slot offset: with
@@ -1148,8 +1306,8 @@ static int scan1d_bwd_run(const KMScan1DBwd *k, const BwdPlan &pl, bool bf, hipS
     const long blocks = std::min<long>((n + 255) / 256, 8192);
 #define KM_FIN(TT)                                                                                 \
     hipLaunchKernelGGL(scan1d_bwd_finalize<TT>, dim3(blocks), dim3(256), 0, stream, a.slot,       \
-                       pl.G, k->dB, k->dC, k->B, k->L, k->N, k->bc_sb, k->bc_st,                  \
-                       a.dApart, k->dA, k->D * k->N, q4)
+                       G, k->dB, k->dC, k->B, k->L, k->N, k->bc_sb, k->bc_st,                     \
+                       a.dApart, k->dA, k->D * k->N, k->B * a.nseg, q4)
     if (bf) KM_FIN(bf16_t);
     else    KM_FIN(f32_t);
 #undef KM_FIN

@@ -32,6 +32,7 @@
 #include <type_traits>
 
 #include "km_device.hpp"
+#include "scan1d_maps.hpp"
 #include "../km_runtime.hpp"
 #include "kmamba_km.h"
 #include "scan.h"
@@ -63,16 +64,10 @@ struct Scan1DFwdArgs {
     // clamp_flag[b * groups + group] and leaves the sequential re-run to
     // scan1d_clamp_repair; null: the workgroup's own fallback.
     int *clamp_flag;
-    // Maps of the parts of a split sequence that precede its last segment,
-    // [B, nmap, D, N] and [B, nmap, D]: the end state from zero and the sum
-    // of delta of every Lm steps. Written by the map pass, read by the
-    // replay, whose segments are map_per of them long (0: not split).
-    float *seg_h, *seg_dsum;
-    int nmap, Lm, map_per;
-    // [B, D, N] copy of h0 the map pass leaves for the replay where h_final
-    // shares h0's memory (the replay's last segment writes it while earlier
-    // segments may not have started), or null.
-    float *h0_copy;
+    // Replay of a split sequence: the maps before its last segment (see
+    // scan1d_maps.hpp); a segment is map_per of them long (0: not split).
+    const float *seg_h, *seg_dsum;
+    int nmap, map_per;
 };
 
 // Output of one step: the readout, plus Dskip*x and times SiLU(z) when
@@ -661,156 +656,6 @@ static int launch_n16(const Scan1DFwdArgs &a, bool shared, bool hist, hipStream_
 // that whole sequence with the sequential clamped recurrence.
 // ---------------------------------------------------------------------------
 
-// Maps of a split sequence: the end state from zero and the sum of delta of
-// each of its first nmap parts of Lm steps (seg_h, seg_dsum).
-//
-// Only the end state is wanted, so there is nothing to replay and no carry
-// to pass along: each of the workgroup's 8 waves runs its own eighth of the
-// part from a zero state without a barrier, and the 8 maps
-// h -> exp(A * sum delta) h + h_end are composed once at the end. A lane owns
-// a whole channel (all 16 states), which halves the work per step that does
-// not depend on the state (exp, delta * x, addresses) against the replay's
-// two lanes per channel. Bound by VALU issue (decay, B*u and the FMA: 3 of
-// ~3.8 instructions per state update): B1 L4992 D1536 bf16 in 5 segments,
-// whole call 79.2 -> 72.4 us against the map pass that ran the replay kernel's
-// local passes and folds. kMapBlock rows of x, delta and B are in
-// flight ahead of the arithmetic; the wave's B rows go through its own LDS
-// rows, from which every lane reads the same 16 values.
-constexpr int kMapWaves = 8, kMapBlock = 8;
-template <typename T, bool SHARED>
-__global__ void __launch_bounds__(64 * kMapWaves, 4) scan1d_segment_map(Scan1DFwdArgs p) {
-    using IO = bio<T>;
-    constexpr int N = 16, TS = IO::size, MB = kMapBlock, W = kMapWaves, PADC = 65;
-    // Staged B rows of each wave (two blocks), then the waves' end states
-    // [wave][state][channel] (rows padded against bank conflicts).
-    __shared__ __align__(16) float lds[W * N * PADC];
-    __shared__ float sds[W][64];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const unsigned ngroups = static_cast<unsigned>((p.D + 63) / 64);
-    const unsigned wg = static_cast<unsigned>(xcd_remap(blockIdx.x, gridDim.x));
-    const unsigned bs = wg / ngroups, grp = wg - bs * ngroups;
-    const unsigned nmap = static_cast<unsigned>(p.nmap);
-    const long b = bs / nmap;
-    const unsigned seg = bs - static_cast<unsigned>(b) * nmap;
-    const long d0 = static_cast<long>(grp) * 64, d = d0 + lane;
-    const bool dvalid = d < p.D;
-    const long dc = dvalid ? d : p.D - 1;
-    // This wave's steps; every part is whole.
-    const int q = (p.Lm + W - 1) / W;
-    const int ta = min(w * q, p.Lm), nt = min(q, p.Lm - ta);
-    const long row0 = b * p.L + static_cast<long>(seg) * p.Lm + ta;
-    const auto rx = make_rsrc(static_cast<const char *>(p.x) + row0 * p.D * TS, static_cast<long>(nt) * p.D * TS);
-    const auto rdt = make_rsrc(static_cast<const char *>(p.dt) + row0 * p.D * TS, static_cast<long>(nt) * p.D * TS);
-    const long bc0 = b * p.sb + (static_cast<long>(seg) * p.Lm + ta) * p.st;
-    const auto rB = make_rsrc(static_cast<const char *>(p.Bm) + bc0 * TS, static_cast<long>(nt) * p.st * TS);
-    const int rowx = static_cast<int>(p.D) * TS, rowbc = static_cast<int>(p.st) * TS;
-    const int vx = static_cast<int>(dc) * TS;
-    const int vb = SHARED ? (lane & 15) * TS + (lane >> 4) * rowbc : static_cast<int>(dc * p.sd) * TS;
-
-    float X[MB], Dl[MB], rb[2];
-    auto load = [&](int t, float (&xo)[MB], float (&dlo)[MB]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int k = 0; k < MB; ++k) {      // rows past the wave's last read as 0: identity steps
-            xo[k] = IO::ld(rx, vx + (t + k) * rowx, 0);
-            dlo[k] = IO::ld(rdt, vx + (t + k) * rowx, 0);
-        }
-        if constexpr (SHARED) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) rb[i] = IO::ld(rB, vb + (t + 4 * i) * rowbc, 0);
-        }
-    };
-    load(0, X, Dl);
-    // Decays of this lane's channel, exp2(delta * A log2 e), and whether every
-    // channel of the workgroup has A[d, n] = (n + 1) A[d, 0].
-    float Ap[N];
-    bool structured = true;
-#pragma unroll
-    for (int n = 0; n < N; ++n) {
-        const float a = p.A[dc * N + n];
-        structured = structured && a == static_cast<float>(n + 1) * p.A[dc * N];
-        Ap[n] = a * kLog2e;
-    }
-    const bool fast = __builtin_amdgcn_readfirstlane(__syncthreads_and(structured)) != 0;
-    // The powers e1^(n+1) as products of two lower ones (log-depth).
-    auto powers = [&](float e1, float (&e)[N]) __attribute__((always_inline)) {
-        e[0] = e1;
-#pragma unroll
-        for (int n = 1; n < N; ++n) e[n] = e[(n - 1) / 2] * e[n - 1 - (n - 1) / 2];
-    };
-    float h[N], dsum = 0.f;
-#pragma unroll
-    for (int n = 0; n < N; ++n) h[n] = 0.f;
-    float *const rows = lds + w * (2 * MB * N);
-    auto sweep = [&](auto fastc) __attribute__((always_inline)) {
-        constexpr bool FAST = decltype(fastc)::value;
-        for (int t = 0, buf = 0; t < nt; t += MB, buf ^= 1) {
-            float *const tile = rows + buf * (MB * N);
-            if constexpr (SHARED) {
-                tile[lane] = rb[0];
-                tile[64 + lane] = rb[1];
-            }
-            float xs[MB], ds[MB];
-#pragma unroll
-            for (int k = 0; k < MB; ++k) {
-                xs[k] = X[k];
-                ds[k] = Dl[k];
-            }
-            load(t + MB, X, Dl);
-            __builtin_amdgcn_wave_barrier();      // the rows are this wave's own: LDS order suffices
-#pragma unroll
-            for (int k = 0; k < MB; ++k) {
-                float bv[N];
-#pragma unroll
-                for (int n = 0; n < N; ++n)
-                    bv[n] = SHARED ? tile[k * N + n] : IO::ld(rB, vb + n * TS + (t + k) * rowbc, 0);
-                const float u = ds[k] * xs[k];
-                dsum += ds[k];
-                float e[N];
-                if constexpr (FAST) {
-                    powers(exp2_fast(ds[k] * Ap[0]), e);
-                } else {
-#pragma unroll
-                    for (int n = 0; n < N; ++n) e[n] = exp2_fast(ds[k] * Ap[n]);
-                }
-#pragma unroll
-                for (int n = 0; n < N; ++n) h[n] = fmaf(e[n], h[n], bv[n] * u);
-            }
-        }
-    };
-    if (fast) sweep(std::true_type{});
-    else sweep(std::false_type{});
-    __syncthreads();                               // the staged rows are read; their memory is reused
-    sds[w][lane] = dsum;
-#pragma unroll
-    for (int n = 0; n < N; ++n) lds[(w * N + n) * PADC + lane] = h[n];
-    __syncthreads();
-    // Compose the waves' maps in order: state i % 16 of channel i / 16 by
-    // thread i (and i + 512), so the stores are contiguous.
-#pragma unroll
-    for (int i = tid; i < 64 * N; i += 64 * W) {
-        const int n = i & 15, c = i >> 4;
-        const long dd = d0 + c;
-        if (dd < p.D) {
-            const float a2 = p.A[dd * N + n] * kLog2e;
-            float run = 0.f;
-#pragma unroll
-            for (int v = 0; v < W; ++v) run = fmaf(exp2_fast(sds[v][c] * a2), run, lds[(v * N + n) * PADC + c]);
-            p.seg_h[(static_cast<long>(bs) * p.D + dd) * N + n] = run;
-            if (seg == 0 && p.h0_copy) p.h0_copy[(b * p.D + dd) * N + n] = p.h0[(b * p.D + dd) * N + n];
-        }
-    }
-    if (w == 0 && dvalid) {
-        float tot = 0.f;
-#pragma unroll
-        for (int v = 0; v < W; ++v) tot += sds[v][lane];
-        p.seg_dsum[static_cast<long>(bs) * p.D + d] = tot;
-    }
-    // Clamp flags of the replay's 32-channel groups.
-    if (p.clamp_flag && seg == 0 && tid < 2 && d0 + 32 * tid < p.D)
-        p.clamp_flag[b * ((p.D + 31) / 32) + 2 * static_cast<long>(grp) + tid] = 0;
-}
-
 // Re-runs every flagged (batch, channel group) sequence from its start with
 // the sequential clamped recurrence (wave 0 of a one-wave workgroup per
 // pair), writing y, the history and the final state over the segmented
@@ -843,7 +688,7 @@ static long scan1d_split_override() {
     return v;
 }
 
-constexpr int kMaxSegments = 64, kMaxMaps = 64;
+constexpr int kMaxSegments = 64;
 
 // Segment length (a multiple of 64; the last segment may be shorter) for a
 // split launch, or 0 to run unsplit. Only N = 16, and only when the unsplit
@@ -900,13 +745,8 @@ static int launch_segmented(const KMScan1DFwd *k, const Scan1DFwdArgs &base, lon
     constexpr int NPL = 8, NS = 2, DL = 32, WS = 8;
     const long S = (k->L + Ls - 1) / Ls;
     const long groups = (k->D + DL - 1) / DL;
-    // The parts the maps cover: a segment, or the half, quarter or eighth of
-    // it that gives the map pass a workgroup (64 channels) per CU.
-    const long groups64 = (k->D + 63) / 64;
-    long r = 1;
-    while (r < 8 && k->B * groups64 * (S - 1) * r < 256 && (S - 1) * r * 2 <= kMaxMaps && Ls / (2 * r) >= 64) r *= 2;
-    const long nmap = (S - 1) * r;
-    const long grid = k->B * S * groups, mgrid = k->B * nmap * groups64;
+    const long r = map_parts(k->B, k->D, S - 1, Ls), nmap = (S - 1) * r;
+    const long grid = k->B * S * groups;
     const size_t nst = static_cast<size_t>(k->B) * k->D * k->N;
     const size_t st = align_up(sizeof(float) * nst * nmap, 256);
     const size_t sd = align_up(sizeof(float) * k->B * k->D * nmap, 256);
@@ -927,29 +767,21 @@ static int launch_segmented(const KMScan1DFwd *k, const Scan1DFwdArgs &base, lon
     const bool gate = k->z || k->Dskip;
     int *flags = reinterpret_cast<int *>(ws + st + sd);
     // (1) map pass over every segment but the last; clamp flags cleared
-    Scan1DFwdArgs a = base;
-    a.nmap = static_cast<int>(nmap);
-    a.Lm = static_cast<int>(Ls / r);
-    a.seg_h = reinterpret_cast<float *>(ws);
-    a.seg_dsum = reinterpret_cast<float *>(ws + st);
-    a.clamp_flag = k->clamp ? flags : nullptr;
-    a.h0_copy = alias ? reinterpret_cast<float *>(ws + st + sd + sf) : nullptr;
-    a.y = nullptr; a.hfin = nullptr; a.hist = nullptr; a.ckpt = nullptr; a.z = nullptr; a.Dskip = nullptr;
-#define KM_SEG(SH) \
-    hipLaunchKernelGGL((scan1d_segment_map<T, SH>), dim3(static_cast<unsigned>(mgrid)), dim3(64 * kMapWaves), 0, s, a)
-    if (shared) KM_SEG(true); else KM_SEG(false);
-#undef KM_SEG
-    KM_HIP_TRY(hipGetLastError());
+    MapArgs m{k->x, k->delta, k->Bm, k->A, k->L, k->D, k->bc_sb, k->bc_st, k->bc_sd, static_cast<int>(nmap),
+              static_cast<int>(Ls / r), 0, reinterpret_cast<float *>(ws), reinterpret_cast<float *>(ws + st),
+              k->clamp ? flags : nullptr, k->h0,
+              alias ? reinterpret_cast<float *>(ws + st + sd + sf) : nullptr};
+    if (launch_maps<T, false>(m, k->B, s) != 0) return -1;
     // (2) replay every segment from the state its predecessors' maps give
     Scan1DFwdArgs q = base;
     q.nseg = static_cast<int>(S);
     q.Ls = static_cast<int>(Ls);
-    q.seg_h = a.seg_h;
-    q.seg_dsum = a.seg_dsum;
-    q.nmap = a.nmap;
+    q.seg_h = m.seg_h;
+    q.seg_dsum = m.seg_dsum;
+    q.nmap = m.nmap;
     q.map_per = static_cast<int>(r);
-    q.clamp_flag = a.clamp_flag;
-    if (alias) q.h0 = a.h0_copy;
+    q.clamp_flag = m.clamp_flag;
+    if (alias) q.h0 = m.h0_copy;
 #define KM_SEGR(SH, HI, GA) \
     hipLaunchKernelGGL((scan1d_fwd_chunked<T, NPL, NS, WS, 8, SH, HI, !HI && !GA, 2, GA>), \
                        dim3(static_cast<unsigned>(grid)), dim3(64 * WS), 0, s, q)
@@ -965,7 +797,7 @@ static int launch_segmented(const KMScan1DFwd *k, const Scan1DFwdArgs &base, lon
     if (k->clamp) {
         // (3) flagged sequences again, sequentially with the clamp
         Scan1DFwdArgs f = base;
-        if (alias) f.h0 = a.h0_copy;
+        if (alias) f.h0 = m.h0_copy;
         const dim3 g2(static_cast<unsigned>(k->B * groups));
         if (shared) {
             if (hist) hipLaunchKernelGGL((scan1d_clamp_repair<T, NPL, NS, true, true>), g2, dim3(64), 0, s, f, flags);
@@ -1027,7 +859,7 @@ int scan1d_fwd_launch(const KMScan1DFwd *k, hipStream_t stream, bool allow_split
     Scan1DFwdArgs a{k->x, k->delta, k->A, k->Bm, k->Cm, k->y, k->h0, k->h_final, k->h_hist,
                     k->h_ckpt, (k->L + kCkptSteps - 1) / kCkptSteps, k->z, k->Dskip,
                     k->B, k->L, k->D, k->N, k->bc_sb, k->bc_st, k->bc_sd, k->clamp, 1,
-                    static_cast<int>(std::min<long>(k->L, 0x7fffffffL)), nullptr, nullptr, nullptr, 0, 0, 0, nullptr};
+                    static_cast<int>(std::min<long>(k->L, 0x7fffffffL)), nullptr, nullptr, nullptr, 0, 0};
     // The register-blocked kernel addresses each batch element's windows with
     // 32-bit byte offsets; larger problems take the sequential kernel.
     const long es = (k->dtype == KM_BF16) ? 2 : 4;

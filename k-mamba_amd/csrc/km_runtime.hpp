@@ -48,6 +48,7 @@ enum class WsUse : int {
     Scan1DSplit = 0,   // segment end states and delta sums, flags
     Scan1DSegments,    // the same, where only try_reserve may provide it
     Scan1DBwd,         // checkpoints and per-workgroup partial sums
+    Scan1DBwdSegments, // adjoint maps and dA partials of a split backward (try_reserve only)
     Scan1DM1,          // M = 1 backward's per-workgroup ddelta partials
     ScanNDPlan,        // per-level fallback's plan offsets
     ScanNDM3,          // Mamba-3 branch: plan offsets and rotated states

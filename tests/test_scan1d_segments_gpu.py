@@ -8,7 +8,8 @@ import pytest
 
 import kmamba as K
 import oracle as O
-from kmtest import TOL_F32, assert_close, rel_err_cond, rng_for, scan1d_inputs, scan1d_kappa
+from kmtest import (TOL_F32, assert_close, rel_err_cond, rng_for, scan1d_bwd_kappa, scan1d_inputs,
+                    scan1d_kappa)
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -93,3 +94,80 @@ def test_captured_call_takes_no_scratch():
         ky, kh, _ = scan1d_kappa(xi, *(a.cpu().numpy() for a in (dt, A, Bm, Cm)))
         assert rel_err_cond(y.cpu().numpy(), yr, ky) <= TOL_F32
         assert rel_err_cond(hf.cpu().numpy(), hr, kh) <= TOL_F32
+
+
+# --- the backward split over workgroups ------------------------------------------
+
+def _bwd(x, dt, A, Bm, Cm, dy, *, mode, strides, h0=None, hist=None, workspace=None):
+    ins = [T(a) for a in (x, dt, A, Bm, Cm)]
+    Bsz, L, D = x.shape
+    out = [torch.full_like(ins[0], float("nan")), torch.full_like(ins[0], float("nan")),
+           torch.full((D, N), float("nan"), device=DEV), torch.full_like(ins[3], float("nan")),
+           torch.full_like(ins[4], float("nan"))]
+    th0 = None if h0 is None else T(h0)
+    kw = dict(h0=th0, bc_strides=strides)
+    if mode == "hist":
+        kw["h_hist"] = T(hist)
+    elif mode == "ckpt":
+        kw["h_ckpt"] = torch.empty((Bsz, -(-L // 32), D, N), device=DEV)
+        K.scan1d_fwd(*ins, None, h0=th0, h_ckpt=kw["h_ckpt"], bc_strides=strides)
+    args = K.scan1d_bwd_args(*ins, T(dy), *out, **kw)
+    need = K.km_scan1d_bwd_workspace_bytes(C.byref(args))
+    if workspace == "queried":
+        kw["workspace"] = torch.empty(need, dtype=torch.uint8, device=DEV)
+    K.scan1d_bwd(*ins, T(dy), *out, **kw)
+    torch.cuda.synchronize()
+    return [t.cpu().numpy() for t in out], need
+
+
+# Last segments of 1, 9, 31 and 64 steps; the fourth fills the chip only with
+# 16-wave workgroups, the last leaves most of its last wave of them empty.
+BWD = [(1, 1025, 64), (2, 1001, 40), (1, 799, 200), (2, 640, 1536), (1, 1024, 33), (9, 160, 1000)]
+
+
+@pytest.mark.parametrize("Bsz,L,D", BWD)
+@pytest.mark.parametrize("mode", ["hist", "ckpt", "recompute"])
+def test_backward_segments_vs_oracle(Bsz, L, D, mode):
+    x, dt, A, Bm, Cm = scan1d_inputs(Bsz, L, D, N, seed=41)
+    g = rng_for("segments-bwd", Bsz, L, D)
+    if D == 40:
+        A = (A * g.uniform(0.02, 1.0, size=A.shape)).astype(np.float32)   # generic, slow decays
+    h0 = g.standard_normal((Bsz, D, N)).astype(np.float32)
+    dy = g.standard_normal((Bsz, L, D)).astype(np.float32)
+    per_channel = D in (40, 33)
+    strides = (L * N, N, 0)
+    if per_channel:
+        strides = (L * D * N, D * N, N)
+        Bm, Cm = ((g.standard_normal((Bsz, L, D, N)) * 0.25).astype(np.float32) for _ in range(2))
+    kw = dict(h0=h0, bc_strides=strides, nthreads=8, fast=True)
+    hh = O.scan1d_batched(x, dt, A, Bm, Cm, hist=True, **kw)[2]
+    ref = O.scan1d_batched_backward(x, dt, A, Bm, Cm, dy, hh, **kw)
+    kap = scan1d_bwd_kappa(x, dt, A, Bm, Cm, dy, h0=h0, bc_strides=strides)
+    got, need = _bwd(x, dt, A, Bm, Cm, dy, mode=mode, strides=strides, h0=h0, hist=hh)
+    for n, a, r, k in zip(("dx", "ddelta", "dA", "dB", "dC"), got, ref, kap):
+        assert_close(a, r, TOL_F32, n, k)
+    # The caller's own workspace of the queried size: the same bits.
+    again, _ = _bwd(x, dt, A, Bm, Cm, dy, mode=mode, strides=strides, h0=h0, hist=hh, workspace="queried")
+    for a, b in zip(got, again):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+def test_backward_segments_clamped_states():
+    # States leave [-1000, 1000] around steps 500-505 of 1001: the segments
+    # they pass through recompute them with the per-step clamp.
+    Bsz, L, D = 2, 1001, 40
+    x, dt, A, Bm, Cm = scan1d_inputs(Bsz, L, D, N, seed=42)
+    g = rng_for("segments-clamp")
+    A = (A * g.uniform(0.001, 0.01, size=A.shape)).astype(np.float32)
+    Bm = Bm.copy()
+    Bm[:, 500:506] *= 4000.0
+    dy = g.standard_normal((Bsz, L, D)).astype(np.float32)
+    strides = (L * N, N, 0)
+    kw = dict(bc_strides=strides, nthreads=8, fast=True)
+    hh = O.scan1d_batched(x, dt, A, Bm, Cm, hist=True, **kw)[2]
+    assert np.abs(hh).max() == 1000.0
+    ref = O.scan1d_batched_backward(x, dt, A, Bm, Cm, dy, hh, **kw)
+    kap = scan1d_bwd_kappa(x, dt, A, Bm, Cm, dy, bc_strides=strides)
+    got, _ = _bwd(x, dt, A, Bm, Cm, dy, mode="ckpt", strides=strides)
+    for n, a, r, k in zip(("dx", "ddelta", "dA", "dB", "dC"), got, ref, kap):
+        assert_close(a, r, TOL_F32, n, k)
