@@ -6,7 +6,7 @@
 //
 // Launches, no atomics:
 //  0. Neighbour flags of every point (successor / predecessor per axis), so
-//     the sweeps below do no index division.
+//     the per-level sweep and the untiled passes do no index division.
 //  1. The adjoint state g[p] = dy[p] C[p] + sum_a e_a[p+s_a] g[p+s_a] flows
 //     against the forward's wavefront, g kept in dB's memory (no P x D x M
 //     scratch): 2D and 3D grids with D*M a multiple of 64 by tile bands (one
@@ -48,6 +48,7 @@ struct NdBwdArgs {
     const uint16_t *nbr;    // per point: bit a = has a successor on axis a, bit 8 + a = a predecessor
     long P, D, M;
     long dims[8], strides[8];
+    int gext;               // gradient tiles: points per row (2D) or rows per plane (3D)
 };
 
 // Neighbour flags of every point: bit a = a successor on axis a, bit 8 + a
@@ -786,14 +787,14 @@ __device__ __forceinline__ void grad_flush(const GradWin &w, const float *stage,
 }
 
 // The gradient pass over tiles of a 2D grid: workgroup x takes tile x (TR
-// rows x TW points) and walks it column by column, down each column, so the
+// rows x a.gext points) and walks it column by column, down each column, so the
 // state of the point above is the previous step's and the one to the left
 // is the previous column's (kept per row): only the tile's first row and
 // first column read a predecessor's state from memory. A column's TR points
 // load one column ahead of the arithmetic.
-template <int TR, int TW, int MM>
+template <int TR, int MM>
 __global__ void __launch_bounds__(256) nd_adjoint_grads_tile2d(NdBwdArgs a) {
-    const long DM = a.D * MM;
+    const long DM = a.D * MM, TW = a.gext;
     // Tile and channel block, numbered XCD-major: the channel blocks of a
     // tile, which share the x / dy / delta row lines, run on one XCD.
     long tile, cbx;
@@ -882,16 +883,16 @@ __global__ void __launch_bounds__(256) nd_adjoint_grads_tile2d(NdBwdArgs a) {
     }
 }
 
-// The same over tiles of a 3D grid (TP planes x TR rows x TW points), TPW
+// The same over tiles of a 3D grid (TP planes x TR = a.gext rows x TW points), TPW
 // consecutive tiles per workgroup (fewer dA partials to add afterwards): the
 // walk goes row by row, point by point, through the tile's planes at each
 // (row, point), so the plane predecessor is the previous step's state, the
 // point to the left the previous point's (per plane) and the row above the
 // previous row's (per point and plane, TW x TP registers). The TP points of
 // a (row, point) load one group ahead of the arithmetic.
-template <int TP, int TR, int TW, int TPW, int MM>
+template <int TP, int TW, int TPW, int MM>
 __global__ void __launch_bounds__(256) nd_adjoint_grads_tile3d(NdBwdArgs a) {
-    const long DM = a.D * MM;
+    const long DM = a.D * MM, TR = a.gext;
     long blk, cbx;                  // tiles [blk * TPW, +TPW), channel block (XCD-major)
     xcd_tile(blk, cbx);
     const long c0 = cbx * 256 + threadIdx.x;
@@ -1555,8 +1556,17 @@ static void sum_dA(float *part, float *dA, long nbx, long n, hipStream_t st) {
     }
 }
 
-constexpr int kGradTR2 = 8, kGradTW2 = 64;                  // 2D gradient tiles (rows, points)
-constexpr int kGradTP3 = 4, kGradTR3 = 8, kGradTW3 = 8;     // 3D gradient tiles
+// Gradient tiles: 2D kGradTR2 rows x up to kGradTW2 points, 3D kGradTP3 planes
+// x up to kGradTR3 rows x kGradTW3 points. A workgroup walks its tile point by
+// point, so on a grid whose largest tiles would not give each CU
+// kGradGroups / 256 workgroups the extent along the walk is halved until they
+// do (not below kGradMin: the first column or row of a tile reads its
+// predecessors' states again). 45 x 61 points, D*M = 1536: 36 tiles of 64
+// points 150 us, 288 of 8 points 34 us.
+constexpr int kGradTR2 = 8, kGradTW2 = 64;
+constexpr int kGradTP3 = 4, kGradTR3 = 8, kGradTW3 = 8;
+constexpr long kGradGroups = 1024;
+constexpr int kGradMin2 = 8, kGradMin3 = 2;
 constexpr int kGradTPW3 = 1;                                 // 3D tiles per workgroup (2 and 4 measured slower)
 
 // The adjoint sweep's dataflow tiles per axis (0 past nd).
@@ -1576,6 +1586,7 @@ struct NdBwdShape {
     long P, nd, D, M;
     bool lanes;          // M a power of two <= 64: nd_adjoint_grads_lanes
     bool gtiles;         // ... and 2D or 3D: the tile walks
+    int gext;            // their extent along the walk (NdBwdArgs::gext)
     bool atile2;         // 2D adjoint state by tile bands
     int db;
     long qc, nbx, nby;
@@ -1641,12 +1652,19 @@ static bool nd_bwd_shape(const KMScanNDBwd *a, NdBwdShape &s) {
         s.gtiles = win < 2147483000.0;
     }
     if (s.gtiles) {
-        const long t2[2] = {kGradTR2, kGradTW2}, t3[3] = {kGradTP3, kGradTR3, kGradTW3};
-        long nt = 1;
-        for (long ax = 0; ax < s.nd; ++ax) {
-            const long te = s.nd == 2 ? t2[ax] : t3[ax];
-            nt *= (a->dims[ax] + te - 1) / te;
-        }
+        s.gext = s.nd == 2 ? kGradTW2 : kGradTR3;
+        auto tiles = [&](int e) {
+            const long t2[2] = {kGradTR2, e}, t3[3] = {kGradTP3, e, kGradTW3};
+            long nt = 1;
+            for (long ax = 0; ax < s.nd; ++ax) {
+                const long te = s.nd == 2 ? t2[ax] : t3[ax];
+                nt *= (a->dims[ax] + te - 1) / te;
+            }
+            return nt;
+        };
+        const int emin = s.nd == 2 ? kGradMin2 : kGradMin3;
+        while (s.gext > emin && tiles(s.gext) * s.nby < kGradGroups) s.gext /= 2;
+        const long nt = tiles(s.gext);
         const long nb = s.nd == 2 ? nt : (nt + kGradTPW3 - 1) / kGradTPW3;
         // Tiles go on the grid's y dimension.
         if (nb <= 65535) s.nbx = nb;
@@ -1741,10 +1759,9 @@ static void grads_tile_go(const NdBwdArgs &args, const NdBwdShape &s, hipStream_
     // tile, next to the neighbouring tiles' states it reads.
     const dim3 grid(static_cast<unsigned>(s.nby), static_cast<unsigned>(s.nbx));
     if constexpr (ND == 2)
-        hipLaunchKernelGGL((nd_adjoint_grads_tile2d<kGradTR2, kGradTW2, MM>), grid, dim3(256), 0, st, args);
+        hipLaunchKernelGGL((nd_adjoint_grads_tile2d<kGradTR2, MM>), grid, dim3(256), 0, st, args);
     else
-        hipLaunchKernelGGL((nd_adjoint_grads_tile3d<kGradTP3, kGradTR3, kGradTW3, kGradTPW3, MM>), grid, dim3(256),
-                           0, st, args);
+        hipLaunchKernelGGL((nd_adjoint_grads_tile3d<kGradTP3, kGradTW3, kGradTPW3, MM>), grid, dim3(256), 0, st, args);
 }
 template <int ND>
 static void grads_tile_launch(const NdBwdArgs &args, const NdBwdShape &s, hipStream_t st) {
@@ -1960,6 +1977,7 @@ int km_scannd_bwd(const KMScanNDBwd *a, void *stream) {
     args.nbr = reinterpret_cast<const uint16_t *>(ws + s.offs_bytes);
     args.part = reinterpret_cast<float *>(ws + s.offs_bytes + s.nbr_bytes);
     args.P = s.P; args.D = s.D; args.M = s.M;
+    args.gext = s.gtiles ? s.gext : 0;
     long stride = 1;
     for (long ax = s.nd - 1; ax >= 0; --ax) {
         args.dims[ax] = a->dims[ax];
@@ -2076,7 +2094,9 @@ int km_scannd_bwd(const KMScanNDBwd *a, void *stream) {
     }
     char *tile_ws = ws + s.offs_bytes + s.nbr_bytes + s.part_bytes;
     int rc = 0;
-    hipLaunchKernelGGL(km::nd_adjoint_flags, dim3(static_cast<unsigned>((s.P + 255) / 256)), dim3(256), 0, st,
+    // Only the per-level sweep and the untiled gradient passes read the flags.
+    if (plan || !s.gtiles)
+        hipLaunchKernelGGL(km::nd_adjoint_flags, dim3(static_cast<unsigned>((s.P + 255) / 256)), dim3(256), 0, st,
                        args, s.nd, reinterpret_cast<uint16_t *>(ws + s.offs_bytes));
     // The host tables must outlive their copies: wait for them.
     if ((plan && hipMemcpyAsync(ws, plan->level_offsets, sizeof(long) * s.P, hipMemcpyHostToDevice, st) !=
