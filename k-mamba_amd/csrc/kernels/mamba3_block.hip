@@ -8,16 +8,14 @@
 //   y_t[r] = sum_n C_t[r, n] h_t[n],  out_t = x_t + W_out y_t
 // with alpha = e^(dt a_n), beta = (1 - lambda) dt alpha, gamma = lambda dt.
 //
-// GPU schedule (five kernels, one pass each):
+// GPU schedule (three kernels after the parameters' upload):
 //   1. proj: P = X . Wcat^T, the R + 2 + 2NR controller rows of every token
-//      at once (fp32 SGEMM, 64x64 register-blocked tiles through LDS).
-//   2. prep: per (t, n) the step's decay a_t = alpha and its drive
-//      c_t = beta Bu_{t-1} + gamma Bu_t, which do not depend on h.
-//   3. scan: h_t = a_t * R(theta) h_{t-1} + c_t per state pair, a chunked
-//      scan of 2x2 maps: one wave per (batch element, pair), one lane per
-//      chunk of steps.
-//   4. readout: Y[t, r] = sum_n C_t[r, n] h_t[n].
-//   5. out: out = x + W_out Y.
+//      at once (fp32 matrix cores).
+//   2. scan: per step the decay a_t = alpha and the drive c_t = beta Bu_{t-1}
+//      + gamma Bu_t, which do not depend on h, and h_t = a_t * R(theta)
+//      h_{t-1} + c_t per state pair, a chunked scan of 2x2 maps: a workgroup
+//      per (batch element, pair), a thread per chunk of steps.
+//   3. out: Y[t, r] = sum_n C_t[r, n] h_t[n] and out = x + W_out Y.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -40,10 +38,12 @@ struct M3Args {
     const float *A;       // [N]
     const float *bB, *bC; // [NR]
     const float *theta;   // [N/2]
-    float *P;             // [T, J]
-    float *a, *c;         // [T, N]
-    float *H;             // [T, N]
-    float *Y;             // [T, R]
+    // Time runs along the rows (of Tp >= T values), so that the scan's threads,
+    // each on a few consecutive steps, read and write whole lines together.
+    float *P;             // [J, Tp]
+    float *H;             // [N, Tp]
+    long Tp;
+    float *Y;             // [T, R] (general output path)
     long T, L, D, N, R, J;
     int has_delta, has_lambda;
     float dt_scale, dt_min, dt_max;
@@ -128,26 +128,27 @@ __global__ void __launch_bounds__(256) m3_proj(M3Args p) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const long jj = j0 + tx * 4 + j;
-            if (jj < p.J) p.P[t * p.J + jj] = acc[i][j];
+            if (jj < p.J) p.P[jj * p.Tp + t] = acc[i][j];
         }
     }
 }
 
 // The same projections on the fp32 matrix cores (v_mfma_f32_16x16x4_f32),
-// for D a multiple of 4: a wave computes 16*kM3TM tokens x 16*TJ rows (each
-// W fragment serves kM3TM token tiles) over every
-// kM3Split-th 16-wide k block (the waves of a workgroup split K; wave 0 adds
-// the other waves' partials from LDS in wave order). Lane l supplies token /
+// for D a multiple of 4: a wave computes 16*TM tokens x 16*TJ rows (each
+// W fragment serves TM token tiles) over every
+// kM3Split-th 16-wide k block (the waves of a workgroup split K; the partials
+// are added in wave order through LDS, every wave taking its share of the
+// sums). Lane l supplies token /
 // row l % 16 and, for k block b, the 16 contiguous bytes k = 16b + 4(l/16)
 // .. +3, one element per MFMA step: the k order within a dot product is
 // free, and both operands use the same one. Operands come from global memory
 // straight into registers, one block ahead; rows past T or J read 0.
 using f32x4v = float __attribute__((ext_vector_type(4)));
-constexpr int kM3Split = 8, kM3TM = 4;
-template <int TJ>
+constexpr int kM3Split = 8;
+template <int TJ, int TM>
 __global__ void __launch_bounds__(64 * kM3Split) m3_proj_mfma(M3Args p) {
-    constexpr int TM = kM3TM;
-    __shared__ float red[kM3Split - 1][TM * TJ * 4][64];
+    constexpr int NV = TM * TJ * 4;               // accumulators per lane
+    __shared__ float red[kM3Split][NV][64];
     constexpr unsigned kDrop = 0x80000000u;
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -195,89 +196,72 @@ __global__ void __launch_bounds__(64 * kM3Split) m3_proj_mfma(M3Args p) {
         __builtin_amdgcn_sched_barrier(0);
         mfma_blk(a1, b1);
     }
-    if (w > 0) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TJ; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) red[w - 1][(i * TJ + j) * 4 + r][lane] = acc[i][j][r];
-    }
-    __syncthreads();
-    if (w != 0) return;
-#pragma unroll 1
-    for (int v = 0; v < kM3Split - 1; ++v)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TJ; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[i][j][r] += red[v][(i * TJ + j) * 4 + r][lane];
-    // Accumulator r of lane l: token 4(l/16) + r, row l % 16 of its tile.
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-            const long jj = j0 + j * 16 + fr;
+        for (int j = 0; j < TJ; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const long t = t0 + i * 16 + 4 * fg + r;
-                if (t < p.T && jj < p.J) p.P[t * p.J + jj] = acc[i][j][r];
-            }
+            for (int r = 0; r < 4; ++r) red[w][(i * TJ + j) * 4 + r][lane] = acc[i][j][r];
+    __syncthreads();
+    // Accumulator r of lane l: token 4(l/16) + r, row l % 16 of its tile. A
+    // wave takes whole tiles: its four sums are four consecutive steps.
+    for (int e = w; e < TM * TJ; e += kM3Split) {
+        const int j = e % TJ, i = e / TJ;
+        const long jj = j0 + j * 16 + fr, t = t0 + i * 16 + 4 * fg;
+        f32x4v sum;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            sum[r] = red[0][e * 4 + r][lane];
+#pragma unroll
+            for (int v = 1; v < kM3Split; ++v) sum[r] += red[v][e * 4 + r][lane];
         }
+        if (jj < p.J) {
+            float *dst = p.P + jj * p.Tp + t;       // Tp and t are multiples of 4
+            if (t + 4 <= p.Tp) *reinterpret_cast<f32x4v *>(dst) = sum;
+        }
+    }
 }
 
 // ---- 2. per-step decay and drive --------------------------------------------
 __device__ __forceinline__ float silu_f(float v) { return v / (1.f + expf(-v)); }
 
-__device__ __forceinline__ void m3_ctrl(const M3Args &p, long t, float &dt, float &lam) {
-    const float *row = p.P + t * p.J;
+__device__ __forceinline__ void m3_ctrl_of(const M3Args &p, float rd, float rl, float &dt, float &lam) {
     if (p.has_delta) {
-        float v = logf(1.f + expf(row[p.R]));
+        float v = logf(1.f + expf(rd));
         v = v < p.dt_min ? p.dt_min : v;
         dt = v > p.dt_max ? p.dt_max : v;
     } else {
         dt = p.dt_scale;
     }
-    lam = p.has_lambda ? 1.f / (1.f + expf(-row[p.R + 1])) : 0.5f;
+    lam = p.has_lambda ? 1.f / (1.f + expf(-rl)) : 0.5f;
+}
+__device__ __forceinline__ void m3_ctrl(const M3Args &p, long t, float &dt, float &lam) {
+    m3_ctrl_of(p, p.P[p.R * p.Tp + t], p.P[(p.R + 1) * p.Tp + t], dt, lam);
 }
 
 // Bu_t[n] = sum_r (W_B x_t + b_B)[r, n] * SiLU(W_in x_t)[r].
 __device__ __forceinline__ float m3_bu(const M3Args &p, long t, long n) {
-    const float *row = p.P + t * p.J;
     float s = 0.f;
     for (long r = 0; r < p.R; ++r)
-        s += (row[p.R + 2 + r * p.N + n] + p.bB[r * p.N + n]) * silu_f(row[r]);
+        s += (p.P[(p.R + 2 + r * p.N + n) * p.Tp + t] + p.bB[r * p.N + n]) * silu_f(p.P[r * p.Tp + t]);
     return s;
 }
 
-__global__ void __launch_bounds__(256) m3_prep(M3Args p) {
-    const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= p.T * p.N) return;
-    const long t = i / p.N, n = i % p.N;
-    const long l = t % p.L;                            // step within the sequence
-    float dt, lam;
-    m3_ctrl(p, t, dt, lam);
-    const float alpha = expf(dt * p.A[n]);
-    const float bu = m3_bu(p, t, n);
-    const float pbu = (l > 0) ? m3_bu(p, t - 1, n) : 0.f;
-    p.a[i] = alpha;
-    p.c[i] = (1.f - lam) * dt * alpha * pbu + lam * dt * bu;
-}
-
-// ---- 3. the recurrence ------------------------------------------------------
+// ---- the recurrence ------------------------------------------------------
 // Per state pair (2i, 2i+1) of one batch element, h_t = M_t h_{t-1} + c_t
 // with M_t = diag(a0_t, a1_t) R(theta): a linear recurrence of 2x2 maps, so
 // it runs as a chunked scan. One workgroup of kM3ScanW waves per (batch
 // element, pair); thread k owns the chunk of CH = ceil(L / (64 kM3ScanW))
-// consecutive steps. (1) Each thread composes its chunk's map h -> P h + v
-// from a zero state. (2) An inclusive scan of the maps across the lanes of
+// consecutive steps. (1) Each thread forms its steps' decays and drives from
+// the controller rows and composes its chunk's map h -> P h + v from a zero
+// state. (2) An inclusive scan of the maps across the lanes of
 // each wave (Hillis-Steele, lane shuffles), then the waves' total maps
 // through LDS, give every chunk the state entering it. (3) Each thread
 // replays its steps from that state with the sequential step formula,
 // writing H. An odd last state has no partner: M_t = diag(a0_t, 0) and no
-// rotation.
-constexpr int kM3ScanW = 4;
+// rotation. ONE: the chunk is at most kM3Chunk steps, whose decays and drives
+// stay in registers for the replay (longer chunks form them again).
+constexpr int kM3ScanW = 4, kM3Chunk = 8;
 __device__ __forceinline__ void m3_step(float a0, float a1, float cs, float sn, bool pair,
                                         float c0, float c1, float &h0, float &h1) {
     if (pair) {
@@ -289,6 +273,7 @@ __device__ __forceinline__ void m3_step(float a0, float a1, float cs, float sn, 
     }
 }
 
+template <bool ONE>
 __global__ void __launch_bounds__(64 * kM3ScanW) m3_scan(M3Args p, long npairs) {
     __shared__ float wmap[kM3ScanW][6];          // each wave's total map (P, v)
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -300,19 +285,92 @@ __global__ void __launch_bounds__(64 * kM3ScanW) m3_scan(M3Args p, long npairs) 
     const long L = p.L, N = p.N;
     const long CH = (L + 64 * kM3ScanW - 1) / (64 * kM3ScanW);
     const long l0 = tid * CH, l1 = min(l0 + CH, L);
-    const float *ab = p.a + b * L * N, *cb = p.c + b * L * N;
+    const long tb = b * L;
+    const float A0 = p.A[n0], A1 = pair ? p.A[n1] : 0.f;
+    // Decay and drive of both states at step l; (q0, q1) is Bu of step l - 1
+    // on entry and of step l on return.
+    auto step = [&](long l, float &q0, float &q1, float &a0, float &a1, float &c0, float &c1) {
+        const long t = tb + l;
+        float dt, lam;
+        m3_ctrl(p, t, dt, lam);
+        const float b0 = m3_bu(p, t, n0), b1 = pair ? m3_bu(p, t, n1) : 0.f;
+        a0 = expf(dt * A0);
+        a1 = pair ? expf(dt * A1) : 0.f;
+        c0 = (1.f - lam) * dt * a0 * q0 + lam * dt * b0;
+        c1 = (1.f - lam) * dt * a1 * q1 + lam * dt * b1;
+        q0 = b0;
+        q1 = b1;
+    };
+    // ONE: every step's controller values are loaded together (steps past the
+    // chunk reload its last one), one memory latency for the chunk. Entry u is
+    // step l0 - 1 + u.
+    constexpr int KU = ONE ? kM3Chunk + 1 : 1;
+    float kb0[KU], kb1[KU], kd[KU], kl[KU];
+    const bool prev = l0 > 0 && l0 < l1;
+    if constexpr (ONE) {
+        int at[KU];
+        const float *Pb = p.P + tb;
+#pragma unroll
+        for (int u = 0; u < KU; ++u) {
+            at[u] = static_cast<int>(std::min(std::max(l0 - 1 + u, 0L), L - 1));
+            kb0[u] = 0.f;
+            kb1[u] = 0.f;
+            kd[u] = Pb[p.R * p.Tp + at[u]];
+            kl[u] = Pb[(p.R + 1) * p.Tp + at[u]];
+        }
+        for (long r = 0; r < p.R; ++r) {
+            const long o = p.R + 2 + r * N;
+            const float c0 = p.bB[r * N + n0], c1 = pair ? p.bB[r * N + n1] : 0.f;
+            float zz[KU], x0[KU], x1[KU];
+#pragma unroll
+            for (int u = 0; u < KU; ++u) {
+                zz[u] = Pb[r * p.Tp + at[u]];
+                x0[u] = Pb[(o + n0) * p.Tp + at[u]];
+                x1[u] = Pb[(o + (pair ? n1 : n0)) * p.Tp + at[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < KU; ++u) {
+                const float sz = silu_f(zz[u]);
+                kb0[u] += (x0[u] + c0) * sz;
+                kb1[u] += pair ? (x1[u] + c1) * sz : 0.f;
+            }
+        }
+    }
+    const float e0 = ONE ? 0.f : prev ? m3_bu(p, tb + l0 - 1, n0) : 0.f;
+    const float e1 = ONE ? 0.f : prev && pair ? m3_bu(p, tb + l0 - 1, n1) : 0.f;
 
     // (1) chunk map: P (2x2) and v, composed step by step from identity / 0.
     float P00 = 1.f, P01 = 0.f, P10 = 0.f, P11 = 1.f, v0 = 0.f, v1 = 0.f;
-    for (long l = l0; l < l1; ++l) {
-        const float a0 = ab[l * N + n0], c0 = cb[l * N + n0];
-        const float a1 = pair ? ab[l * N + n1] : 0.f, c1 = pair ? cb[l * N + n1] : 0.f;
+    float ka0[ONE ? kM3Chunk : 1], ka1[ONE ? kM3Chunk : 1], kc0[ONE ? kM3Chunk : 1], kc1[ONE ? kM3Chunk : 1];
+    auto compose = [&](float a0, float a1, float c0, float c1) {
         const float m00 = pair ? a0 * cs : a0, m01 = pair ? -a0 * sn : 0.f;
         const float m10 = a1 * sn, m11 = a1 * cs;
         const float q00 = m00 * P00 + m01 * P10, q01 = m00 * P01 + m01 * P11;
         const float q10 = m10 * P00 + m11 * P10, q11 = m10 * P01 + m11 * P11;
         P00 = q00; P01 = q01; P10 = q10; P11 = q11;
         m3_step(a0, a1, cs, sn, pair, c0, c1, v0, v1);
+    };
+    float q0 = e0, q1 = e1;
+    if constexpr (ONE) {
+#pragma unroll
+        for (int u = 0; u < kM3Chunk; ++u) {
+            if (l0 + u < l1) {
+                float dt, lam;
+                m3_ctrl_of(p, kd[u + 1], kl[u + 1], dt, lam);
+                const float pb0 = l0 + u > 0 ? kb0[u] : 0.f, pb1 = l0 + u > 0 ? kb1[u] : 0.f;
+                ka0[u] = expf(dt * A0);
+                ka1[u] = pair ? expf(dt * A1) : 0.f;
+                kc0[u] = (1.f - lam) * dt * ka0[u] * pb0 + lam * dt * kb0[u + 1];
+                kc1[u] = (1.f - lam) * dt * ka1[u] * pb1 + lam * dt * kb1[u + 1];
+                compose(ka0[u], ka1[u], kc0[u], kc1[u]);
+            }
+        }
+    } else {
+        for (long l = l0; l < l1; ++l) {
+            float a0, a1, c0, c1;
+            step(l, q0, q1, a0, a1, c0, c1);
+            compose(a0, a1, c0, c1);
+        }
     }
     // (2) inclusive scan over the wave's lanes: (P, v) <- (P, v) o (P', v')
     // of lane - d; then the waves' totals.
@@ -344,33 +402,43 @@ __global__ void __launch_bounds__(64 * kM3ScanW) m3_scan(M3Args p, long npairs) 
     }
     // (3) replay from the state after the previous chunk: lane k > 0 of the
     // wave starts from lane k-1's inclusive map applied to V.
-    const float e00 = __shfl_up(P00, 1), e01 = __shfl_up(P01, 1);
-    const float e10 = __shfl_up(P10, 1), e11 = __shfl_up(P11, 1);
+    const float i00 = __shfl_up(P00, 1), i01 = __shfl_up(P01, 1);
+    const float i10 = __shfl_up(P10, 1), i11 = __shfl_up(P11, 1);
     const float w0 = __shfl_up(v0, 1), w1 = __shfl_up(v1, 1);
     float h0 = V0, h1 = V1;
     if (lane > 0) {
-        h0 = e00 * V0 + e01 * V1 + w0;
-        h1 = e10 * V0 + e11 * V1 + w1;
+        h0 = i00 * V0 + i01 * V1 + w0;
+        h1 = i10 * V0 + i11 * V1 + w1;
     }
-    float *Hb = p.H + b * L * N;
-    for (long l = l0; l < l1; ++l) {
-        const float a0 = ab[l * N + n0], c0 = cb[l * N + n0];
-        const float a1 = pair ? ab[l * N + n1] : 0.f, c1 = pair ? cb[l * N + n1] : 0.f;
+    float *H0 = p.H + n0 * p.Tp + tb, *H1 = p.H + (pair ? n1 : n0) * p.Tp + tb;
+    auto emit = [&](long l, float a0, float a1, float c0, float c1) {
         m3_step(a0, a1, cs, sn, pair, c0, c1, h0, h1);
-        Hb[l * N + n0] = h0;
-        if (pair) Hb[l * N + n1] = h1;
+        H0[l] = h0;
+        if (pair) H1[l] = h1;
+    };
+    if constexpr (ONE) {
+#pragma unroll
+        for (int u = 0; u < kM3Chunk; ++u)
+            if (l0 + u < l1) emit(l0 + u, ka0[u], ka1[u], kc0[u], kc1[u]);
+    } else {
+        q0 = e0;
+        q1 = e1;
+        for (long l = l0; l < l1; ++l) {
+            float a0, a1, c0, c1;
+            step(l, q0, q1, a0, a1, c0, c1);
+            emit(l, a0, a1, c0, c1);
+        }
     }
 }
 
-// ---- 4. readout, 5. output ---------------------------------------------------
+// ---- 3. readout and output ---------------------------------------------------
 __global__ void __launch_bounds__(256) m3_readout(M3Args p) {
     const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
     if (i >= p.T * p.R) return;
     const long t = i / p.R, r = i % p.R;
-    const float *row = p.P + t * p.J + p.R + 2 + p.N * p.R + r * p.N;
-    const float *h = p.H + t * p.N;
+    const float *C = p.P + (p.R + 2 + p.N * p.R + r * p.N) * p.Tp + t;
     float s = 0.f;
-    for (long n = 0; n < p.N; ++n) s = fmaf(row[n] + p.bC[r * p.N + n], h[n], s);
+    for (long n = 0; n < p.N; ++n) s = fmaf(C[n * p.Tp] + p.bC[r * p.N + n], p.H[n * p.Tp + t], s);
     p.Y[i] = s;
 }
 
@@ -383,24 +451,78 @@ __global__ void __launch_bounds__(256) m3_out(M3Args p) {
     p.out[i] = p.x[i] + s;
 }
 
-// The same for D a multiple of 4 and 16-byte aligned x / out: thread (t, q)
-// handles channels 4q .. 4q+3 of token t with 16-byte loads and stores (no
-// per-element index division).
+// Both for D a multiple of 4 and 16-byte aligned x / out: a workgroup takes
+// kM3OutT tokens and up to 1024 channels. 16 threads per token form Y (each
+// the states n, n + 16, ..., then a sum over the threads through LDS), and
+// each thread then handles 4 channels of every token with 16-byte loads
+// and stores, W_out's rows read once. Bound by HBM (x read, out written).
+// T 16384, D 1024: 20.7 us (6.2 TB/s; a workgroup per token, after a readout
+// kernel of its own, took 22.9 + 5.9 us).
+constexpr int kM3OutT = 16, kM3OutR = 64;
 __global__ void __launch_bounds__(256) m3_out4(M3Args p) {
-    const long q = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
-    if (4 * q >= p.D) return;
-    for (long t = blockIdx.y; t < p.T; t += gridDim.y) {
-        const long i = t * p.D + 4 * q;
-        float4 v = *reinterpret_cast<const float4 *>(p.x + i);
-        for (long r = 0; r < p.R; ++r) {
-            const float y = p.Y[t * p.R + r];
-            v.x = fmaf(p.W_out[(4 * q + 0) * p.R + r], y, v.x);
-            v.y = fmaf(p.W_out[(4 * q + 1) * p.R + r], y, v.y);
-            v.z = fmaf(p.W_out[(4 * q + 2) * p.R + r], y, v.z);
-            v.w = fmaf(p.W_out[(4 * q + 3) * p.R + r], y, v.w);
-        }
-        *reinterpret_cast<float4 *>(p.out + i) = v;
+    __shared__ float ys[kM3OutT][kM3OutR];
+    __shared__ float part[16][kM3OutT + 1];
+    const int tid = threadIdx.x, tt = tid & 15, ln = tid >> 4;
+    const long t0 = static_cast<long>(blockIdx.y) * kM3OutT;
+    const int nt = static_cast<int>(std::min<long>(kM3OutT, p.T - t0));
+    const long q = static_cast<long>(blockIdx.x) * 256 + tid;
+    const bool on = 4 * q < p.D;
+    const int R = static_cast<int>(p.R);
+    const long i0 = t0 * p.D + (on ? 4 * q : 0);
+    // The first tokens' rows of x are on their way while Y is formed.
+    constexpr int AH = 4;
+    float4 xv[AH];
+#pragma unroll
+    for (int u = 0; u < AH; ++u) xv[u] = *reinterpret_cast<const float4 *>(p.x + i0 + std::min(u, nt - 1) * p.D);
+    const long t = t0 + std::min(tt, nt - 1);
+    for (int r = 0; r < R; ++r) {
+        const float *C = p.P + (R + 2 + p.N * R + r * p.N) * p.Tp + t;
+        float s = 0.f;
+        for (long n = ln; n < p.N; n += 16) s = fmaf(C[n * p.Tp] + p.bC[r * p.N + n], p.H[n * p.Tp + t], s);
+        part[ln][tt] = s;
+        __syncthreads();
+        // Thread (token tid / 16, term tid % 16): the terms' sum over 16 lanes.
+        float v = part[tid & 15][tid >> 4];
+        v += dpp<0x128>(v);                       // row_ror:8, :4, :2, :1
+        v += dpp<0x124>(v);
+        v += dpp<0x122>(v);
+        v += dpp<0x121>(v);
+        if ((tid & 15) == 0) ys[tid >> 4][r] = v;
+        __syncthreads();
     }
+    if (!on) return;
+    for (int u0 = 0; u0 < nt; u0 += AH) {
+        float4 v[AH];
+#pragma unroll
+        for (int u = 0; u < AH; ++u) {
+            v[u] = xv[u];
+            xv[u] = *reinterpret_cast<const float4 *>(p.x + i0 + std::min(u0 + AH + u, nt - 1) * p.D);
+        }
+        for (int r = 0; r < R; ++r) {
+            const float w0 = p.W_out[(4 * q + 0) * R + r], w1 = p.W_out[(4 * q + 1) * R + r];
+            const float w2 = p.W_out[(4 * q + 2) * R + r], w3 = p.W_out[(4 * q + 3) * R + r];
+#pragma unroll
+            for (int u = 0; u < AH; ++u) {
+                const float y = ys[std::min(u0 + u, nt - 1)][r];
+                v[u].x = fmaf(w0, y, v[u].x);
+                v[u].y = fmaf(w1, y, v[u].y);
+                v[u].z = fmaf(w2, y, v[u].z);
+                v[u].w = fmaf(w3, y, v[u].w);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < AH; ++u)
+            if (u0 + u < nt) *reinterpret_cast<float4 *>(p.out + i0 + (u0 + u) * p.D) = v[u];
+    }
+}
+
+// The parameters, packed in pinned host memory, to the device: the CUs read
+// the host memory themselves (a copy this small through a DMA engine costs
+// more in hand-over than in transfer: 6 us for 148 KB, against 8 to 10).
+constexpr size_t kM3UploadMax = size_t(1) << 20;      // floats; larger blocks go by DMA
+__global__ void __launch_bounds__(256) m3_upload(const float *src, float *dst, long n) {
+    const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[i];
 }
 
 static long grid256(long n) { return (n + 255) / 256; }
@@ -416,33 +538,45 @@ int mamba3_launch(M3Args &a, hipStream_t s) {
         set_error("mamba_block_forward: too many projection rows");
         return -1;
     }
-    if (a.D % 4 == 0 && a.D * 16 * kM3TM * 4 < 0x7fffffffL && a.D * 64 * 4 < 0x7fffffffL) {
+    if (a.D % 4 == 0 && a.D * 64 * 4 < 0x7fffffffL) {
         const int tj = static_cast<int>(std::min<long>(4, (a.J + 15) / 16));
-        const dim3 gm(static_cast<unsigned>((a.T + 16 * kM3TM - 1) / (16 * kM3TM)),
-                      static_cast<unsigned>((a.J + 16 * tj - 1) / (16 * tj)));
-        if (gm.y > 65535) {
+        const long gj = (a.J + 16 * tj - 1) / (16 * tj);
+        if (gj > 65535) {
             set_error("mamba_block_forward: too many projection rows");
             return -1;
         }
+        // Tiles of 64 tokens (one workgroup per CU) where they come close to
+        // whole rounds of the 256 CUs, else of 32 (two per CU): T 16384, 35
+        // rows 18.6 against 21.1 us; whole call at T 6000, 134 rows 69.1
+        // against 62.6 us, T 2048, 35 rows 54.4 against 49.7, T 12288, 68
+        // rows (1.5 rounds) 98.9 against 96.1.
+        const long g4 = (a.T + 63) / 64 * gj;
+        const bool t64 = g4 * 100 >= (g4 + 255) / 256 * 256 * 85;
+        const dim3 gm(static_cast<unsigned>(t64 ? (a.T + 63) / 64 : (a.T + 31) / 32), static_cast<unsigned>(gj));
+#define KM_M3P(TJ)                                                                                       \
+        if (t64) hipLaunchKernelGGL((m3_proj_mfma<TJ, 4>), gm, dim3(64 * kM3Split), 0, s, a);            \
+        else     hipLaunchKernelGGL((m3_proj_mfma<TJ, 2>), gm, dim3(64 * kM3Split), 0, s, a)
         switch (tj) {
-        case 1: hipLaunchKernelGGL(m3_proj_mfma<1>, gm, dim3(64 * kM3Split), 0, s, a); break;
-        case 2: hipLaunchKernelGGL(m3_proj_mfma<2>, gm, dim3(64 * kM3Split), 0, s, a); break;
-        case 3: hipLaunchKernelGGL(m3_proj_mfma<3>, gm, dim3(64 * kM3Split), 0, s, a); break;
-        default: hipLaunchKernelGGL(m3_proj_mfma<4>, gm, dim3(64 * kM3Split), 0, s, a); break;
+        case 1: KM_M3P(1); break;
+        case 2: KM_M3P(2); break;
+        case 3: KM_M3P(3); break;
+        default: KM_M3P(4); break;
         }
+#undef KM_M3P
     } else {
         hipLaunchKernelGGL(m3_proj, gp, dim3(256), 0, s, a);
     }
-    hipLaunchKernelGGL(m3_prep, dim3(grid256(a.T * a.N)), dim3(256), 0, s, a);
     const long npairs = (a.N + 1) / 2;
-    const long waves = (a.T / a.L) * npairs;          // workgroups: one per (batch element, pair)
-    hipLaunchKernelGGL(m3_scan, dim3(static_cast<unsigned>(waves)), dim3(64 * kM3ScanW), 0, s, a, npairs);
-    hipLaunchKernelGGL(m3_readout, dim3(grid256(a.T * a.R)), dim3(256), 0, s, a);
+    const dim3 gs(static_cast<unsigned>((a.T / a.L) * npairs));   // workgroups: one per (batch element, pair)
+    if (a.L <= 64L * kM3ScanW * kM3Chunk) hipLaunchKernelGGL(m3_scan<true>, gs, dim3(64 * kM3ScanW), 0, s, a, npairs);
+    else                                 hipLaunchKernelGGL(m3_scan<false>, gs, dim3(64 * kM3ScanW), 0, s, a, npairs);
     const bool al16 = ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
-    if (a.D % 4 == 0 && al16) {
-        const dim3 go(static_cast<unsigned>(grid256(a.D / 4)), static_cast<unsigned>(std::min<long>(a.T, 65535)));
+    const long gt = (a.T + kM3OutT - 1) / kM3OutT;
+    if (a.D % 4 == 0 && al16 && a.R <= kM3OutR && gt <= 65535) {
+        const dim3 go(static_cast<unsigned>(grid256(a.D / 4)), static_cast<unsigned>(gt));
         hipLaunchKernelGGL(m3_out4, go, dim3(256), 0, s, a);
     } else {
+        hipLaunchKernelGGL(m3_readout, dim3(grid256(a.T * a.R)), dim3(256), 0, s, a);
         hipLaunchKernelGGL(m3_out, dim3(grid256(a.T * a.D)), dim3(256), 0, s, a);
     }
     KM_HIP_TRY(hipGetLastError());
@@ -570,13 +704,13 @@ void mamba_block_forward(MambaBlock *b, float *output, const float *input, size_
     const bool has_delta = b->delta_proj.rows > 0 && b->delta_proj.data;
     const bool has_lambda = b->lambda_proj.rows > 0 && b->lambda_proj.data;
     const long J = R + 2 + 2 * NR;
-    const long TS = N / 2 > 0 ? N / 2 : 1;
+    const long TS = N / 2 > 0 ? N / 2 : 1, Tp = (T + 63) / 64 * 64;
     const bool dev_io = km::is_device_ptr(input) && km::is_device_ptr(output);
     km::Staging::lock();
     do {
         const size_t io_bytes = dev_io ? 0 : 2 * km::align_up(sizeof(float) * T * D, 256);
         const size_t bytes = io_bytes + sizeof(float) * (J * D + D * R + N + 2 * NR + TS) + 8 * 256 +
-                             sizeof(float) * (T * J + 3 * T * N + T * R) + 8 * 256;
+                             sizeof(float) * (Tp * J + Tp * N + T * R) + 8 * 256;
         void *base = km::Staging::reserve(bytes);
         if (!base) break;
         km::Carver cv(base);
@@ -606,7 +740,16 @@ void mamba_block_forward(MambaBlock *b, float *output, const float *input, size_
         put(bB, b->b_B, NR);
         put(bC, b->b_C, NR);
         put(th, b->theta, TS);
-        bool ok = hipMemcpyAsync(dpar, hp, sizeof(float) * nP, hipMemcpyHostToDevice, nullptr) == hipSuccess;
+        bool ok;
+        void *hd = nullptr;
+        if (nP <= km::kM3UploadMax && hipHostGetDevicePointer(&hd, hp, 0) == hipSuccess && hd) {
+            hipLaunchKernelGGL(km::m3_upload, dim3(km::grid256(static_cast<long>(nP))), dim3(256), 0, nullptr,
+                               static_cast<const float *>(hd), dpar, static_cast<long>(nP));
+            ok = hipGetLastError() == hipSuccess;
+        } else {
+            (void)hipGetLastError();
+            ok = hipMemcpyAsync(dpar, hp, sizeof(float) * nP, hipMemcpyHostToDevice, nullptr) == hipSuccess;
+        }
         if (!dev_io)
             ok = ok && km::copy_h2d(x, input, sizeof(float) * T * D) == hipSuccess;
         if (!ok) {
@@ -616,10 +759,9 @@ void mamba_block_forward(MambaBlock *b, float *output, const float *input, size_
         km::M3Args a{};
         a.x = x; a.out = o; a.Wcat = Wcat; a.W_out = Wout; a.A = A; a.bB = bB; a.bC = bC;
         a.theta = th;
-        a.P = cv.take<float>(T * J);
-        a.a = cv.take<float>(T * N);
-        a.c = cv.take<float>(T * N);
-        a.H = cv.take<float>(T * N);
+        a.P = cv.take<float>(Tp * J);
+        a.H = cv.take<float>(Tp * N);
+        a.Tp = Tp;
         a.Y = cv.take<float>(T * R);
         a.T = T; a.L = L; a.D = D; a.N = N; a.R = R; a.J = J;
         a.has_delta = has_delta; a.has_lambda = has_lambda;

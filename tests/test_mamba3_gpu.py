@@ -193,3 +193,22 @@ def test_kmamba_checkpoint_roundtrip_forward(tmp_path):
     assert "NULL" in K.km_last_error()
     K.kmamba_free(m)
     K.kmamba_free(m2)
+
+
+# Tokens at the edges of the projection's 32- and 64-token tiles and of the
+# output's 16-token groups, chunks of one, eight and nine steps in the scan
+# (L = 256, 2048, 2049), an odd last state, several ranks, and a width that
+# leaves part of the last output workgroup idle.
+@pytest.mark.parametrize("batch,L,dim,N,R", [(1, 1, 4, 1, 1), (3, 17, 36, 5, 2), (1, 256, 1028, 16, 1),
+                                             (2, 2048, 64, 16, 4), (1, 2049, 32, 7, 1), (9, 64, 20, 16, 3),
+                                             (1, 33, 8, 40, 1)])
+def test_block_tile_edges(batch, L, dim, N, R):
+    p = mamba3_params(dim, N, R)
+    x = rng_for("m3-edges", batch, L, dim, N, R).standard_normal((batch, L, dim)).astype(np.float32)
+    want = O.mamba3_forward(p, x, dt_min=0.01, dt_max=0.5)
+    blk = make_block(dim, N, L, R, p)
+    tx, out = torch.from_numpy(x).cuda(), torch.full((batch, L, dim), float("nan"), device="cuda")
+    K.mamba_block_forward(blk, K.ptr(out), K.ptr(tx), batch)
+    assert K.km_last_error() == ""
+    check(out.cpu().numpy(), want, x)
+    K.mamba_block_free(blk)
