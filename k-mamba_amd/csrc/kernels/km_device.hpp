@@ -114,6 +114,31 @@ __device__ __forceinline__ float row_readout(const float (&yr)[TW]) {
     return cur[0];
 }
 
+// Sum over the M consecutive lanes of a channel (M a power of two <= 64);
+// every lane of the group receives the sum. Within a 16-lane row the steps
+// are DPP VALU ops (no LDS round trip).
+template <int MM>
+__device__ __forceinline__ float sum_m_lanes(float v) {
+    if constexpr (MM == 2) {
+        v += dpp<0xB1>(v);                       // quad_perm [1,0,3,2]
+    } else if constexpr (MM == 4) {
+        v += dpp<0x4E>(v);                       // quad_perm [2,3,0,1]
+        v += dpp<0xB1>(v);
+    } else if constexpr (MM == 8) {
+        v += dpp<0x141>(v);                      // row_half_mirror
+        v += dpp<0x4E>(v);
+        v += dpp<0xB1>(v);
+    } else if constexpr (MM >= 16) {
+        v += dpp<0x128>(v);                      // row_ror:8
+        v += dpp<0x124>(v);                      // row_ror:4
+        v += dpp<0x122>(v);                      // row_ror:2
+        v += dpp<0x121>(v);                      // row_ror:1
+        if constexpr (MM >= 32) v = sum_xor16(v);
+        if constexpr (MM >= 64) v = sum_xor32(v);
+    }
+    return v;
+}
+
 // Workgroup id in an order where consecutive ids share an XCD: the hardware
 // deals workgroups to the 8 XCDs round-robin (XCD x runs ids x, x + 8, ...);
 // this maps XCD x's ids to one contiguous range, so neighbouring tiles (which

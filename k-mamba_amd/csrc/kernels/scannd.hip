@@ -31,6 +31,7 @@
 #include <cstdio>
 
 #include "km_device.hpp"
+#include "scan2d_strips.hpp"
 #include "scannd_flow.hpp"
 #include "../km_runtime.hpp"
 #include "kmamba_km.h"
@@ -65,31 +66,6 @@ struct ScanNDArgs {
 // Tile band b, ordinal o of the grid's tiles (band_tile_n).
 __device__ inline bool band_tile(const ScanNDArgs &p, int band, int ordinal, int *ti) {
     return band_tile_n(p.nd, p.ntile, band, ordinal, ti);
-}
-
-// Sum over the M consecutive lanes of a channel (M a power of two <= 64);
-// every lane of the group receives the sum. Within a 16-lane row the steps
-// are DPP VALU ops (no LDS round trip).
-template <int MM>
-__device__ __forceinline__ float sum_m_lanes(float v) {
-    if constexpr (MM == 2) {
-        v += dpp<0xB1>(v);                       // quad_perm [1,0,3,2]
-    } else if constexpr (MM == 4) {
-        v += dpp<0x4E>(v);                       // quad_perm [2,3,0,1]
-        v += dpp<0xB1>(v);
-    } else if constexpr (MM == 8) {
-        v += dpp<0x141>(v);                      // row_half_mirror
-        v += dpp<0x4E>(v);
-        v += dpp<0xB1>(v);
-    } else if constexpr (MM >= 16) {
-        v += dpp<0x128>(v);                      // row_ror:8
-        v += dpp<0x124>(v);                      // row_ror:4
-        v += dpp<0x122>(v);                      // row_ror:2
-        v += dpp<0x121>(v);                      // row_ror:1
-        if constexpr (MM >= 32) v = sum_xor16(v);
-        if constexpr (MM >= 64) v = sum_xor32(v);
-    }
-    return v;
 }
 
 // One wave per (tile, channel group). The wave walks its tile row by row
@@ -1000,6 +976,29 @@ static int scannd_launch(ScanNDArgs &a, long P, hipStream_t s, bool allow_flow,
         Tlead = 8;
     }
     int nbands = 1;
+    // 2D under the dataflow schedule: strips of rows, unless a tile shape is
+    // asked for (KM_SCANND_T2).
+    a.ncg = a.DM / 64;
+    if (fast && flow_pref && a.nd == 2 && !std::getenv("KM_SCANND_T2") &&
+        strip_fits(a.dims[0], a.dims[1], a.D, a.DM)) {
+        const long nfl = strip_flags(a.dims[0], a.dims[1], a.ncg);
+        if (!ext || kFlowHead + static_cast<size_t>(nfl) <= ext->cap) {
+            static thread_local FlowArgs fs;
+            int kind = 0;
+            fs.nbands = 0;
+            for (int x = 0; x <= 8; ++x) fs.cg_lo[x] = static_cast<int>(static_cast<long>(x) * a.ncg / 8);
+            const int bound = flow_bind(s, static_cast<size_t>(nfl), ext, fs, &kind);
+            if (bound < 0) return -1;
+            if (bound > 0) {
+                note_flow(s, kind, kind == 2 ? fs.counter : nullptr);
+                if (status) *status = fs.status;
+                const StripArgs sa{a.x, a.B, a.C, a.dt[0], a.dt[1], a.A[0], a.A[1], a.h, a.y,
+                                   a.dims[0], a.dims[1], a.D, a.DM, a.ncg,
+                                   (a.dims[1] + kStripCols - 1) / kStripCols};
+                return launch_strips<false>(sa, fs, a.M, s);
+            }
+        }
+    }
     if (fast) {
         scannd_tile_shape(a.nd, TWc, Tlead);
         // Rows are prefetched one ahead, so every tile needs at least two
