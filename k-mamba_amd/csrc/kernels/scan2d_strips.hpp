@@ -30,13 +30,16 @@
 //
 // Forward, M = 16 (tiles before -> strips): 64x64 D256 161 -> 95 us, 45x61 D96
 // 125 -> 55, 12x250 D32 262 -> 53, 250x12 D32 156 -> 134 (36 strips in a
-// chain), 17x19 D16 34.5 -> 17.4, 200x190 D48 399 -> 285; 128x128 D1024
-// batches, which fill the chip either way, 949 -> 870 (4.0 TB/s). Blocks in
-// flight on the last two: 3: 300, 965; 4: 285, 870; 5: 287, 866; 6 (spills):
-// 286, 877.
+// chain), 17x19 D16 34.5 -> 17.4, 200x190 D48 399 -> 285; 256x256 D256, which
+// fills the chip either way, 949 -> 870 (4.0 TB/s). Blocks in flight on the
+// last two: 3: 300, 965; 4: 285, 870; 5: 287, 866; 6 (spills): 286, 877.
+// Forward and backward, tiles in both -> strips in both: 45x61 D96 401 -> 144
+// (221 with the forward's alone), 12x250 D48 719 -> 126, 30x24 D32 153 -> 80,
+// 250x12 D48 381 -> 292, one row of 600 802 -> 102, one column of 600 568 -> 97.
 #pragma once
 
 #include <algorithm>
+#include <utility>
 
 #include "km_device.hpp"
 #include "../km_runtime.hpp"
@@ -57,7 +60,7 @@ struct StripArgs {
     const float *A0, *A1;      // [D, M] per axis
     float *s;                  // [P, D, M] the states (adjoint: g)
     float *y;                  // [P, D] (forward)
-    int n0, n1, D, DM, ncg, nblk;
+    int n0, n1, D, DM, ncg, nblk, M;
 };
 
 __device__ __forceinline__ int strip_count(const int *p) {
@@ -82,6 +85,8 @@ __device__ __forceinline__ void strip_wait(const int *p, int v, int &seen) {
 
 // ADJ runs rows and columns backwards: strip 0 holds the last rows, block 0
 // the last columns.
+// MM: the M lanes of a channel (forward; the adjoint sums no lanes and takes
+// any M).
 template <int MM, bool ADJ>
 __global__ void __launch_bounds__(64 * kStripWaves, 2) scan2d_strips(StripArgs p, FlowArgs f) {
     using F = bio<f32_t>;
@@ -114,7 +119,7 @@ __global__ void __launch_bounds__(64 * kStripWaves, 2) scan2d_strips(StripArgs p
         if (item >= nitems) break;
         const int strip = static_cast<int>(item / ncx), cg = cg0 + static_cast<int>(item % ncx);
         const int fl = cg * 64 + lane;            // this lane's channel-state
-        const int d = fl / MM;
+        const int d = ADJ ? fl / p.M : fl / MM;
         const int vf = fl * 4, vd = d * 4;
         const int i0 = strip * kStripRows;        // the strip's first row, in walking order
         const int nrow = min(kStripRows, p.n0 - i0);
@@ -346,27 +351,35 @@ __global__ void __launch_bounds__(64 * kStripWaves, 2) scan2d_strips(StripArgs p
 inline long strip_flags(long n0, long n1, long ncg) {
     return ((n0 + kStripRows - 1) / kStripRows) * ((n1 + kStripCols - 1) / kStripCols) * ncg;
 }
-inline bool strip_fits(long n0, long n1, long D, long DM) {
-    return DM % 64 == 0 && (n1 + kStripCols) * DM * 4 < 0x7fffffffL && n0 > 1 && n1 > 1 &&
-           strip_flags(n0, n1, DM / 64) < 0x7fffffffL && D > 0;
+inline bool strip_fits(long n0, long n1, long DM) {
+    return DM % 64 == 0 && ((n1 == 1 ? n0 : n1) + kStripCols) * DM * 4 < 0x7fffffffL &&
+           strip_flags(n0, n1, DM / 64) < 0x7fffffffL;
 }
 
-// The launch: up to one workgroup per CU of an XCD (their registers allow no more).
+// The launch: up to one workgroup per CU of an XCD (their registers allow no
+// more). A grid of one column is one row with the axes exchanged: a single
+// strip (which uses no flag) instead of a chain of them.
 template <bool ADJ>
-static int launch_strips(const StripArgs &a, const FlowArgs &fa, long M, hipStream_t s) {
+static int launch_strips(StripArgs a, const FlowArgs &fa, hipStream_t s) {
+    if (a.n1 == 1) {
+        std::swap(a.n0, a.n1);
+        std::swap(a.dt0, a.dt1);
+        std::swap(a.A0, a.A1);
+        a.nblk = (a.n1 + kStripCols - 1) / kStripCols;
+    }
     const long nstrip = (a.n0 + kStripRows - 1) / kStripRows;
     long per_xcd = 0;
     for (int x = 0; x < 8; ++x) per_xcd = std::max<long>(per_xcd, nstrip * (fa.cg_lo[x + 1] - fa.cg_lo[x]));
     const dim3 grid(static_cast<unsigned>(8 * std::min<long>(per_xcd, 32))), blk(64 * kStripWaves);
 #define KM_STRIP(MMv) hipLaunchKernelGGL((scan2d_strips<MMv, ADJ>), grid, blk, 0, s, a, fa)
-    switch (M) {
+    switch (ADJ ? 1 : a.M) {
     case 1: KM_STRIP(1); break;
-    case 2: KM_STRIP(2); break;
-    case 4: KM_STRIP(4); break;
-    case 8: KM_STRIP(8); break;
-    case 16: KM_STRIP(16); break;
-    case 32: KM_STRIP(32); break;
-    default: KM_STRIP(64); break;
+    case 2: KM_STRIP(ADJ ? 1 : 2); break;
+    case 4: KM_STRIP(ADJ ? 1 : 4); break;
+    case 8: KM_STRIP(ADJ ? 1 : 8); break;
+    case 16: KM_STRIP(ADJ ? 1 : 16); break;
+    case 32: KM_STRIP(ADJ ? 1 : 32); break;
+    default: KM_STRIP(ADJ ? 1 : 64); break;
     }
 #undef KM_STRIP
     KM_HIP_TRY(hipGetLastError());

@@ -980,7 +980,7 @@ static int scannd_launch(ScanNDArgs &a, long P, hipStream_t s, bool allow_flow,
     // asked for (KM_SCANND_T2).
     a.ncg = a.DM / 64;
     if (fast && flow_pref && a.nd == 2 && !std::getenv("KM_SCANND_T2") &&
-        strip_fits(a.dims[0], a.dims[1], a.D, a.DM)) {
+        strip_fits(a.dims[0], a.dims[1], a.DM)) {
         const long nfl = strip_flags(a.dims[0], a.dims[1], a.ncg);
         if (!ext || kFlowHead + static_cast<size_t>(nfl) <= ext->cap) {
             static thread_local FlowArgs fs;
@@ -994,8 +994,8 @@ static int scannd_launch(ScanNDArgs &a, long P, hipStream_t s, bool allow_flow,
                 if (status) *status = fs.status;
                 const StripArgs sa{a.x, a.B, a.C, a.dt[0], a.dt[1], a.A[0], a.A[1], a.h, a.y,
                                    a.dims[0], a.dims[1], a.D, a.DM, a.ncg,
-                                   (a.dims[1] + kStripCols - 1) / kStripCols};
-                return launch_strips<false>(sa, fs, a.M, s);
+                                   (a.dims[1] + kStripCols - 1) / kStripCols, a.M};
+                return launch_strips<false>(sa, fs, s);
             }
         }
     }

@@ -26,6 +26,7 @@
 #include <cstring>
 
 #include "km_device.hpp"
+#include "scan2d_strips.hpp"
 #include "scannd_flow.hpp"
 #include "../km_runtime.hpp"
 #include "kmamba_km.h"
@@ -141,11 +142,11 @@ __device__ __forceinline__ void adj_store(const AdjWin &w, long r, float g) {
 // launch (the next band). Workgroups are numbered XCD-major (xcd_remap):
 // the channel groups of a tile, which share the dy / delta row lines (four
 // channels, 16 bytes, each), run on one XCD's L2.
-//
-// adj_tile2d runs one (tile (ti0, ti1), channel group cg); wait() runs before
-// any state written by another tile is read (false: nothing is computed).
-template <int TR, int TW, int RB, bool COH, typename Wait>
-__device__ __forceinline__ bool adj_tile2d(const NdBwdArgs &a, int ti0, int ti1, int cg, Wait &&wait) {
+template <int TR, int TW, int RB>
+__global__ void __launch_bounds__(64) nd_adjoint_tile2d(NdBwdArgs a, int band, int nt1, int ncg) {
+    const int lb = static_cast<int>(xcd_remap(blockIdx.x, gridDim.x));
+    const int o = lb / ncg, cg = lb - o * ncg;
+    const int ti0 = (band > nt1 - 1 ? band - (nt1 - 1) : 0) + o, ti1 = band - ti0;
     const int lane = threadIdx.x & 63;
     const long n0 = a.dims[0], n1 = a.dims[1];
     const long r0 = static_cast<long>(ti0) * TR, r1 = std::min<long>(n0, r0 + TR);
@@ -164,9 +165,7 @@ __device__ __forceinline__ bool adj_tile2d(const NdBwdArgs &a, int ti0, int ti1,
         float dyc[TW], d0[TW], d1[TW];
         float gr, dr1;
     };
-    // The operands no other tile writes (ops) and the right successor's
-    // state (succ).
-    auto load_ops = [&](long r, Row &rw) __attribute__((always_inline)) {
+    auto load_row = [&](long r, Row &rw) __attribute__((always_inline)) {
         const long rq = r * n1 - qb;
 #pragma unroll
         for (int jj = 0; jj < TW; ++jj) {
@@ -176,26 +175,16 @@ __device__ __forceinline__ bool adj_tile2d(const NdBwdArgs &a, int ti0, int ti1,
             rw.d1[jj] = adj_dl(w, 1, q);
         }
         rw.dr1 = adj_dl(w, 1, rq + std::min<long>(j1, n1 - 1));
+        rw.gr = adj_g(w, rq + std::min<long>(j1, n1 - 1));
     };
-    auto load_succ = [&](long r, Row &rw) __attribute__((always_inline)) {
-        rw.gr = adj_g<COH>(w, r * n1 - qb + std::min<long>(j1, n1 - 1));
-    };
-    auto load_row = [&](long r, Row &rw) __attribute__((always_inline)) {
-        load_ops(r, rw);
-        load_succ(r, rw);
-    };
-    // The first batch's operands go out before the wait on the successors.
     Row ba[RB], bb[RB];
 #pragma unroll
-    for (int i = 0; i < RB; ++i) load_ops(std::max<long>(r1 - 1 - i, r0), ba[i]);
-    if (!wait()) return false;
-#pragma unroll
-    for (int i = 0; i < RB; ++i) load_succ(std::max<long>(r1 - 1 - i, r0), ba[i]);
+    for (int i = 0; i < RB; ++i) load_row(std::max<long>(r1 - 1 - i, r0), ba[i]);
     float gb[TW], db0[TW];
 #pragma unroll
     for (int jj = 0; jj < TW; ++jj) {
         const long q = std::min<long>(r1, n0 - 1) * n1 + std::min<long>(j0 + jj, j1 - 1) - qb;
-        gb[jj] = adj_g<COH>(w, q);
+        gb[jj] = adj_g(w, q);
         db0[jj] = adj_dl(w, 0, q);
     }
     // Rows go in batches of RB, the next batch's loads issued before the
@@ -238,15 +227,6 @@ __device__ __forceinline__ bool adj_tile2d(const NdBwdArgs &a, int ti0, int ti1,
             compute_batch(rt - RB, bb);
         }
     }
-    return true;
-}
-
-template <int TR, int TW, int RB>
-__global__ void __launch_bounds__(64) nd_adjoint_tile2d(NdBwdArgs a, int band, int nt1, int ncg) {
-    const int lb = static_cast<int>(xcd_remap(blockIdx.x, gridDim.x));
-    const int o = lb / ncg, cg = lb - o * ncg;
-    const int ti0 = (band > nt1 - 1 ? band - (nt1 - 1) : 0) + o;
-    adj_tile2d<TR, TW, RB, false>(a, ti0, band - ti0, cg, [] { return true; });
 }
 
 // 3D grids with D*M a multiple of 64: the same by TP x TR x TW tiles (axis
@@ -391,16 +371,15 @@ __global__ void __launch_bounds__(64) nd_adjoint_tile3d(NdBwdArgs a, const int *
 // The adjoint sweep on the dataflow schedule (scannd_flow.hpp), one launch:
 // items in reverse band order (a tile's successors come first), a tile
 // waiting on its successor along each axis; channel groups pinned to XCDs,
-// workgroups of flow_q waves, one group per wave. 2D tiles are 8 rows x 4
-// points (the critical path runs through nt0 + nt1 - 1 of them), 3D tiles
-// those of the band schedule.
-constexpr int kAdjFTR = 8, kAdjFTW = 4;   // 2D dataflow tiles (rows, points)
+// workgroups of flow_q waves, one group per wave. 3D tiles are those of the
+// band schedule; 2D grids run on strips of rows instead (scan2d_strips.hpp).
+constexpr int kAdjFTR = 8, kAdjFTW = 4;   // fused 2D pencils: rows per sub-tile, columns
 constexpr int kF3S = 2, kF3R = 4, kF3W = 4;   // fused 3D pencils: planes per sub-tile, rows, points
 
 // NaN into the states of one (tile, channel group) whose wait gave up, so
 // every tile that depends on it, and every gradient, turns NaN too.
-template <int ND>
 __device__ void adj_tile_poison(const NdBwdArgs &a, const int *ti, const int *text, int cg) {
+    constexpr int ND = 3;
     const long DM = a.D * a.M;
     const long c = static_cast<long>(cg) * 64 + (threadIdx.x & 63);
     long lo[ND], ext[ND], npts = 1;
@@ -422,9 +401,9 @@ __device__ void adj_tile_poison(const NdBwdArgs &a, const int *ti, const int *te
     }
 }
 
-template <int ND>
 __global__ void __launch_bounds__(64 * kFlowQ, 2) nd_adjoint_flow(NdBwdArgs a, FlowArgs f, int nt0, int nt1,
                                                                   int nt2, int ncg) {
+    constexpr int ND = 3;
     const int xcd = flow_xcd();
     const int cg0 = f.cg_lo[xcd], ncx = f.cg_lo[xcd + 1] - cg0;
     if (ncx <= 0) return;
@@ -436,7 +415,7 @@ __global__ void __launch_bounds__(64 * kFlowQ, 2) nd_adjoint_flow(NdBwdArgs a, F
     const unsigned epoch = __builtin_amdgcn_readfirstlane(
         __hip_atomic_load(f.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     const int ntile[3] = {nt0, nt1, nt2};
-    const int text[3] = {ND == 2 ? kAdjFTR : kAdj3P, ND == 2 ? kAdjFTW : kAdj3R, kAdj3W};
+    const int text[3] = {kAdj3P, kAdj3R, kAdj3W};
     int tstride[3];
     tstride[ND - 1] = 1;
 #pragma unroll
@@ -466,13 +445,9 @@ __global__ void __launch_bounds__(64 * kFlowQ, 2) nd_adjoint_flow(NdBwdArgs a, F
                                       f.spin) && ready;
             return ready;
         };
-        bool ok;
-        if constexpr (ND == 2)
-            ok = adj_tile2d<kAdjFTR, kAdjFTW, 4, true>(a, ti[0], ti[1], cg, successors_done);
-        else
-            ok = adj_tile3d<kAdj3P, kAdj3R, kAdj3W, true>(a, ti[0], ti[1], ti[2], cg, successors_done);
+        const bool ok = adj_tile3d<kAdj3P, kAdj3R, kAdj3W, true>(a, ti[0], ti[1], ti[2], cg, successors_done);
         if (!ok) {
-            adj_tile_poison<ND>(a, ti, text, cg);
+            adj_tile_poison(a, ti, text, cg);
             if ((threadIdx.x & 63) == 0)
                 __hip_atomic_store(f.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
@@ -997,7 +972,7 @@ __global__ void __launch_bounds__(256) nd_adjoint_grads_tile3d(NdBwdArgs a) {
 // column strip of TW points through every row, run of kFlowQ channel
 // groups), taken right to left. Each wave walks its group's pencil
 // bottom-up in sub-tiles of TR rows (a completion flag after each), each
-// row right to left as adj_tile2d does, and at each point forms every
+// row right to left as nd_adjoint_tile2d does, and at each point forms every
 // gradient from the adjoint state it just computed, in grad_finish's
 // arithmetic. The adjoint state is never stored whole: the row below stays
 // in registers across sub-tiles and only the pencil's first column goes to
@@ -1569,17 +1544,11 @@ constexpr long kGradGroups = 1024;
 constexpr int kGradMin2 = 8, kGradMin3 = 2;
 constexpr int kGradTPW3 = 1;                                 // 3D tiles per workgroup (2 and 4 measured slower)
 
-// The adjoint sweep's dataflow tiles per axis (0 past nd).
-static void adj_flow_tiles(const KMScanNDBwd *a, int nd, int nt[3]) {
-    nt[0] = nt[1] = nt[2] = 0;
-    if (nd == 2) {
-        nt[0] = static_cast<int>((a->dims[0] + kAdjFTR - 1) / kAdjFTR);
-        nt[1] = static_cast<int>((a->dims[1] + kAdjFTW - 1) / kAdjFTW);
-    } else if (nd == 3) {
-        nt[0] = static_cast<int>((a->dims[0] + kAdj3P - 1) / kAdj3P);
-        nt[1] = static_cast<int>((a->dims[1] + kAdj3R - 1) / kAdj3R);
-        nt[2] = static_cast<int>((a->dims[2] + kAdj3W - 1) / kAdj3W);
-    }
+// The 3D adjoint sweep's dataflow tiles per axis.
+static void adj_flow_tiles(const KMScanNDBwd *a, int nt[3]) {
+    nt[0] = static_cast<int>((a->dims[0] + kAdj3P - 1) / kAdj3P);
+    nt[1] = static_cast<int>((a->dims[1] + kAdj3R - 1) / kAdj3R);
+    nt[2] = static_cast<int>((a->dims[2] + kAdj3W - 1) / kAdj3W);
 }
 
 struct NdBwdShape {
@@ -1588,6 +1557,7 @@ struct NdBwdShape {
     bool gtiles;         // ... and 2D or 3D: the tile walks
     int gext;            // their extent along the walk (NdBwdArgs::gext)
     bool atile2;         // 2D adjoint state by tile bands
+    bool strips;         // ... or on strips of rows (the dataflow schedule)
     int db;
     long qc, nbx, nby;
     size_t offs_bytes, nbr_bytes, part_bytes, tile_bytes;
@@ -1680,6 +1650,7 @@ static bool nd_bwd_shape(const KMScanNDBwd *a, NdBwdShape &s) {
         return std::max(n * s.D * s.M * 4, (static_cast<double>(s.nd - 1) * s.P + n) * s.D * 4) < 2147483000.0;
     };
     s.atile2 = s.nd == 2 && (s.D * s.M) % 64 == 0 && adj_win_ok((kAdjTR + 1) * a->dims[1]);
+    s.strips = s.atile2 && strip_fits(a->dims[0], a->dims[1], s.D * s.M);
     if (s.nd == 3 && (s.D * s.M) % 64 == 0 && adj_win_ok((kAdj3P + 1) * a->dims[1] * a->dims[2])) {
         long nt = 1;
         const long tdim[3] = {kAdj3P, kAdj3R, kAdj3W};
@@ -1731,11 +1702,15 @@ static bool nd_bwd_shape(const KMScanNDBwd *a, NdBwdShape &s) {
         }
     }
     s.flow_bytes = 0;
-    if (s.atile2 || s.tile_bytes) {
+    if (s.tile_bytes) {
         int nt[3];
-        adj_flow_tiles(a, static_cast<int>(s.nd), nt);
-        const long ntiles = static_cast<long>(nt[0]) * nt[1] * (s.nd == 3 ? nt[2] : 1);
+        adj_flow_tiles(a, nt);
+        const long ntiles = static_cast<long>(nt[0]) * nt[1] * nt[2];
         s.flow_bytes = align_up(4 * (kFlowHead + static_cast<size_t>(ntiles) * (s.D * s.M / 64)), 256);
+    }
+    if (s.strips) {
+        const size_t nfl = static_cast<size_t>(strip_flags(a->dims[0], a->dims[1], s.D * s.M / 64));
+        s.flow_bytes = align_up(4 * (kFlowHead + nfl), 256);
     }
     if (s.fused3) {
         const size_t nfl = static_cast<size_t>(s.f3nsub * s.f3nt1 * s.f3nt2) * (s.D * s.M / 64);
@@ -1778,40 +1753,40 @@ static void grads_tile_launch(const NdBwdArgs &args, const NdBwdShape &s, hipStr
     }
 }
 
-// Binds the adjoint sweep's dataflow state (band table, channel groups per
-// XCD) when the tiled sweep applies, the device has 8 XCDs and the bands fit
-// the kernel arguments: in the caller's workspace (ext, cleared here, so
+// Binds the adjoint sweep's dataflow state (channel groups per XCD; 3D: the
+// band table) when a tiled sweep applies, the device has 8 XCDs and the bands
+// fit the kernel arguments: in the caller's workspace (ext, cleared here, so
 // nothing is allocated) or in the stream's dataflow block. Returns 1 when
 // bound, 0 for the band schedule, -1 on an error.
 static int adj_flow_setup(const KMScanNDBwd *a, const NdBwdShape &s, hipStream_t st, FlowArgs &fa,
                           int nt[3], FlowBuf *ext) {
-    const bool tiled = (s.nd == 2 && s.atile2) || (s.nd == 3 && s.tile_bytes);
-    if (!tiled || !flow_wanted(s.nd)) return 0;
-    adj_flow_tiles(a, static_cast<int>(s.nd), nt);
-    const int nb = nt[0] + nt[1] + (s.nd == 3 ? nt[2] : 1) - (s.nd == 3 ? 2 : 1);
+    if (!(s.strips || s.tile_bytes) || !flow_wanted(s.nd)) return 0;
     const long ncg = s.D * s.M / 64;
-    if (nb > kMaxFlowBands || nb <= 0) return 0;
-    fa.nbands = nb;
     for (int x = 0; x <= 8; ++x) fa.cg_lo[x] = static_cast<int>(static_cast<long>(x) * ncg / 8);
-    fa.band_start[0] = 0;
-    for (int b = 0; b < nb; ++b) {
-        long c = 0;
-        if (s.nd == 2) {
-            const int lo = std::max(0, b - (nt[1] - 1)), hi = std::min(b, nt[0] - 1);
-            c = hi >= lo ? hi - lo + 1 : 0;
-        } else {
+    fa.nbands = 0;
+    long nfl = 0;
+    if (s.strips) {
+        nfl = strip_flags(a->dims[0], a->dims[1], ncg);
+    } else {
+        adj_flow_tiles(a, nt);
+        const int nb = nt[0] + nt[1] + nt[2] - 2;
+        if (nb > kMaxFlowBands || nb <= 0) return 0;
+        fa.nbands = nb;
+        fa.band_start[0] = 0;
+        for (int b = 0; b < nb; ++b) {
+            long c = 0;
             for (int t0 = 0; t0 < nt[0] && t0 <= b; ++t0) {
                 const int r = b - t0, lo = std::max(0, r - (nt[2] - 1)), hi = std::min(r, nt[1] - 1);
                 c += hi >= lo ? hi - lo + 1 : 0;
             }
+            fa.band_start[b + 1] = fa.band_start[b] + static_cast<int>(c);
         }
-        fa.band_start[b + 1] = fa.band_start[b] + static_cast<int>(c);
+        nfl = fa.band_start[nb] * ncg;
     }
-    const long ntiles = fa.band_start[nb];
-    if (ntiles * ncg >= 0x7fffffffL) return 0;
+    if (nfl >= 0x7fffffffL) return 0;
     if (ext) flow_zero(ext->buf, ext->cap, st);
     int kind = 0;
-    const int bound = flow_bind(st, static_cast<size_t>(ntiles * ncg), ext, fa, &kind);
+    const int bound = flow_bind(st, static_cast<size_t>(nfl), ext, fa, &kind);
     note_flow(st, kind, kind == 2 ? fa.counter : nullptr);
     return bound;
 }
@@ -1860,12 +1835,18 @@ static int fused2p_flow_setup(const NdBwdShape &s, hipStream_t st, FlowArgs &fa,
 }
 
 template <int ND>
-static void nd_bwd_launch(const NdBwdArgs &args, const NdBwdShape &s, const KMWavefrontPlan *plan,
+static int nd_bwd_launch(const NdBwdArgs &args, const NdBwdShape &s, const KMWavefrontPlan *plan,
                           float *dA, const int *dtiles, const std::vector<long> &bstart, hipStream_t st,
                           const FlowArgs *flow, const int *nt) {
     const long DM = s.D * s.M;
     const unsigned bx = static_cast<unsigned>((DM + 255) / 256);
-    if ((ND == 2 || ND == 3) && flow) {
+    if (ND == 2 && flow) {
+        const StripArgs sa{args.dy, nullptr, args.C, args.delta, args.delta + s.P * s.D, args.A, args.A + DM,
+                           args.dB, nullptr, static_cast<int>(args.dims[0]), static_cast<int>(args.dims[1]),
+                           static_cast<int>(s.D), static_cast<int>(DM), static_cast<int>(DM / 64),
+                           static_cast<int>((args.dims[1] + kStripCols - 1) / kStripCols), static_cast<int>(s.M)};
+        if (launch_strips<true>(sa, *flow, st)) return -1;
+    } else if (ND == 3 && flow) {
         // One dataflow launch: 8k workgroups of Q waves (k <= 256 / Q, two
         // waves per SIMD), k = the largest per-XCD item count.
         const int q = flow_q(*flow);
@@ -1875,7 +1856,7 @@ static void nd_bwd_launch(const NdBwdArgs &args, const NdBwdShape &s, const KMWa
             per_xcd = std::max<long>(per_xcd, ntiles * ((flow->cg_lo[x + 1] - flow->cg_lo[x]) / q));
         const long grid = 8 * std::min<long>(per_xcd, 256 / q);
         if (grid > 0)
-            hipLaunchKernelGGL((nd_adjoint_flow<ND == 2 ? 2 : 3>), dim3(static_cast<unsigned>(grid)),
+            hipLaunchKernelGGL(nd_adjoint_flow, dim3(static_cast<unsigned>(grid)),
                                dim3(64 * q), 0, st, args, *flow, nt[0], nt[1], nt[2],
                                static_cast<int>(DM / 64));
     } else if (ND == 3 && s.tile_bytes) {
@@ -1921,6 +1902,7 @@ static void nd_bwd_launch(const NdBwdArgs &args, const NdBwdShape &s, const KMWa
                            args, s.qc, s.db);
     }
     sum_dA(args.part, dA, s.nbx, s.nd * DM, st);
+    return 0;
 }
 
 }  // namespace km
@@ -2109,17 +2091,17 @@ int km_scannd_bwd(const KMScanNDBwd *a, void *stream) {
     } else {
         const int *dtiles = reinterpret_cast<const int *>(tile_ws);
         switch (s.nd) {
-        case 1: km::nd_bwd_launch<1>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
-        case 2: km::nd_bwd_launch<2>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
-        case 3: km::nd_bwd_launch<3>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
-        case 4: km::nd_bwd_launch<4>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
-        case 5: km::nd_bwd_launch<5>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
-        case 6: km::nd_bwd_launch<6>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
-        case 7: km::nd_bwd_launch<7>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
-        default: km::nd_bwd_launch<8>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
+        case 1: rc = km::nd_bwd_launch<1>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
+        case 2: rc = km::nd_bwd_launch<2>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
+        case 3: rc = km::nd_bwd_launch<3>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
+        case 4: rc = km::nd_bwd_launch<4>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
+        case 5: rc = km::nd_bwd_launch<5>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
+        case 6: rc = km::nd_bwd_launch<6>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
+        case 7: rc = km::nd_bwd_launch<7>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
+        default: rc = km::nd_bwd_launch<8>(args, s, plan, a->dA, dtiles, bstart, st, flow, nt); break;
         }
         const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) {
+        if (rc == 0 && e != hipSuccess) {
             km::set_error("km_scannd_bwd: launch failed: %s", hipGetErrorString(e));
             rc = -1;
         }

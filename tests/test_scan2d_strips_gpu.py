@@ -12,7 +12,7 @@ import pytest
 
 import oracle as O
 from kmtest import TOL_F32, assert_close
-from test_scannd_gpu import _BUDGET0, _stable_nd_inputs, kappa, run_device
+from test_scannd_gpu import _BUDGET0, _stable_nd_inputs, bwd_inputs, kappa, run_bwd, run_device
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -22,7 +22,8 @@ pytestmark = pytest.mark.gpu
 # than a ring holds. M covers every lane sum; one channel group leaves seven
 # XCDs without work.
 STRIPS = [((2, 2), 4, 16), ((7, 3), 64, 1), ((8, 4), 96, 2), ((14, 5), 48, 4), ((15, 16), 8, 8),
-          ((22, 33), 20, 16), ((3, 37), 10, 32), ((40, 2), 3, 64), ((29, 70), 36, 16)]
+          ((22, 33), 20, 16), ((3, 37), 10, 32), ((40, 2), 3, 64), ((29, 70), 36, 16), ((1, 41), 8, 8),
+          ((30, 1), 8, 8)]
 
 
 @pytest.mark.parametrize("dims,D,M", STRIPS)
@@ -36,6 +37,22 @@ def test_strip_edges(dims, D, M, monkeypatch):
     monkeypatch.setenv("KM_SCANND_SCHED", "band")
     _, hb = run_device(dims, x, A, B, Cm, dt)
     assert np.array_equal(h.view(np.uint32), hb.view(np.uint32))
+
+
+# (24 states: the adjoint sums no lanes and takes any M.)
+@pytest.mark.parametrize("dims,D,M", STRIPS + [((16, 19), 8, 24)])
+def test_strip_edges_backward(dims, D, M, monkeypatch):
+    ins = bwd_inputs(dims, D, M, 8)
+    a = run_bwd(dims, *ins)
+    want = O.scannd_backward(dims, *ins, fast=True)
+    for k in want:
+        assert np.isfinite(a[k]).all(), k
+        err = np.abs(a[k] - want[k]).max() / max(np.abs(want[k]).max(), 1e-30)
+        assert err <= 1e-4, f"{k}: normwise error {err:.2e}"
+    monkeypatch.setenv("KM_SCANND_SCHED", "band")
+    b = run_bwd(dims, *ins)
+    for k in a:
+        assert np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)), k
 
 
 def test_wait_budget_exhausted_fails_loudly_and_sync_api_recovers(tmp_path):
