@@ -1815,6 +1815,19 @@ static int fused3_flow_setup(const NdBwdShape &s, hipStream_t st, FlowArgs &fa, 
     return bound;
 }
 
+// The fused 2D backward saves writing and reading the adjoint state, but its
+// pencils hand over through the L2, so it wins only where enough of them run at
+// once: nt0 x nt1 sub-tiles in nt0 + nt1 - 1 fronts, a wave each, against a
+// wave for each of the 1024 SIMDs. Forward + backward, M = 16, fused / two
+// passes (us), by the average front: 349 waves (128x128 D128) 736 / 555, 356
+// (64x64 D256) 363 / 274, 632 (256x200 D128) 1528 / 1372, 690 (256x256 D128)
+// 1751 / 1595, 745 (32x32 D1024) 228 / 220, 868 (160x160 D256) 1214 / 1194,
+// 1046 (128x128 D384) 1074 / 1121, 1053 (96x96 D512) 790 / 840, 1081 (200x200
+// D256) 1675 / 1891, 1394 (128x128 D512) 1293 / 1503.
+static bool fused2_fills(const NdBwdShape &s) {
+    return s.fnt0 * s.fnt1 * (s.D * s.M / 64) >= 1024 * (s.fnt0 + s.fnt1 - 1);
+}
+
 // The fused 2D pencils' dataflow state: pencils are taken right to left
 // (the kernel derives a pencil from its item), a flag per (sub-tile, pencil,
 // channel group).
@@ -1970,11 +1983,13 @@ int km_scannd_bwd(const KMScanNDBwd *a, void *stream) {
     // list to upload), else by tile bands.
     static thread_local km::FlowArgs fa;
     int nt[3] = {0, 0, 0};
-    // 2D on the dataflow schedule: the fused backward on pencils
-    // (KM_SCANND_BWD_FUSED=0: the adjoint sweep, then the gradient pass).
+    // 2D on the dataflow schedule: the fused backward on pencils where its
+    // fronts fill the chip, else the adjoint sweep on strips, then the gradient
+    // pass (KM_SCANND_BWD_FUSED=0: always; any other value: never).
     {
         const char *fe = std::getenv("KM_SCANND_BWD_FUSED");
-        if (s.fused2 && km::flow_wanted(2) && !(fe && std::strcmp(fe, "0") == 0)) {
+        const bool want = fe ? std::strcmp(fe, "0") != 0 : km::fused2_fills(s);
+        if (s.fused2 && km::flow_wanted(2) && want) {
             km::FlowBuf wf{reinterpret_cast<unsigned *>(ws + s.offs_bytes + s.nbr_bytes + s.part_bytes + s.tile_bytes),
                            s.flow_bytes / 4, 8};
             const int fbp = km::fused2p_flow_setup(s, st, fa, (a->workspace && s.flow_bytes) ? &wf : nullptr);

@@ -12,7 +12,7 @@ import pytest
 
 import oracle as O
 from kmtest import TOL_F32, assert_close
-from test_scannd_gpu import _BUDGET0, _stable_nd_inputs, bwd_inputs, kappa, run_bwd, run_device
+from test_scannd_gpu import FUSED_CASES, _BUDGET0, _stable_nd_inputs, bwd_inputs, kappa, run_bwd, run_device
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -53,6 +53,21 @@ def test_strip_edges_backward(dims, D, M, monkeypatch):
     b = run_bwd(dims, *ins)
     for k in a:
         assert np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)), k
+
+
+# Small 2D grids run the two passes by default; forced, the fused backward
+# gives the same values (dA sums its terms in another order). The last grid
+# is over the line, so its default is the fused one.
+@pytest.mark.parametrize("dims,D,M", [c for c in FUSED_CASES if len(c[0]) == 2] + [((9, 10), 4096, 16)])
+def test_fused_forced_matches_default(dims, D, M, monkeypatch):
+    ins = bwd_inputs(dims, D, M, 9)
+    a = run_bwd(dims, *ins)
+    for forced in ("1", "0"):
+        monkeypatch.setenv("KM_SCANND_BWD_FUSED", forced)
+        b = run_bwd(dims, *ins)
+        for k in ("dx", "ddelta", "dB", "dC"):
+            assert np.isfinite(a[k]).all() and np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)), k
+        np.testing.assert_allclose(a["dA"], b["dA"], rtol=1e-5, atol=1e-6 * float(np.abs(b["dA"]).max()))
 
 
 def test_wait_budget_exhausted_fails_loudly_and_sync_api_recovers(tmp_path):
