@@ -274,12 +274,14 @@ int km_scannd_fwd_noalloc(const ScanNDParams *p, void *stream);
  * bytes of device memory, or NULL for the library's scratch of this
  * (device, stream). The adjoint state runs against the forward's wavefront:
  * on 2D and 3D grids with D*M a multiple of 64 as one dataflow launch over
- * tiles on a device with 8 XCDs (KM_SCANND_SCHED=band: one launch per tile
- * band), otherwise one launch per anti-diagonal level, last to first. With
- * D*M a multiple of 2048 and 4 <= M <= 32 (3D: 8 <= M <= 32) that launch
- * runs on pencils and also forms every gradient (the workspace then holds
- * the pencils' boundary states, 1/4 of a [P, D, M] tensor in 2D, 1/2 in
- * 3D; KM_SCANND_BWD_FUSED=0: the sweep, then a separate gradient pass). */
+ * strips of rows (2D) or tiles (3D) on a device with 8 XCDs
+ * (KM_SCANND_SCHED=band: one launch per tile band), otherwise one launch per
+ * anti-diagonal level, last to first. With D*M a multiple of 2048 and
+ * 4 <= M <= 32 (3D: 8 <= M <= 32) that launch can run on pencils and also form
+ * every gradient (the workspace holds the pencils' boundary states, 1/4 of a
+ * [P, D, M] tensor in 2D, 1/2 in 3D): always in 3D, in 2D where enough pencils
+ * run at once. KM_SCANND_BWD_FUSED=0: always the sweep, then a separate
+ * gradient pass; 1: always pencils. */
 typedef struct {
     const long  *dims;
     long ndims, D, M;

@@ -14,12 +14,14 @@
 //    256-byte coalesced accesses and y is a reduction over the M lanes of a
 //    channel;
 //  * the grid is cut into tiles; tiles with equal tile-index sum (a tile
-//    band) are independent. 2D grids run one launch per tile band (47 for a
-//    256x256 grid with 16x8 tiles instead of 511 per-level launches); the
-//    kernel boundary publishes every tile's h to the next band. Grids of 3
-//    or more dims run one dataflow launch per step, in which a tile waits
-//    only for its own axis predecessors (completion flags, each channel
-//    group kept on one XCD so producer and consumer share an L2);
+//    band) are independent. On a device with 8 XCDs a grid of 3 or more
+//    dims runs one dataflow launch, in which a tile waits only for its own
+//    axis predecessors (completion flags, each channel group kept on one XCD
+//    so producer and consumer share an L2), and a 2D grid one launch over
+//    strips of rows (scan2d_strips.hpp). Elsewhere, or when asked to, there
+//    is one launch per tile band (47 for a 256x256 grid with 16x8 tiles
+//    instead of 511 per-level launches), whose boundary publishes every
+//    tile's h to the next band;
 //  * one wave per (tile, channel group) walks its tile row by row (rows
 //    along the last axis), keeping the row above in registers and taking
 //    the left neighbour from the previous column; neighbours across the
@@ -972,9 +974,9 @@ static int scannd_launch(ScanNDArgs &a, long P, hipStream_t s, bool allow_flow,
     int TWc = (a.nd <= 3) ? 8 : 4;
     int Tlead = (a.nd == 2) ? 16 : 4;
     if (a.nd == 2 && flow_pref) {
-        // 2D under the dataflow schedule: the critical path runs through
-        // ntile0 + ntile1 - 1 tiles, so smaller tiles than the band
-        // schedule's (measured fastest: 8 rows of 4 points).
+        // 2D tiles under the dataflow schedule (grids that the strips below
+        // do not take): the critical path runs through ntile0 + ntile1 - 1
+        // tiles, so smaller tiles than the band schedule's.
         TWc = 4;
         Tlead = 8;
     }
