@@ -35,6 +35,7 @@
 #include "km_device.hpp"
 #include "scan2d_strips.hpp"
 #include "scannd_flow.hpp"
+#include "scannd_tiles.hpp"
 #include "../km_runtime.hpp"
 #include "kmamba_km.h"
 #include "scan.h"
@@ -768,9 +769,6 @@ __global__ void __launch_bounds__(256) scannd_m3_level_kernel(ScanM3Args p, cons
 // Tuning knob (read once): KM_SCANND_T2 / KM_SCANND_T3 = "TW,TL" sets the
 // 2D / 3D tile to TW points along the last axis (4, 8 or 16 in 2D; 4 or 8 in
 // 3D) and TL along each leading axis.
-// Waves of an average front up to which 3D dataflow tiles are 2 x 2 x 8 (see
-// scannd_launch).
-constexpr long kSmallFront = 768;
 static void scannd_tile_shape(int nd, int &tw, int &tl) {
     static int t2w = 0, t2l = 0, t3w = 0, t3l = 0;
     static bool once = [] {
@@ -980,7 +978,7 @@ static int scannd_launch(ScanNDArgs &a, long P, hipStream_t s, bool allow_flow,
         TWc = 4;
         Tlead = 8;
     }
-    int nbands = 1;
+    long nbands = 1;
     // 2D under the dataflow schedule: strips of rows, unless a tile shape is
     // asked for (KM_SCANND_T2).
     a.ncg = a.DM / 64;
@@ -1004,26 +1002,9 @@ static int scannd_launch(ScanNDArgs &a, long P, hipStream_t s, bool allow_flow,
             }
         }
     }
-    auto set_tiles = [&](int lead) {
-        // Rows are prefetched one ahead, so every tile needs at least two
-        // rows per plane below an in-tile leading axis: grow the row-axis
-        // tile while its last tile would hold one row, and use tiles of 1
-        // along the leading axes when the row axis has length 1.
-        const int rax = a.nd - 2;
-        int trow = (a.dims[rax] < lead) ? a.dims[rax] : lead;
-        while (trow < a.dims[rax] && a.dims[rax] % trow == 1) ++trow;
-        nbands = 1;
-        for (int ax = 0; ax < a.nd; ++ax) {
-            int t = (ax == a.nd - 1) ? TWc : (ax == rax ? trow : lead);
-            if (ax < rax && a.dims[rax] == 1) t = 1;
-            a.tile[ax] = (a.dims[ax] < t) ? a.dims[ax] : t;
-            a.ntile[ax] = (a.dims[ax] + a.tile[ax] - 1) / a.tile[ax];
-            nbands += a.ntile[ax] - 1;
-        }
-    };
     if (fast) {
         scannd_tile_shape(a.nd, TWc, Tlead);
-        set_tiles(Tlead);
+        nbands = nd_tiles(a.nd, a.dims, TWc, Tlead, a.tile, a.ntile);
         // The tile kernel addresses a tile (and the axis-0 plane before it)
         // with 32-bit byte offsets.
         long span = a.tile[a.nd - 1] + a.pstride[0];
@@ -1031,49 +1012,29 @@ static int scannd_launch(ScanNDArgs &a, long P, hipStream_t s, bool allow_flow,
         if (span * static_cast<long>(a.DM) * 4 >= 0x7fffffffL) fast = false;
     }
     if (fast) {
-        if (nbands > 4096) {
+        if (nbands > kMaxBands) {
             set_error("scannd: too many tile bands");
             return -1;
         }
         // Tiles per band: distribution of tile-index sums.
-        static thread_local long cnt[4096], nxt[4096];
+        static thread_local long cnt[kMaxBands], nxt[kMaxBands];
         auto count_bands = [&]() {
             nbands = 1;
             for (int ax = 0; ax < a.nd; ++ax) nbands += a.ntile[ax] - 1;
-            for (int i = 0; i < nbands; ++i) cnt[i] = 0;
-            cnt[0] = 1;
-            int reach = 0;
-            for (int ax = 0; ax < a.nd; ++ax) {
-                for (int i = 0; i <= reach + a.ntile[ax] - 1; ++i) nxt[i] = 0;
-                for (int sidx = 0; sidx <= reach; ++sidx)
-                    for (int v = 0; v < a.ntile[ax]; ++v) nxt[sidx + v] += cnt[sidx];
-                reach += a.ntile[ax] - 1;
-                for (int sidx = 0; sidx <= reach; ++sidx) cnt[sidx] = nxt[sidx];
-            }
-            long n = 0;
-            for (int b = 0; b < nbands; ++b) n += cnt[b];
-            return n;
+            return nd_band_counts(a.nd, a.ntile, cnt, nxt);
         };
-        // 3D under the dataflow schedule, unless a tile shape is asked for: a
-        // small grid leaves the chip idle while 4 x 4 x 8 sub-tiles hand over
-        // from one to the next, so it takes tiles of 2 x 2 x 8 while their
-        // average front (tiles / bands, a wave per channel group each) is below
-        // three quarters of a wave per SIMD; above, the pencils' ring, which
-        // reads less back, wins. M = 16, pencils / small tiles (us), by that
-        // front: 20x17x23 D64 (216) 218 / 155, 32x32x32 D64 (482) 378 / 293,
-        // 48x20x40 D64 (519) 420 / 318, 6x60x60 D128 (591) 530 / 327, 32x32x32
-        // D96 (723) 405 / 371, 40x40x40 D64 (744) 525 / 476, 40x30x36 D112
-        // (1105) 541 / 614, 50x50x50 D64 (1272) 779 / 932. Both are 8 points
-        // wide, so y's sums keep their order. (Width 4 was faster still, 133 and
-        // 441, 984 on the first, second and last but one, but changes it.)
+        // 3D under the dataflow schedule, unless a tile shape is asked for:
+        // smaller tiles on small grids.
         bool small = false;
         if (flow_pref && a.nd == 3 && !std::getenv("KM_SCANND_T3")) {
-            set_tiles(2);
-            const long n = static_cast<long>(a.ntile[0]) * a.ntile[1] * a.ntile[2] * a.ncg;
-            small = n <= kSmallFront * nbands && (!ext || kFlowHead + static_cast<size_t>(n) <= ext->cap);
-            if (!small) set_tiles(Tlead);
+            small = nd_small_tiles(a.dims, TWc, a.ncg, ext ? ext->cap - kFlowHead : SIZE_MAX, a.tile, a.ntile);
+            if (!small) nd_tiles(a.nd, a.dims, TWc, Tlead, a.tile, a.ntile);
         }
         long ntiles = count_bands();
+        if (ntiles <= 0) {
+            set_error("scannd: too many tile bands");
+            return -1;
+        }
         // 3D tiles of 4 rows along axis 1 keep the previous plane in registers.
         bool ring = a.nd == 3 && a.tile[1] == 4;
         // Under the dataflow schedule 3D ring tiles become pencils along
@@ -1098,7 +1059,7 @@ static int scannd_launch(ScanNDArgs &a, long P, hipStream_t s, bool allow_flow,
         static thread_local FlowArgs fa;
         int kind = 0, bound = 0;
         if (flow_pref && nbands <= kMaxFlowBands && nflags < 0x7fffffffL) {
-            fa.nbands = nbands;
+            fa.nbands = static_cast<int>(nbands);
             for (int x = 0; x <= 8; ++x) fa.cg_lo[x] = static_cast<int>(static_cast<long>(x) * a.ncg / 8);
             fa.band_start[0] = 0;
             for (int b = 0; b < nbands; ++b) fa.band_start[b + 1] = fa.band_start[b] + static_cast<int>(cnt[b]);
@@ -1112,7 +1073,7 @@ static int scannd_launch(ScanNDArgs &a, long P, hipStream_t s, bool allow_flow,
             a.ntile[0] = ntile0;
             ntiles = count_bands();
         } else if (small && bound == 0) {
-            set_tiles(Tlead);
+            nd_tiles(a.nd, a.dims, TWc, Tlead, a.tile, a.ntile);
             ring = a.tile[1] == 4;
             ntiles = count_bands();
         }
@@ -1136,7 +1097,7 @@ static int scannd_launch(ScanNDArgs &a, long P, hipStream_t s, bool allow_flow,
         if (flow)
             for (int x = 0; x < 8; ++x)
                 per_xcd = std::max<long>(per_xcd, ntiles * ((fa.cg_lo[x + 1] - fa.cg_lo[x]) / fq));
-        const int nlaunch = flow ? 1 : nbands;
+        const int nlaunch = flow ? 1 : static_cast<int>(nbands);
         for (int b = 0; b < nlaunch; ++b) {
             a.band = b;
             const long grid = flow ? 8 * std::min<long>(per_xcd, kcap / fq) : cnt[b] * a.ncg;

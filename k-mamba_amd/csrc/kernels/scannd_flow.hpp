@@ -26,6 +26,8 @@
 #include <hip/hip_runtime.h>
 #include <cstddef>
 
+#include "scannd_tiles.hpp"
+
 namespace km {
 
 // Number of pairs (u, v), 0 <= u < n1, 0 <= v < n2, with u + v = s.
@@ -68,7 +70,6 @@ __device__ inline bool band_tile_n(int nd, const int *ntile, int band, int ordin
     return true;
 }
 
-constexpr int kMaxFlowBands = 768;
 constexpr unsigned kFlowSpinDefault = 1u << 20;
 struct FlowArgs {
     unsigned *flags;                     // [ntiles * ncg] epoch of the last finish
