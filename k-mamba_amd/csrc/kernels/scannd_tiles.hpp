@@ -69,11 +69,14 @@ inline long nd_band_counts(int nd, const int *ntile, long *cnt, long *nxt) {
 constexpr long kSmallFront = 768;
 // Sets tile and ntile to the 2 x 2 x `row` tiles and returns true where they
 // are the faster ones for ncg channel groups, their flags fit max_flags and
-// their bands, about twice those of the larger tiles, fit the tables.
+// their bands, about twice those of the larger tiles (whose pencils leave axis 0
+// out), fit the dataflow schedule's table: without it they would run a launch
+// per band (1600x16x16 D128, M = 16: 16940 us, on pencils 9220; 2000x8x8 D64:
+// 23490 and 9210).
 inline bool nd_small_tiles(const int *dims, int row, long ncg, size_t max_flags, int *tile, int *ntile) {
     const long nbands = nd_tiles(3, dims, row, 2, tile, ntile);
     const long n = static_cast<long>(ntile[0]) * ntile[1] * ntile[2] * ncg;
-    return nbands <= kMaxBands && n <= kSmallFront * nbands && static_cast<size_t>(n) <= max_flags;
+    return nbands <= kMaxFlowBands && n <= kSmallFront * nbands && static_cast<size_t>(n) <= max_flags;
 }
 
 }  // namespace km

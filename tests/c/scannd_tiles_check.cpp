@@ -36,6 +36,11 @@ int main() {
                                     n_tiles, sum, want);
                         return 1;
                     }
+                    // Without a band table a launch per band would follow.
+                    if (small && nbands > km::kMaxFlowBands) {
+                        std::printf("%dx%dx%d: small tiles in %ld bands\n", dims[0], dims[1], dims[2], nbands);
+                        return 1;
+                    }
                     ++checked;
                     took_small += small;
                 }
