@@ -67,16 +67,26 @@ inline long nd_band_counts(int nd, const int *ntile, long *cnt, long *nxt) {
 // (Width 4 was faster still, 133 and 441, 984 on the first, second and last but
 // one, but changes it.)
 constexpr long kSmallFront = 768;
-// Sets tile and ntile to the 2 x 2 x `row` tiles and returns true where they
-// are the faster ones for ncg channel groups, their flags fit max_flags and
-// their bands, about twice those of the larger tiles (whose pencils leave axis 0
-// out), fit the dataflow schedule's table: without it they would run a launch
-// per band (1600x16x16 D128, M = 16: 16940 us, on pencils 9220; 2000x8x8 D64:
-// 23490 and 9210).
+// The critical path of a tiling (us): its fronts, each a hand-over and the
+// tile's rows of 8 points one after the other. Smaller tiles shorten it where
+// they split a plane, not where they only split axis 0 (an axis of 3 or 7 rows
+// is one tile, or two of 4, either way). M = 16, D64, pencils / small tiles:
+// 700x8x8 3270 / 2035, 8x8x600 1490 / 520, but 400x7x8 1850 / 2005, 100x3x3 320
+// / 357, 60x7x7 296 / 312.
+inline double nd_path_us(long nbands, const int *tile) { return nbands * (1.6 + 1.05 * tile[0] * tile[1]); }
+// Sets tile and ntile to the 2 x 2 x `row` tiles (axis 1 may have more rows,
+// see nd_tiles) and returns true where they are the faster ones for ncg channel
+// groups, their flags fit max_flags and their bands, about twice those of the
+// larger tiles (whose pencils leave axis 0 out), fit the dataflow schedule's
+// table: without it they would run a launch per band (1600x16x16 D128, M = 16:
+// 16940 us, on pencils 9220; 2000x8x8 D64: 23490 and 9210).
 inline bool nd_small_tiles(const int *dims, int row, long ncg, size_t max_flags, int *tile, int *ntile) {
+    int tile4[3], ntile4[3];
+    const double path4 = nd_path_us(nd_tiles(3, dims, row, 4, tile4, ntile4), tile4);
     const long nbands = nd_tiles(3, dims, row, 2, tile, ntile);
     const long n = static_cast<long>(ntile[0]) * ntile[1] * ntile[2] * ncg;
-    return nbands <= kMaxFlowBands && n <= kSmallFront * nbands && static_cast<size_t>(n) <= max_flags;
+    return nbands <= kMaxFlowBands && n <= kSmallFront * nbands && nd_path_us(nbands, tile) < path4 &&
+           static_cast<size_t>(n) <= max_flags;
 }
 
 }  // namespace km
