@@ -348,6 +348,14 @@ __global__ void __launch_bounds__(HWT == 2 ? 1024 : 512, 4) scan1d_bwd_chunked(S
                     for (int i = 0; i < kFoldRun; ++i)
                         if (m1 - i >= m0) run = fmaf(exp2_fast(dsv[i] * a2), run, gv[i]);
                 }
+                if (fold_overflowed(run)) {
+                    run = 0.f;
+#pragma unroll 1
+                    for (int m1 = p.nmap - 1; m1 >= m0; --m1) {
+                        const long m = (b * p.nmap + m1) * Dm + dc;
+                        run = decay_add(p.seg_dsum[m] * a2, run, p.seg_g[m * N + n0 + w]);
+                    }
+                }
             }
             acar[0][w][lh] = run;
             if (!HIN && dvalid) p.dApart[(static_cast<long>(bs) * Dm + d) * N + n0 + w] = run;

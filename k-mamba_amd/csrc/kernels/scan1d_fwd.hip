@@ -151,8 +151,10 @@ __device__ __forceinline__ void pow_chain_il(float e1, int ns, float (&e)[NPL]) 
 
 // OCC: waves per SIMD the register allocation must allow (2 workgroups of
 // 8 waves per CU need 4).
+// SEG: the workgroup owns a segment of the sequence and starts from the state
+// it folds from the maps before it.
 template <typename T, int NPL, int NS, int W, int TC, bool SHARED, bool HIST, bool STORE_BU, int OCC,
-          bool GATE>
+          bool GATE, bool SEG>
 __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs p) {
     using IO = bio<T>;
     constexpr int DL = 64 / NS;      // channels per wave
@@ -177,14 +179,13 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
     const unsigned wg = static_cast<unsigned>(xcd_remap(blockIdx.x, gridDim.x));
     const unsigned bs = wg / ngroups;                       // (batch element, segment)
     const unsigned grp = wg - bs * ngroups;
-    const unsigned nseg = static_cast<unsigned>(p.nseg);
-    const long b = bs / nseg;
-    const int seg = static_cast<int>(bs - static_cast<unsigned>(b) * nseg);
-    const long t00 = static_cast<long>(seg) * p.Ls;         // the workgroup's first step
+    const long b = SEG ? bs / static_cast<unsigned>(p.nseg) : bs;
+    const int seg = SEG ? static_cast<int>(bs - static_cast<unsigned>(b) * static_cast<unsigned>(p.nseg)) : 0;
+    const long t00 = SEG ? static_cast<long>(seg) * p.Ls : 0;   // the workgroup's first step
     const long d = static_cast<long>(grp) * DL + dl;
     const bool dvalid = d < p.D;
     const int dc = static_cast<int>(dvalid ? d : p.D - 1);
-    const int L = static_cast<int>(min(static_cast<long>(p.Ls), p.L - t00));
+    const int L = static_cast<int>(SEG ? min(static_cast<long>(p.Ls), p.L - t00) : p.L);
     const int Dm = static_cast<int>(p.D);
     const int nit = (L + SC - 1) / SC;
     const bool store_y = dvalid && ns == 0;
@@ -277,21 +278,31 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
     for (int j = w; j < NPL; j += W) {
         const long hi = (b * Dm + dc) * N + NS * j + ns;
         float run = p.h0 ? p.h0[hi] : 0.f;
-        if (const int nm = seg * p.map_per) {
-            constexpr int kFoldRun = 8;
-            const float a2 = p.A[dc * N + NS * j + ns] * kLog2e;
-            const long m0 = b * p.nmap * Dm + dc;
-            for (int s0 = 0; s0 < nm; s0 += kFoldRun) {
-                float ds[kFoldRun], hv[kFoldRun];
+        if constexpr (SEG) {
+            if (const int nm = seg * p.map_per) {
+                constexpr int kFoldRun = 8;
+                const float a2 = p.A[dc * N + NS * j + ns] * kLog2e, first = run;
+                const long m0 = b * p.nmap * Dm + dc;
+                for (int s0 = 0; s0 < nm; s0 += kFoldRun) {
+                    float ds[kFoldRun], hv[kFoldRun];
 #pragma unroll
-                for (int i = 0; i < kFoldRun; ++i) {
-                    const long m = m0 + static_cast<long>(min(s0 + i, nm - 1)) * Dm;
-                    ds[i] = p.seg_dsum[m];
-                    hv[i] = p.seg_h[m * N + NS * j + ns];
+                    for (int i = 0; i < kFoldRun; ++i) {
+                        const long m = m0 + static_cast<long>(min(s0 + i, nm - 1)) * Dm;
+                        ds[i] = p.seg_dsum[m];
+                        hv[i] = p.seg_h[m * N + NS * j + ns];
+                    }
+#pragma unroll
+                    for (int i = 0; i < kFoldRun; ++i)
+                        if (s0 + i < nm) run = fmaf(exp2_fast(ds[i] * a2), run, hv[i]);
                 }
-#pragma unroll
-                for (int i = 0; i < kFoldRun; ++i)
-                    if (s0 + i < nm) run = fmaf(exp2_fast(ds[i] * a2), run, hv[i]);
+                if (fold_overflowed(run)) {
+                    run = first;
+#pragma unroll 1
+                    for (int i = 0; i < nm; ++i) {
+                        const long m = m0 + static_cast<long>(i) * Dm;
+                        run = decay_add(p.seg_dsum[m] * a2, run, p.seg_h[m * N + NS * j + ns]);
+                    }
+                }
             }
         }
         carry[0][j][lane] = run;
@@ -538,7 +549,7 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
     for (int j = 0; j < NPL; ++j) nan_seen |= !(fabsf(h[j]) <= 1000.f);
     const int bad = p.clamp && (nan_seen || hmax > 1000.f);
     if (__syncthreads_or(bad)) {
-        if (p.clamp_flag) {
+        if (SEG && p.clamp_flag) {
             // A segment of a split sequence: states entering later segments
             // are also off, so the whole sequence is re-run by the repair.
             if (tid == 0) p.clamp_flag[b * ngroups + grp] = 1;
@@ -554,7 +565,7 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
         }
         return;
     }
-    if (w == W - 1 && p.hfin && dvalid && seg == p.nseg - 1) {
+    if (w == W - 1 && p.hfin && dvalid && (!SEG || seg == p.nseg - 1)) {
 #pragma unroll
         for (int j = 0; j < NPL; ++j) p.hfin[(b * Dm + d) * N + NS * j + ns] = h[j];
     }
@@ -613,7 +624,7 @@ static int launch_chunked(const Scan1DFwdArgs &a, bool shared, bool hist, hipStr
     // B*u is kept in registers only without history stores or gating, whose
     // extra registers would otherwise spill.
 #define KM_CH(SH, HI, GA) \
-    hipLaunchKernelGGL((scan1d_fwd_chunked<T, NPL, NS, W, TC, SH, HI, SBU && !HI && !GA, OCC, GA>), \
+    hipLaunchKernelGGL((scan1d_fwd_chunked<T, NPL, NS, W, TC, SH, HI, SBU && !HI && !GA, OCC, GA, false>), \
                        g, blk, 0, s, a)
     if (shared) {
         if (hist) { if (gate) KM_CH(true, true, true); else KM_CH(true, true, false); }
@@ -783,7 +794,7 @@ static int launch_segmented(const KMScan1DFwd *k, const Scan1DFwdArgs &base, lon
     q.clamp_flag = m.clamp_flag;
     if (alias) q.h0 = m.h0_copy;
 #define KM_SEGR(SH, HI, GA) \
-    hipLaunchKernelGGL((scan1d_fwd_chunked<T, NPL, NS, WS, 8, SH, HI, !HI && !GA, 2, GA>), \
+    hipLaunchKernelGGL((scan1d_fwd_chunked<T, NPL, NS, WS, 8, SH, HI, !HI && !GA, 2, GA, true>), \
                        dim3(static_cast<unsigned>(grid)), dim3(64 * WS), 0, s, q)
     if (shared) {
         if (hist) { if (gate) KM_SEGR(true, true, true); else KM_SEGR(true, true, false); }

@@ -16,6 +16,20 @@
 
 namespace km {
 
+// A fold of maps takes h to 2^z h + add from map to map, z the exponent of the
+// decay over the map's steps, which may be out of range by itself: with 2^z =
+// inf a state of exactly 0 (padded x, masked dy) becomes NaN, with 2^z = 0 an
+// infinite one. An overflow anywhere leaves the fold's result infinite or NaN
+// in some lane; then it is run again with decay_add, where the integer part of
+// z goes to h's exponent, so that a product is in range where the steps' own
+// products are. (decay_add in every fold takes 1 us of the 72 us of B1 L5003
+// D1536 bf16 gated; the check 0.2.)
+__device__ __forceinline__ bool fold_overflowed(float h) { return __any(!(fabsf(h) < __builtin_inff())); }
+__device__ __forceinline__ float decay_add(float z, float h, float add) {
+    const float k = fminf(fmaxf(floorf(z), -1e9f), 1e9f);
+    return fmaf(exp2_fast(z - k), __builtin_amdgcn_ldexpf(h, static_cast<int>(k)), add);
+}
+
 struct MapArgs {
     const void *x;         // [B, L, D] the forward's x, the adjoint's dy
     const void *dt;        // [B, L, D]
@@ -177,6 +191,14 @@ __global__ void __launch_bounds__(64 * kMapWaves, 4) scan1d_segment_map(MapArgs 
             for (int u = 0; u < W; ++u) {
                 const int v = ADJ ? W - 1 - u : u;
                 run = fmaf(exp2_fast(sds[v][c] * a2), run, lds[(v * N + n) * PADC + c]);
+            }
+            if (fold_overflowed(run)) {
+                run = 0.f;
+#pragma unroll 1
+                for (int u = 0; u < W; ++u) {
+                    const int v = ADJ ? W - 1 - u : u;
+                    run = decay_add(sds[v][c] * a2, run, lds[(v * N + n) * PADC + c]);
+                }
             }
             p.seg_h[(static_cast<long>(bs) * p.D + dd) * N + n] = run;
             if (!ADJ && part == 0 && p.h0_copy)

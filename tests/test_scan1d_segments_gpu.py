@@ -171,3 +171,76 @@ def test_backward_segments_clamped_states():
     got, _ = _bwd(x, dt, A, Bm, Cm, dy, mode="ckpt", strides=strides)
     for n, a, r, k in zip(("dx", "ddelta", "dA", "dB", "dC"), got, ref, kap):
         assert_close(a, r, TOL_F32, n, k)
+
+
+# --- decays over a whole segment that are out of range -----------------------------
+
+def _growing(Bsz, L, D, kind):
+    """Decays of up to e^2 a step: over the parts of a split (64 steps or more)
+    they overflow, while the 20 steps that carry data keep every value finite."""
+    x, dt, _, Bm, Cm = scan1d_inputs(Bsz, L, D, N, seed=51)
+    dt = np.full_like(dt, 0.5)
+    if kind == "structured":
+        A = np.tile(np.arange(1, N + 1, dtype=np.float32) / 4, (D, 1))
+    elif kind == "generic":
+        A = np.tile(np.where(np.arange(N) % 2, -3.0, 4.0).astype(np.float32), (D, 1))
+    else:                                       # negative steps
+        A = -np.tile(np.arange(1, N + 1, dtype=np.float32) / 4, (D, 1))
+        dt = -dt
+    return x, dt, A, Bm, Cm
+
+
+@pytest.mark.parametrize("L", [1024, 1001])
+@pytest.mark.parametrize("kind", ["structured", "generic", "negative delta"])
+def test_growing_decays_keep_padding_zero(L, kind):
+    Bsz, D = 2, 40
+    x, dt, A, Bm, Cm = _growing(Bsz, L, D, kind)
+    x[:, :L - 20] = 0.0                         # padded at the front
+    yr, hr, _ = O.scan1d_batched(x, dt, A, Bm, Cm, clamp=False)
+    assert np.isfinite(yr).all() and np.isfinite(hr).all()
+    ky, kh, _ = (np.abs(a) for a in scan1d_kappa(x, np.abs(dt), A * np.sign(dt[0, 0, 0]), Bm, Cm))
+    y = torch.full((Bsz, L, D), float("nan"), device=DEV)
+    hf = torch.full((Bsz, D, N), float("nan"), device=DEV)
+    K.scan1d_fwd(*(T(a) for a in (x, dt, A, Bm, Cm)), y, h_final=hf, clamp=False)
+    assert_close(y.cpu().numpy(), yr, TOL_F32, "y", ky)
+    assert_close(hf.cpu().numpy(), hr, TOL_F32, "h_final", kh)
+
+
+def test_overflowed_state_stays_infinite():
+    # Without the clamp an infinite state decays to itself, however far the
+    # decay over the following segments underflows.
+    Bsz, L, D = 1, 1001, 64
+    x, dt, A, Bm, Cm = scan1d_inputs(Bsz, L, D, N, seed=52)
+    x[:, 100] = 3e38
+    Bm[:, 100] = 40.0
+    hr = O.scan1d_batched(x, dt, A, Bm, Cm, clamp=False)[1]
+    assert np.isposinf(hr).all()
+    hf = torch.zeros((Bsz, D, N), device=DEV)
+    K.scan1d_fwd(*(T(a) for a in (x, dt, A, Bm, Cm)), torch.empty((Bsz, L, D), device=DEV), h_final=hf, clamp=False)
+    assert np.isposinf(hf.cpu().numpy()).all()
+
+
+@pytest.mark.parametrize("L", [1024, 1001])
+@pytest.mark.parametrize("kind", ["structured", "generic"])
+@pytest.mark.parametrize("mode", ["hist", "ckpt"])
+def test_growing_decays_backward_of_masked_loss(L, kind, mode):
+    # dy reaches only the first 20 steps: the adjoint is exactly zero after.
+    Bsz, D = 2, 40
+    x, dt, A, Bm, Cm = _growing(Bsz, L, D, kind)
+    dy = rng_for("masked", L).standard_normal((Bsz, L, D)).astype(np.float32)
+    dy[:, 20:] = 0.0
+    if mode == "ckpt":
+        x[:, 30:] = 0.0                         # the clamp keeps the states finite
+    strides = (L * N, N, 0)
+    hh = O.scan1d_batched(x, dt, A, Bm, Cm, hist=True)[2]
+    ref = O.scan1d_batched_backward(x, dt, A, Bm, Cm, dy, hh)
+    assert all(np.isfinite(r).all() for r in ref)
+    ax, aB, aC, ady = (np.abs(a) for a in (x, Bm, Cm, dy))
+    kap = O.scan1d_batched_backward(ax, dt, np.abs(A) if kind == "structured" else A, aB, aC, ady, np.abs(hh))
+    got, _ = _bwd(x, dt, A, Bm, Cm, dy, mode=mode, strides=strides, hist=hh)
+    for n, a, r, k in zip(("dx", "ddelta", "dA", "dB", "dC"), got, ref, kap):
+        assert np.isfinite(a).all(), n
+        if kind == "structured":
+            assert_close(a, r, TOL_F32, n, np.abs(k))
+        else:                                   # mixed signs of A: per tensor
+            assert np.abs(a - r).max() <= TOL_F32 * np.abs(r).max(), n
