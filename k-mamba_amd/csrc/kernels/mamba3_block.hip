@@ -12,7 +12,8 @@
 //   1. proj: P = X . Wcat^T, the R + 2 + 2NR controller rows of every token
 //      at once (fp32 matrix cores).
 //   2. scan: per step the decay a_t = alpha and the drive c_t = beta Bu_{t-1}
-//      + gamma Bu_t, which do not depend on h, and h_t = a_t * R(theta)
+//      + gamma Bu_t, which do not depend on h (long sequences on few workgroups
+//      and many ranks: in a kernel before it), and h_t = a_t * R(theta)
 //      h_{t-1} + c_t per state pair, a chunked scan of 2x2 maps: a workgroup
 //      per (batch element, pair), a thread per chunk of steps.
 //   3. out: Y[t, r] = sum_n C_t[r, n] h_t[n] and out = x + W_out Y.
@@ -20,6 +21,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 #include "km_device.hpp"
 #include "../km_runtime.hpp"
@@ -41,6 +43,7 @@ struct M3Args {
     // Time runs along the rows (of Tp >= T values), so that the scan's threads,
     // each on a few consecutive steps, read and write whole lines together.
     float *P;             // [J, Tp]
+    float *a, *c;         // [N, Tp] (m3_prep)
     float *H;             // [N, Tp]
     long Tp;
     float *Y;             // [T, R] (general output path)
@@ -225,7 +228,7 @@ __global__ void __launch_bounds__(64 * kM3Split) m3_proj_mfma(M3Args p) {
 // ---- 2. per-step decay and drive --------------------------------------------
 __device__ __forceinline__ float silu_f(float v) { return v / (1.f + expf(-v)); }
 
-__device__ __forceinline__ void m3_ctrl_of(const M3Args &p, float rd, float rl, float &dt, float &lam) {
+__device__ __forceinline__ void m3_ctrl(const M3Args &p, float rd, float rl, float &dt, float &lam) {
     if (p.has_delta) {
         float v = logf(1.f + expf(rd));
         v = v < p.dt_min ? p.dt_min : v;
@@ -234,9 +237,6 @@ __device__ __forceinline__ void m3_ctrl_of(const M3Args &p, float rd, float rl, 
         dt = p.dt_scale;
     }
     lam = p.has_lambda ? 1.f / (1.f + expf(-rl)) : 0.5f;
-}
-__device__ __forceinline__ void m3_ctrl(const M3Args &p, long t, float &dt, float &lam) {
-    m3_ctrl_of(p, p.P[p.R * p.Tp + t], p.P[(p.R + 1) * p.Tp + t], dt, lam);
 }
 
 // Bu_t[n] = sum_r (W_B x_t + b_B)[r, n] * SiLU(W_in x_t)[r].
@@ -247,21 +247,39 @@ __device__ __forceinline__ float m3_bu(const M3Args &p, long t, long n) {
     return s;
 }
 
+// Both of every step and state, for m3_scan<PREP>: whole chip, time along the
+// lanes. a_t = alpha, c_t = beta Bu_{t-1} + gamma Bu_t.
+__global__ void __launch_bounds__(256) m3_prep(M3Args p) {
+    const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
+    const long n = i / p.Tp, t = i - n * p.Tp;
+    if (n >= p.N || t >= p.T) return;
+    float dt, lam;
+    m3_ctrl(p, p.P[p.R * p.Tp + t], p.P[(p.R + 1) * p.Tp + t], dt, lam);
+    const float alpha = expf(dt * p.A[n]);
+    const float bu = m3_bu(p, t, n);
+    const float pbu = t % p.L > 0 ? m3_bu(p, t - 1, n) : 0.f;
+    p.a[i] = alpha;
+    p.c[i] = (1.f - lam) * dt * alpha * pbu + lam * dt * bu;
+}
+
 // ---- the recurrence ------------------------------------------------------
 // Per state pair (2i, 2i+1) of one batch element, h_t = M_t h_{t-1} + c_t
 // with M_t = diag(a0_t, a1_t) R(theta): a linear recurrence of 2x2 maps, so
 // it runs as a chunked scan. One workgroup of kM3ScanW waves per (batch
-// element, pair); thread k owns the chunk of CH = ceil(L / (64 kM3ScanW))
-// consecutive steps. (1) Each thread forms its steps' decays and drives from
-// the controller rows and composes its chunk's map h -> P h + v from a zero
-// state. (2) An inclusive scan of the maps across the lanes of
-// each wave (Hillis-Steele, lane shuffles), then the waves' total maps
-// through LDS, give every chunk the state entering it. (3) Each thread
-// replays its steps from that state with the sequential step formula,
-// writing H. An odd last state has no partner: M_t = diag(a0_t, 0) and no
-// rotation. ONE: the chunk is at most kM3Chunk steps, whose decays and drives
-// stay in registers for the replay (longer chunks form them again).
+// element, pair) walks the sequence in super-chunks, thread k of them on CH
+// <= kM3Chunk consecutive steps. (1) Each thread forms its steps' decays and
+// drives from the controller rows (PREP: reads m3_prep's) and composes its
+// chunk's map h -> P h + v from a zero state. (2) An inclusive scan of the maps
+// across the lanes of each wave (Hillis-Steele, lane shuffles), then the waves'
+// total maps through LDS, give every chunk the state entering it, and the next
+// super-chunk its first. (3) Each thread replays its steps from that state with
+// the sequential step formula, writing H. An odd last state has no partner: M_t
+// = diag(a0_t, 0) and no rotation. FULL: chunks of kM3Chunk steps, so no branch
+// between a chunk's steps.
 constexpr int kM3ScanW = 4, kM3Chunk = 8;
+inline __host__ __device__ int m3_chunk(long L) {
+    return static_cast<int>(std::min<long>(kM3Chunk, (L + 64 * kM3ScanW - 1) / (64 * kM3ScanW)));
+}
 __device__ __forceinline__ void m3_step(float a0, float a1, float cs, float sn, bool pair,
                                         float c0, float c1, float &h0, float &h1) {
     if (pair) {
@@ -273,160 +291,147 @@ __device__ __forceinline__ void m3_step(float a0, float a1, float cs, float sn, 
     }
 }
 
-template <bool ONE>
+template <bool PREP, bool FULL>
 __global__ void __launch_bounds__(64 * kM3ScanW) m3_scan(M3Args p, long npairs) {
-    __shared__ float wmap[kM3ScanW][6];          // each wave's total map (P, v)
+    __shared__ float wmap[2][kM3ScanW][6];       // each wave's total map (P, v), by super-chunk parity
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const long b = blockIdx.x / npairs, pi = blockIdx.x % npairs;
     const long n0 = 2 * pi, n1 = n0 + 1;
     const bool pair = n1 < p.N;
     const float th = pair ? p.theta[pi] : 0.f;
     const float cs = pair ? cosf(th) : 1.f, sn = pair ? sinf(th) : 0.f;
-    const long L = p.L, N = p.N;
-    const long CH = (L + 64 * kM3ScanW - 1) / (64 * kM3ScanW);
-    const long l0 = tid * CH, l1 = min(l0 + CH, L);
-    const long tb = b * L;
+    const long L = p.L, N = p.N, tb = b * L;
+    const int CH = FULL ? kM3Chunk : m3_chunk(L);
     const float A0 = p.A[n0], A1 = pair ? p.A[n1] : 0.f;
-    // Decay and drive of both states at step l; (q0, q1) is Bu of step l - 1
-    // on entry and of step l on return.
-    auto step = [&](long l, float &q0, float &q1, float &a0, float &a1, float &c0, float &c1) {
-        const long t = tb + l;
-        float dt, lam;
-        m3_ctrl(p, t, dt, lam);
-        const float b0 = m3_bu(p, t, n0), b1 = pair ? m3_bu(p, t, n1) : 0.f;
-        a0 = expf(dt * A0);
-        a1 = pair ? expf(dt * A1) : 0.f;
-        c0 = (1.f - lam) * dt * a0 * q0 + lam * dt * b0;
-        c1 = (1.f - lam) * dt * a1 * q1 + lam * dt * b1;
-        q0 = b0;
-        q1 = b1;
-    };
-    // ONE: every step's controller values are loaded together (steps past the
-    // chunk reload its last one), one memory latency for the chunk. Entry u is
-    // step l0 - 1 + u.
-    constexpr int KU = ONE ? kM3Chunk + 1 : 1;
-    float kb0[KU], kb1[KU], kd[KU], kl[KU];
-    const bool prev = l0 > 0 && l0 < l1;
-    if constexpr (ONE) {
-        int at[KU];
-        const float *Pb = p.P + tb;
+    float *const H0 = p.H + n0 * p.Tp + tb, *const H1 = p.H + (pair ? n1 : n0) * p.Tp + tb;
+    float E0 = 0.f, E1 = 0.f;                    // the state entering the super-chunk
+    int par = 0;
+    for (long s0 = 0; s0 < L; s0 += 64 * kM3ScanW * CH, par ^= 1) {
+        const long l0 = s0 + tid * CH, l1 = min(l0 + CH, L);
+        // The chunk's decays and drives. Every load of the chunk goes out
+        // together (steps past its end reload the last one): one memory
+        // latency for the chunk.
+        float ka0[kM3Chunk], ka1[kM3Chunk], kc0[kM3Chunk], kc1[kM3Chunk];
+        if constexpr (PREP) {
+            const float *const a0 = p.a + n0 * p.Tp + tb, *const a1 = p.a + (pair ? n1 : n0) * p.Tp + tb;
+            const float *const c0 = p.c + n0 * p.Tp + tb, *const c1 = p.c + (pair ? n1 : n0) * p.Tp + tb;
 #pragma unroll
-        for (int u = 0; u < KU; ++u) {
-            at[u] = static_cast<int>(std::min(std::max(l0 - 1 + u, 0L), L - 1));
-            kb0[u] = 0.f;
-            kb1[u] = 0.f;
-            kd[u] = Pb[p.R * p.Tp + at[u]];
-            kl[u] = Pb[(p.R + 1) * p.Tp + at[u]];
-        }
-        for (long r = 0; r < p.R; ++r) {
-            const long o = p.R + 2 + r * N;
-            const float c0 = p.bB[r * N + n0], c1 = pair ? p.bB[r * N + n1] : 0.f;
-            float zz[KU], x0[KU], x1[KU];
+            for (int u = 0; u < kM3Chunk; ++u) {
+                const long at = min(l0 + u, L - 1);
+                ka0[u] = a0[at];
+                ka1[u] = pair ? a1[at] : 0.f;
+                kc0[u] = c0[at];
+                kc1[u] = pair ? c1[at] : 0.f;
+            }
+        } else {
+            // Entry u of the controller values is step l0 - 1 + u.
+            constexpr int KU = kM3Chunk + 1;
+            float kb0[KU], kb1[KU], kd[KU], kl[KU];
+            long at[KU];
+            const float *const Pb = p.P + tb;
 #pragma unroll
             for (int u = 0; u < KU; ++u) {
-                zz[u] = Pb[r * p.Tp + at[u]];
-                x0[u] = Pb[(o + n0) * p.Tp + at[u]];
-                x1[u] = Pb[(o + (pair ? n1 : n0)) * p.Tp + at[u]];
+                at[u] = min(max(l0 - 1 + u, 0L), L - 1);
+                kb0[u] = 0.f;
+                kb1[u] = 0.f;
+                kd[u] = Pb[p.R * p.Tp + at[u]];
+                kl[u] = Pb[(p.R + 1) * p.Tp + at[u]];
+            }
+            for (long r = 0; r < p.R; ++r) {
+                const long o = p.R + 2 + r * N;
+                const float c0 = p.bB[r * N + n0], c1 = pair ? p.bB[r * N + n1] : 0.f;
+                float zz[KU], x0[KU], x1[KU];
+#pragma unroll
+                for (int u = 0; u < KU; ++u) {
+                    zz[u] = Pb[r * p.Tp + at[u]];
+                    x0[u] = Pb[(o + n0) * p.Tp + at[u]];
+                    x1[u] = Pb[(o + (pair ? n1 : n0)) * p.Tp + at[u]];
+                }
+#pragma unroll
+                for (int u = 0; u < KU; ++u) {
+                    const float sz = silu_f(zz[u]);
+                    kb0[u] += (x0[u] + c0) * sz;
+                    kb1[u] += pair ? (x1[u] + c1) * sz : 0.f;
+                }
             }
 #pragma unroll
-            for (int u = 0; u < KU; ++u) {
-                const float sz = silu_f(zz[u]);
-                kb0[u] += (x0[u] + c0) * sz;
-                kb1[u] += pair ? (x1[u] + c1) * sz : 0.f;
-            }
-        }
-    }
-    const float e0 = ONE ? 0.f : prev ? m3_bu(p, tb + l0 - 1, n0) : 0.f;
-    const float e1 = ONE ? 0.f : prev && pair ? m3_bu(p, tb + l0 - 1, n1) : 0.f;
-
-    // (1) chunk map: P (2x2) and v, composed step by step from identity / 0.
-    float P00 = 1.f, P01 = 0.f, P10 = 0.f, P11 = 1.f, v0 = 0.f, v1 = 0.f;
-    float ka0[ONE ? kM3Chunk : 1], ka1[ONE ? kM3Chunk : 1], kc0[ONE ? kM3Chunk : 1], kc1[ONE ? kM3Chunk : 1];
-    auto compose = [&](float a0, float a1, float c0, float c1) {
-        const float m00 = pair ? a0 * cs : a0, m01 = pair ? -a0 * sn : 0.f;
-        const float m10 = a1 * sn, m11 = a1 * cs;
-        const float q00 = m00 * P00 + m01 * P10, q01 = m00 * P01 + m01 * P11;
-        const float q10 = m10 * P00 + m11 * P10, q11 = m10 * P01 + m11 * P11;
-        P00 = q00; P01 = q01; P10 = q10; P11 = q11;
-        m3_step(a0, a1, cs, sn, pair, c0, c1, v0, v1);
-    };
-    float q0 = e0, q1 = e1;
-    if constexpr (ONE) {
-#pragma unroll
-        for (int u = 0; u < kM3Chunk; ++u) {
-            if (l0 + u < l1) {
+            for (int u = 0; u < kM3Chunk; ++u) {
+                if (!FULL && l0 + u >= l1) continue;
                 float dt, lam;
-                m3_ctrl_of(p, kd[u + 1], kl[u + 1], dt, lam);
+                m3_ctrl(p, kd[u + 1], kl[u + 1], dt, lam);
                 const float pb0 = l0 + u > 0 ? kb0[u] : 0.f, pb1 = l0 + u > 0 ? kb1[u] : 0.f;
                 ka0[u] = expf(dt * A0);
                 ka1[u] = pair ? expf(dt * A1) : 0.f;
                 kc0[u] = (1.f - lam) * dt * ka0[u] * pb0 + lam * dt * kb0[u + 1];
                 kc1[u] = (1.f - lam) * dt * ka1[u] * pb1 + lam * dt * kb1[u + 1];
-                compose(ka0[u], ka1[u], kc0[u], kc1[u]);
             }
         }
-    } else {
-        for (long l = l0; l < l1; ++l) {
-            float a0, a1, c0, c1;
-            step(l, q0, q1, a0, a1, c0, c1);
-            compose(a0, a1, c0, c1);
-        }
-    }
-    // (2) inclusive scan over the wave's lanes: (P, v) <- (P, v) o (P', v')
-    // of lane - d; then the waves' totals.
+
+        // (1) chunk map: P (2x2) and v, composed step by step from identity / 0.
+        float P00 = 1.f, P01 = 0.f, P10 = 0.f, P11 = 1.f, v0 = 0.f, v1 = 0.f;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const float e00 = __shfl_up(P00, d), e01 = __shfl_up(P01, d);
-        const float e10 = __shfl_up(P10, d), e11 = __shfl_up(P11, d);
-        const float w0 = __shfl_up(v0, d), w1 = __shfl_up(v1, d);
-        if (lane >= d) {
-            const float nv0 = P00 * w0 + P01 * w1 + v0, nv1 = P10 * w0 + P11 * w1 + v1;
-            const float q00 = P00 * e00 + P01 * e10, q01 = P00 * e01 + P01 * e11;
-            const float q10 = P10 * e00 + P11 * e10, q11 = P10 * e01 + P11 * e11;
-            P00 = q00; P01 = q01; P10 = q10; P11 = q11;
-            v0 = nv0; v1 = nv1;
+        for (int u = 0; u < kM3Chunk; ++u) {
+            if (l0 + u < l1) {
+                const float a0 = ka0[u], a1 = ka1[u];
+                const float m00 = pair ? a0 * cs : a0, m01 = pair ? -a0 * sn : 0.f;
+                const float m10 = a1 * sn, m11 = a1 * cs;
+                const float q00 = m00 * P00 + m01 * P10, q01 = m00 * P01 + m01 * P11;
+                const float q10 = m10 * P00 + m11 * P10, q11 = m10 * P01 + m11 * P11;
+                P00 = q00; P01 = q01; P10 = q10; P11 = q11;
+                m3_step(a0, a1, cs, sn, pair, kc0[u], kc1[u], v0, v1);
+            }
         }
-    }
-    if (lane == 63) {
-        wmap[w][0] = P00; wmap[w][1] = P01; wmap[w][2] = P10; wmap[w][3] = P11;
-        wmap[w][4] = v0; wmap[w][5] = v1;
-    }
-    __syncthreads();
-    // State entering this wave: the earlier waves' maps applied in order to 0.
-    float V0 = 0.f, V1 = 0.f;
-    for (int u = 0; u < w; ++u) {
-        const float n0v = wmap[u][0] * V0 + wmap[u][1] * V1 + wmap[u][4];
-        const float n1v = wmap[u][2] * V0 + wmap[u][3] * V1 + wmap[u][5];
-        V0 = n0v;
-        V1 = n1v;
-    }
-    // (3) replay from the state after the previous chunk: lane k > 0 of the
-    // wave starts from lane k-1's inclusive map applied to V.
-    const float i00 = __shfl_up(P00, 1), i01 = __shfl_up(P01, 1);
-    const float i10 = __shfl_up(P10, 1), i11 = __shfl_up(P11, 1);
-    const float w0 = __shfl_up(v0, 1), w1 = __shfl_up(v1, 1);
-    float h0 = V0, h1 = V1;
-    if (lane > 0) {
-        h0 = i00 * V0 + i01 * V1 + w0;
-        h1 = i10 * V0 + i11 * V1 + w1;
-    }
-    float *H0 = p.H + n0 * p.Tp + tb, *H1 = p.H + (pair ? n1 : n0) * p.Tp + tb;
-    auto emit = [&](long l, float a0, float a1, float c0, float c1) {
-        m3_step(a0, a1, cs, sn, pair, c0, c1, h0, h1);
-        H0[l] = h0;
-        if (pair) H1[l] = h1;
-    };
-    if constexpr (ONE) {
+        // (2) inclusive scan over the wave's lanes: (P, v) <- (P, v) o (P', v')
+        // of lane - d; then the waves' totals.
 #pragma unroll
-        for (int u = 0; u < kM3Chunk; ++u)
-            if (l0 + u < l1) emit(l0 + u, ka0[u], ka1[u], kc0[u], kc1[u]);
-    } else {
-        q0 = e0;
-        q1 = e1;
-        for (long l = l0; l < l1; ++l) {
-            float a0, a1, c0, c1;
-            step(l, q0, q1, a0, a1, c0, c1);
-            emit(l, a0, a1, c0, c1);
+        for (int d = 1; d < 64; d <<= 1) {
+            const float e00 = __shfl_up(P00, d), e01 = __shfl_up(P01, d);
+            const float e10 = __shfl_up(P10, d), e11 = __shfl_up(P11, d);
+            const float w0 = __shfl_up(v0, d), w1 = __shfl_up(v1, d);
+            if (lane >= d) {
+                const float nv0 = P00 * w0 + P01 * w1 + v0, nv1 = P10 * w0 + P11 * w1 + v1;
+                const float q00 = P00 * e00 + P01 * e10, q01 = P00 * e01 + P01 * e11;
+                const float q10 = P10 * e00 + P11 * e10, q11 = P10 * e01 + P11 * e11;
+                P00 = q00; P01 = q01; P10 = q10; P11 = q11;
+                v0 = nv0; v1 = nv1;
+            }
+        }
+        if (lane == 63) {
+            wmap[par][w][0] = P00; wmap[par][w][1] = P01; wmap[par][w][2] = P10; wmap[par][w][3] = P11;
+            wmap[par][w][4] = v0; wmap[par][w][5] = v1;
+        }
+        __syncthreads();
+        // State entering this wave: the earlier waves' maps applied in order;
+        // all of them: the state entering the next super-chunk.
+        float V0 = E0, V1 = E1;
+#pragma unroll
+        for (int u = 0; u < kM3ScanW; ++u) {
+            if (u == w) {
+                V0 = E0;
+                V1 = E1;
+            }
+            const float f0 = wmap[par][u][0] * E0 + wmap[par][u][1] * E1 + wmap[par][u][4];
+            const float f1 = wmap[par][u][2] * E0 + wmap[par][u][3] * E1 + wmap[par][u][5];
+            E0 = f0;
+            E1 = f1;
+        }
+        // (3) replay from the state after the previous chunk: lane k > 0 of the
+        // wave starts from lane k-1's inclusive map applied to V.
+        const float i00 = __shfl_up(P00, 1), i01 = __shfl_up(P01, 1);
+        const float i10 = __shfl_up(P10, 1), i11 = __shfl_up(P11, 1);
+        const float w0 = __shfl_up(v0, 1), w1 = __shfl_up(v1, 1);
+        float h0 = V0, h1 = V1;
+        if (lane > 0) {
+            h0 = i00 * V0 + i01 * V1 + w0;
+            h1 = i10 * V0 + i11 * V1 + w1;
+        }
+#pragma unroll
+        for (int u = 0; u < kM3Chunk; ++u) {
+            if (l0 + u < l1) {
+                m3_step(ka0[u], ka1[u], cs, sn, pair, kc0[u], kc1[u], h0, h1);
+                H0[l0 + u] = h0;
+                if (pair) H1[l0 + u] = h1;
+            }
         }
     }
 }
@@ -527,6 +532,21 @@ __global__ void __launch_bounds__(256) m3_upload(const float *src, float *dst, l
 
 static long grid256(long n) { return (n + 255) / 256; }
 
+// Whether decays and drives are formed by m3_prep, over the whole chip, or by
+// the scan's own threads (twice the states, not the steps, apart). Few scan
+// workgroups (one per batch element and pair): their time is R loads and drives
+// for every chunk of a thread in turn, against one more launch. Scan / m3_prep,
+// N 16, whole call (us): B1 R1 L1000 34.3 / 35.3, L4096 49.0 / 45.4, L16384 114
+// / 90; B1 L2048 R4 53.4 / 46.9, R16 120 / 87. Enough of them to fill the chip:
+// the scan's own, B64 L2048 R1 128 / 139, R2 203 / 213, unless there are many
+// ranks (B64 L256 R8 93.1 / 88.6) or sequences so short that most of a
+// workgroup idles (B4000 L16 R1 226 / 143).
+static bool m3_prep_wanted(long B, long L, long N, long R) {
+    const long wgs = B * ((N + 1) / 2);
+    if (wgs < 256) return R * ((L + 255) / 256) > 8;
+    return R > 4 || (L <= 256 && wgs >= 1024);
+}
+
 int mamba3_launch(M3Args &a, hipStream_t s) {
     if (a.T <= 0) return 0;
     if (grid256(a.T * std::max(a.N, a.D)) > 0x7fffffffL) {
@@ -568,8 +588,16 @@ int mamba3_launch(M3Args &a, hipStream_t s) {
     }
     const long npairs = (a.N + 1) / 2;
     const dim3 gs(static_cast<unsigned>((a.T / a.L) * npairs));   // workgroups: one per (batch element, pair)
-    if (a.L <= 64L * kM3ScanW * kM3Chunk) hipLaunchKernelGGL(m3_scan<true>, gs, dim3(64 * kM3ScanW), 0, s, a, npairs);
-    else                                 hipLaunchKernelGGL(m3_scan<false>, gs, dim3(64 * kM3ScanW), 0, s, a, npairs);
+    const bool full = m3_chunk(a.L) == kM3Chunk;
+    const dim3 bs(64 * kM3ScanW);
+    if (a.a) {
+        hipLaunchKernelGGL(m3_prep, dim3(static_cast<unsigned>(grid256(a.Tp * a.N))), dim3(256), 0, s, a);
+        if (full) hipLaunchKernelGGL((m3_scan<true, true>), gs, bs, 0, s, a, npairs);
+        else      hipLaunchKernelGGL((m3_scan<true, false>), gs, bs, 0, s, a, npairs);
+    } else {
+        if (full) hipLaunchKernelGGL((m3_scan<false, true>), gs, bs, 0, s, a, npairs);
+        else      hipLaunchKernelGGL((m3_scan<false, false>), gs, bs, 0, s, a, npairs);
+    }
     const bool al16 = ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
     const long gt = (a.T + kM3OutT - 1) / kM3OutT;
     if (a.D % 4 == 0 && al16 && a.R <= kM3OutR && gt <= 65535) {
@@ -705,12 +733,13 @@ void mamba_block_forward(MambaBlock *b, float *output, const float *input, size_
     const bool has_lambda = b->lambda_proj.rows > 0 && b->lambda_proj.data;
     const long J = R + 2 + 2 * NR;
     const long TS = N / 2 > 0 ? N / 2 : 1, Tp = (T + 63) / 64 * 64;
+    const bool prep = km::m3_prep_wanted(static_cast<long>(batch_size), L, N, R);
     const bool dev_io = km::is_device_ptr(input) && km::is_device_ptr(output);
     km::Staging::lock();
     do {
         const size_t io_bytes = dev_io ? 0 : 2 * km::align_up(sizeof(float) * T * D, 256);
         const size_t bytes = io_bytes + sizeof(float) * (J * D + D * R + N + 2 * NR + TS) + 8 * 256 +
-                             sizeof(float) * (Tp * J + Tp * N + T * R) + 8 * 256;
+                             sizeof(float) * (Tp * J + (prep ? 3 : 1) * Tp * N + T * R) + 8 * 256;
         void *base = km::Staging::reserve(bytes);
         if (!base) break;
         km::Carver cv(base);
@@ -761,6 +790,10 @@ void mamba_block_forward(MambaBlock *b, float *output, const float *input, size_
         a.theta = th;
         a.P = cv.take<float>(Tp * J);
         a.H = cv.take<float>(Tp * N);
+        if (prep) {
+            a.a = cv.take<float>(Tp * N);
+            a.c = cv.take<float>(Tp * N);
+        }
         a.Tp = Tp;
         a.Y = cv.take<float>(T * R);
         a.T = T; a.L = L; a.D = D; a.N = N; a.R = R; a.J = J;

@@ -201,7 +201,16 @@ def test_kmamba_checkpoint_roundtrip_forward(tmp_path):
 # leaves part of the last output workgroup idle.
 @pytest.mark.parametrize("batch,L,dim,N,R", [(1, 1, 4, 1, 1), (3, 17, 36, 5, 2), (1, 256, 1028, 16, 1),
                                              (2, 2048, 64, 16, 4), (1, 2049, 32, 7, 1), (9, 64, 20, 16, 3),
-                                             (1, 33, 8, 40, 1)])
+                                             (1, 33, 8, 40, 1),
+                                             # Decays in a kernel of their own: chunks of eight steps (two
+                                             # whole super-chunks of 2048, one step or 1808 past them, one
+                                             # super-chunk) and of one step.
+                                             (1, 4096, 8, 16, 1), (2, 4097, 12, 5, 3), (1, 10000, 8, 3, 2),
+                                             (1, 2048, 16, 16, 16), (1, 200, 16, 8, 9), (130, 16, 8, 16, 1),
+                                             (520, 5, 4, 4, 1),
+                                             # In the scan: one whole super-chunk; several on workgroups that
+                                             # fill the chip.
+                                             (1, 2048, 32, 16, 1), (32, 2500, 4, 16, 2)])
 def test_block_tile_edges(batch, L, dim, N, R):
     p = mamba3_params(dim, N, R)
     x = rng_for("m3-edges", batch, L, dim, N, R).standard_normal((batch, L, dim)).astype(np.float32)
