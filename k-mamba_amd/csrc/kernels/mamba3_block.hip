@@ -16,7 +16,8 @@
 //      and many ranks: in a kernel before it), and h_t = a_t * R(theta)
 //      h_{t-1} + c_t per state pair, a chunked scan of 2x2 maps: a workgroup
 //      per (batch element, pair), a thread per chunk of steps.
-//   3. out: Y[t, r] = sum_n C_t[r, n] h_t[n] and out = x + W_out Y.
+//   3. out: Y[t, r] = sum_n C_t[r, n] h_t[n] and out = x + W_out Y (many
+//      ranks, or rows that are not whole 16-byte blocks: in two kernels).
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -46,7 +47,7 @@ struct M3Args {
     float *a, *c;         // [N, Tp] (m3_prep)
     float *H;             // [N, Tp]
     long Tp;
-    float *Y;             // [T, R] (general output path)
+    float *Y;             // [R, Tp] (m3_readout)
     long T, L, D, N, R, J;
     int has_delta, has_lambda;
     float dt_scale, dt_min, dt_max;
@@ -437,10 +438,11 @@ __global__ void __launch_bounds__(64 * kM3ScanW) m3_scan(M3Args p, long npairs) 
 }
 
 // ---- 3. readout and output ---------------------------------------------------
+// Y[r, t], time along the lanes.
 __global__ void __launch_bounds__(256) m3_readout(M3Args p) {
     const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= p.T * p.R) return;
-    const long t = i / p.R, r = i % p.R;
+    const long r = i / p.Tp, t = i - r * p.Tp;
+    if (r >= p.R || t >= p.T) return;
     const float *C = p.P + (p.R + 2 + p.N * p.R + r * p.N) * p.Tp + t;
     float s = 0.f;
     for (long n = 0; n < p.N; ++n) s = fmaf(C[n * p.Tp] + p.bC[r * p.N + n], p.H[n * p.Tp + t], s);
@@ -452,23 +454,33 @@ __global__ void __launch_bounds__(256) m3_out(M3Args p) {
     if (i >= p.T * p.D) return;
     const long t = i / p.D, d = i % p.D;
     float s = 0.f;
-    for (long r = 0; r < p.R; ++r) s = fmaf(p.W_out[d * p.R + r], p.Y[t * p.R + r], s);
+    for (long r = 0; r < p.R; ++r) s = fmaf(p.W_out[d * p.R + r], p.Y[r * p.Tp + t], s);
     p.out[i] = p.x[i] + s;
 }
 
+// Tokens of an output workgroup, and the ranks up to which it forms Y itself:
+// its ranks' sums come one after the other, which from 16 ranks on costs more
+// than a launch. D 256, N 16, whole call (us), Y here / in m3_readout: T 2048 R8
+// 54.7 / 57.1, R16 80.8 / 78.3, R24 106.8 / 99.9, R64 241 / 214; T 65536 R12
+// 312 / 321, R32 829 / 776.
+constexpr int kM3OutT = 16, kM3OutR = 16;
+// The token group of a workgroup: the grid's y, and z past its 65535.
+__device__ __forceinline__ long m3_out_t0() {
+    return (static_cast<long>(blockIdx.z) * gridDim.y + blockIdx.y) * kM3OutT;
+}
 // Both for D a multiple of 4 and 16-byte aligned x / out: a workgroup takes
 // kM3OutT tokens and up to 1024 channels. 16 threads per token form Y (each
 // the states n, n + 16, ..., then a sum over the threads through LDS), and
 // each thread then handles 4 channels of every token with 16-byte loads
-// and stores, W_out's rows read once. Bound by HBM (x read, out written).
+// and stores, W_out's rows read once for 4 tokens. Bound by HBM (x read, out written).
 // T 16384, D 1024: 20.7 us (6.2 TB/s; a workgroup per token, after a readout
 // kernel of its own, took 22.9 + 5.9 us).
-constexpr int kM3OutT = 16, kM3OutR = 64;
 __global__ void __launch_bounds__(256) m3_out4(M3Args p) {
     __shared__ float ys[kM3OutT][kM3OutR];
     __shared__ float part[16][kM3OutT + 1];
     const int tid = threadIdx.x, tt = tid & 15, ln = tid >> 4;
-    const long t0 = static_cast<long>(blockIdx.y) * kM3OutT;
+    const long t0 = m3_out_t0();
+    if (t0 >= p.T) return;
     const int nt = static_cast<int>(std::min<long>(kM3OutT, p.T - t0));
     const long q = static_cast<long>(blockIdx.x) * 256 + tid;
     const bool on = 4 * q < p.D;
@@ -519,6 +531,48 @@ __global__ void __launch_bounds__(256) m3_out4(M3Args p) {
         for (int u = 0; u < AH; ++u)
             if (u0 + u < nt) *reinterpret_cast<float4 *>(p.out + i0 + (u0 + u) * p.D) = v[u];
     }
+}
+
+// The output alone, Y from m3_readout. A thread keeps its 4 channels of
+// the kM3OutT tokens, so W_out's rows are read once; Y comes through LDS,
+// kM3YR ranks at a time.
+constexpr int kM3YR = 64;
+__global__ void __launch_bounds__(256) m3_out4_y(M3Args p) {
+    __shared__ float ys[kM3YR][kM3OutT];
+    const int tid = threadIdx.x;
+    const long t0 = m3_out_t0();
+    if (t0 >= p.T) return;
+    const int nt = static_cast<int>(std::min<long>(kM3OutT, p.T - t0));
+    const long q = static_cast<long>(blockIdx.x) * 256 + tid;
+    const bool on = 4 * q < p.D;
+    const int R = static_cast<int>(p.R);
+    const long q0 = on ? 4 * q : 0, i0 = t0 * p.D + q0;
+    float4 v[kM3OutT];
+#pragma unroll
+    for (int u = 0; u < kM3OutT; ++u) v[u] = *reinterpret_cast<const float4 *>(p.x + i0 + std::min(u, nt - 1) * p.D);
+    for (int r0 = 0; r0 < R; r0 += kM3YR) {
+        const int nr = std::min(kM3YR, R - r0);
+        __syncthreads();
+        // (Y's rows hold whole groups of tokens: Tp is a multiple of 64.)
+        for (int e = tid; e < nr * kM3OutT; e += 256)
+            ys[e / kM3OutT][e % kM3OutT] = p.Y[(r0 + e / kM3OutT) * p.Tp + t0 + e % kM3OutT];
+        __syncthreads();
+        const float *w = p.W_out + q0 * R + r0;
+        for (int r = 0; r < nr; ++r) {
+            const float w0 = w[r], w1 = w[R + r], w2 = w[2 * R + r], w3 = w[3 * R + r];
+#pragma unroll
+            for (int u = 0; u < kM3OutT; ++u) {
+                const float y = ys[r][u];
+                v[u].x = fmaf(w0, y, v[u].x);
+                v[u].y = fmaf(w1, y, v[u].y);
+                v[u].z = fmaf(w2, y, v[u].z);
+                v[u].w = fmaf(w3, y, v[u].w);
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kM3OutT; ++u)
+        if (on && u < nt) *reinterpret_cast<float4 *>(p.out + i0 + u * p.D) = v[u];
 }
 
 // The parameters, packed in pinned host memory, to the device: the CUs read
@@ -599,13 +653,16 @@ int mamba3_launch(M3Args &a, hipStream_t s) {
         else      hipLaunchKernelGGL((m3_scan<false, false>), gs, bs, 0, s, a, npairs);
     }
     const bool al16 = ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
-    const long gt = (a.T + kM3OutT - 1) / kM3OutT;
-    if (a.D % 4 == 0 && al16 && a.R <= kM3OutR && gt <= 65535) {
-        const dim3 go(static_cast<unsigned>(grid256(a.D / 4)), static_cast<unsigned>(gt));
+    const long gt = (a.T + kM3OutT - 1) / kM3OutT, gy = std::min<long>(gt, 65535);
+    const dim3 go(static_cast<unsigned>(grid256(a.D / 4)), static_cast<unsigned>(gy),
+                  static_cast<unsigned>((gt + gy - 1) / gy));
+    const bool wide = a.D % 4 == 0 && al16;
+    if (wide && a.R <= kM3OutR) {
         hipLaunchKernelGGL(m3_out4, go, dim3(256), 0, s, a);
     } else {
-        hipLaunchKernelGGL(m3_readout, dim3(grid256(a.T * a.R)), dim3(256), 0, s, a);
-        hipLaunchKernelGGL(m3_out, dim3(grid256(a.T * a.D)), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(m3_readout, dim3(static_cast<unsigned>(grid256(a.Tp * a.R))), dim3(256), 0, s, a);
+        if (wide) hipLaunchKernelGGL(m3_out4_y, go, dim3(256), 0, s, a);
+        else      hipLaunchKernelGGL(m3_out, dim3(grid256(a.T * a.D)), dim3(256), 0, s, a);
     }
     KM_HIP_TRY(hipGetLastError());
     return 0;
@@ -739,7 +796,7 @@ void mamba_block_forward(MambaBlock *b, float *output, const float *input, size_
     do {
         const size_t io_bytes = dev_io ? 0 : 2 * km::align_up(sizeof(float) * T * D, 256);
         const size_t bytes = io_bytes + sizeof(float) * (J * D + D * R + N + 2 * NR + TS) + 8 * 256 +
-                             sizeof(float) * (Tp * J + (prep ? 3 : 1) * Tp * N + T * R) + 8 * 256;
+                             sizeof(float) * (Tp * J + (prep ? 3 : 1) * Tp * N + Tp * R) + 8 * 256;
         void *base = km::Staging::reserve(bytes);
         if (!base) break;
         km::Carver cv(base);
@@ -795,7 +852,7 @@ void mamba_block_forward(MambaBlock *b, float *output, const float *input, size_
             a.c = cv.take<float>(Tp * N);
         }
         a.Tp = Tp;
-        a.Y = cv.take<float>(T * R);
+        a.Y = cv.take<float>(Tp * R);
         a.T = T; a.L = L; a.D = D; a.N = N; a.R = R; a.J = J;
         a.has_delta = has_delta; a.has_lambda = has_lambda;
         a.dt_scale = c.dt_scale; a.dt_min = c.dt_min; a.dt_max = c.dt_max;

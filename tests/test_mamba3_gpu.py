@@ -210,7 +210,12 @@ def test_kmamba_checkpoint_roundtrip_forward(tmp_path):
                                              (520, 5, 4, 4, 1),
                                              # In the scan: one whole super-chunk; several on workgroups that
                                              # fill the chip.
-                                             (1, 2048, 32, 16, 1), (32, 2500, 4, 16, 2)])
+                                             (1, 2048, 32, 16, 1), (32, 2500, 4, 16, 2),
+                                             # Ranks on both sides of the readout's own kernel and past its
+                                             # LDS rows, whole 16-byte rows and not; more tokens than 65535
+                                             # groups of 16.
+                                             (1, 19, 8, 4, 16), (3, 21, 1032, 3, 17), (1, 50, 12, 2, 64),
+                                             (2, 16, 4, 3, 65), (2, 33, 10, 5, 17), (131075, 8, 4, 2, 1)])
 def test_block_tile_edges(batch, L, dim, N, R):
     p = mamba3_params(dim, N, R)
     x = rng_for("m3-edges", batch, L, dim, N, R).standard_normal((batch, L, dim)).astype(np.float32)
