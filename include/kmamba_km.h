@@ -116,8 +116,10 @@ int km_scan1d_fwd(const KMScan1DFwd *a, void *stream);
  *                 NULL for the library's scratch of this (device, stream).
  *                 It holds per-workgroup partial sums (dA and, with shared
  *                 B/C, dB/dC per channel group; the group width depends on
- *                 the kernel the shape runs on) and, when neither h_hist
- *                 nor h_ckpt is given, the recomputed checkpoints.
+ *                 the kernel the shape runs on), when neither h_hist nor
+ *                 h_ckpt is given the recomputed checkpoints, and the scratch
+ *                 of sequences split over workgroups, without which (a
+ *                 workspace smaller by that part) the call runs unsplit.
  * dA (summed over batch and time) and the shared dB/dC (summed over
  * channels) are formed from those partials in a fixed order, with no
  * atomics: every output is identical run to run. */
@@ -202,8 +204,11 @@ int km_gemm_bf16(const KMGemm *g, void *stream);
  * be NULL), dt_bias [di], A [di, N], Dskip [di] (may be NULL) fp32.
  * clamp: the +-1000 state clamp of the reference scan (1) or none (0).
  * workspace: km_mamba1_block_workspace_bytes() bytes of device memory, or
- * NULL for the library's scratch of this (device, stream). Every projection
- * runs on km_gemm_bf16's bf16 MFMA kernels. */
+ * NULL for the library's scratch of this (device, stream). It holds the
+ * activations and the scratch of a scan split over workgroups; where it holds
+ * the activations only, the scan runs unsplit or, when L is a multiple of 64,
+ * takes the library's scratch. Every projection runs on km_gemm_bf16's bf16
+ * MFMA kernels. */
 typedef struct {
     long dim, d_inner, d_state, d_conv, dt_rank;
     const void  *W_in;

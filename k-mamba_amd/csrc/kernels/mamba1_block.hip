@@ -20,7 +20,9 @@
 
 namespace km {
 
-int scan1d_fwd_launch(const KMScan1DFwd *k, hipStream_t stream, bool allow_split);
+int scan1d_fwd_launch(const KMScan1DFwd *k, hipStream_t stream, bool allow_split,
+                      const GivenScratch *given = nullptr);
+size_t scan1d_fwd_scratch(const KMScan1DFwd *k);
 int gemm_bf16_launch(const KMGemm *g, hipStream_t s);
 int gemm_bf16_launch_split(const KMGemm *g, void *C2, long nsplit, hipStream_t s);
 
@@ -83,7 +85,19 @@ __global__ void __launch_bounds__(256) conv1d_silu_bf16(const uint32_t *x, const
 
 struct BlockLayout {
     size_t xi, z, u, xdbl, delta, y, bytes;
+    size_t split_bytes;   // past bytes: the scan's scratch, which it can do without
 };
+
+// The block's scan, on its activations.
+static KMScan1DFwd block_scan(const KMMamba1Weights *w, long B, long L) {
+    const long NX = w->dt_rank + 2 * w->d_state;
+    KMScan1DFwd k{};
+    k.A = w->A; k.Dskip = w->Dskip;
+    k.B = B; k.L = L; k.D = w->d_inner; k.N = w->d_state;
+    k.bc_sb = L * NX; k.bc_st = NX; k.bc_sd = 0;
+    k.dtype = KM_BF16; k.clamp = w->clamp;
+    return k;
+}
 
 static BlockLayout block_layout(const KMMamba1Weights *w, long B, long L) {
     BlockLayout l{};
@@ -97,6 +111,8 @@ static BlockLayout block_layout(const KMMamba1Weights *w, long B, long L) {
     l.y = off; off += act;
     l.xdbl = off; off += align_up(T * (w->dt_rank + 2 * w->d_state) * 2, 256);
     l.bytes = off;
+    const KMScan1DFwd k = block_scan(w, B, L);
+    l.split_bytes = scan1d_fwd_scratch(&k);
     return l;
 }
 
@@ -120,7 +136,8 @@ static bool block_ok(const KMMamba1Weights *w, const void *x, const void *out, l
 
 size_t mamba1_workspace(const KMMamba1Weights *w, long B, long L) {
     if (!w || B <= 0 || L <= 0) return 0;
-    return block_layout(w, B, L).bytes;
+    const BlockLayout l = block_layout(w, B, L);
+    return l.bytes + l.split_bytes;
 }
 
 int mamba1_block_fwd(const KMMamba1Weights *w, const void *x, void *out, long B, long L,
@@ -183,15 +200,13 @@ int mamba1_block_fwd(const KMMamba1Weights *w, const void *x, void *out, long B,
     g.lda = NX; g.ldb = R; g.ldc = di; g.bias = w->dt_bias; g.epilogue = KM_EPI_SOFTPLUS;
     if (gemm_bf16_launch(&g, s) != 0) return -1;
     // selective scan with the skip and SiLU(z) gate fused into its store
-    KMScan1DFwd k{};
-    k.x = u; k.delta = delta; k.A = w->A;
+    KMScan1DFwd k = block_scan(w, B, L);
+    k.x = u; k.delta = delta;
     k.Bm = reinterpret_cast<uint16_t *>(xdbl) + R;
     k.Cm = reinterpret_cast<uint16_t *>(xdbl) + R + N;
-    k.y = y; k.B = B; k.L = L; k.D = di; k.N = N;
-    k.bc_sb = L * NX; k.bc_st = NX; k.bc_sd = 0;
-    k.dtype = KM_BF16; k.clamp = w->clamp;
-    k.z = z; k.Dskip = w->Dskip;
-    if (scan1d_fwd_launch(&k, s, true) != 0) return -1;
+    k.y = y; k.z = z;
+    const GivenScratch given{ws + lay.bytes, workspace ? ws_bytes - lay.bytes : 0};
+    if (scan1d_fwd_launch(&k, s, true, workspace ? &given : nullptr) != 0) return -1;
     // out_proj
     KMGemm o{};
     o.A = y; o.B = w->W_out; o.C = out; o.M = T; o.N = w->dim; o.K = di;

@@ -51,7 +51,9 @@
 
 namespace km {
 
-int scan1d_fwd_launch(const KMScan1DFwd *k, hipStream_t stream, bool allow_split);
+int scan1d_fwd_launch(const KMScan1DFwd *k, hipStream_t stream, bool allow_split,
+                      const GivenScratch *given = nullptr);
+size_t scan1d_fwd_scratch(const KMScan1DFwd *k);
 
 struct Scan1DBwdArgs {
     const void *x, *dt, *dy;
@@ -1013,9 +1015,11 @@ struct BwdPlan {
     long G;                 // channel groups per batch element (partial slots)
     size_t off_slots, off_dA, off_ckpt, off_hist, bytes;
     // Split over S segments of sps super-chunks (S = 1: not split), the maps'
-    // parts per segment, and its scratch: maps, delta sums, dA partials.
+    // parts per segment, and its scratch: maps, delta sums, dA partials. The
+    // checkpoints' forward, over before, uses the same memory where the caller
+    // gave it (extra_bytes: the larger of both).
     long S, sps, parts;
-    size_t off_g, off_ds, off_dAS, seg_bytes;
+    size_t off_g, off_ds, off_dAS, seg_bytes, extra_bytes;
 };
 
 // Channels per workgroup of the register-blocked backward for a state size.
@@ -1089,6 +1093,18 @@ static void bwd_segments(const KMScan1DBwd *k, BwdPlan &pl) {
     if (pl.S > 1) pl.parts = map_parts(k->B, k->D, pl.S - 1, pl.sps * kCkptSteps);
 }
 
+// The forward that finds the states again from the same inputs (y not written).
+static KMScan1DFwd bwd_states_args(const KMScan1DBwd *k, float *ckpt, float *hist) {
+    KMScan1DFwd f{};
+    f.x = k->x; f.delta = k->delta; f.A = k->A; f.Bm = k->Bm; f.Cm = k->Cm; f.y = nullptr;
+    f.h0 = k->h0; f.B = k->B; f.L = k->L; f.D = k->D; f.N = k->N;
+    f.bc_sb = k->bc_sb; f.bc_st = k->bc_st; f.bc_sd = k->bc_sd;
+    f.dtype = k->dtype; f.clamp = k->clamp;
+    f.h_ckpt = ckpt;
+    f.h_hist = hist;
+    return f;
+}
+
 static BwdPlan bwd_plan(const KMScan1DBwd *k) {
     BwdPlan pl{};
     pl.shared = (k->bc_sd == 0);
@@ -1123,6 +1139,11 @@ static BwdPlan bwd_plan(const KMScan1DBwd *k) {
         pl.off_ds = align_up(sizeof(float) * nst * nmap, 256);
         pl.off_dAS = pl.off_ds + align_up(sizeof(float) * k->B * k->D * nmap, 256);
         pl.seg_bytes = pl.off_dAS + align_up(sizeof(float) * nst * pl.S, 256);
+    }
+    pl.extra_bytes = pl.seg_bytes;
+    if (pl.need_ckpt) {
+        const KMScan1DFwd f = bwd_states_args(k, nullptr, nullptr);   // (the outputs' addresses play no part)
+        pl.extra_bytes = std::max(pl.extra_bytes, scan1d_fwd_scratch(&f));
     }
     return pl;
 }
@@ -1217,7 +1238,7 @@ static int scan1d_bwd_run(const KMScan1DBwd *k, const BwdPlan &pl, bool bf, hipS
 size_t scan1d_bwd_workspace(const KMScan1DBwd *k) {
     if (!bwd_args_ok(k, "km_scan1d_bwd_workspace_bytes")) return 0;
     const BwdPlan pl = bwd_plan(k);
-    return pl.bytes + pl.seg_bytes;
+    return pl.bytes + pl.extra_bytes;
 }
 
 int scan1d_bwd_launch(const KMScan1DBwd *k, hipStream_t stream) {
@@ -1231,6 +1252,7 @@ int scan1d_bwd_launch(const KMScan1DBwd *k, hipStream_t stream) {
 
 static int scan1d_bwd_run(const KMScan1DBwd *k, const BwdPlan &pl, bool bf, hipStream_t stream) {
     char *ws = nullptr, *seg_ws = nullptr;
+    GivenScratch given{nullptr, 0};
     if (pl.bytes > 0) {
         if (k->workspace) {
             if (k->workspace_bytes < pl.bytes) {
@@ -1239,7 +1261,8 @@ static int scan1d_bwd_run(const KMScan1DBwd *k, const BwdPlan &pl, bool bf, hipS
                 return -1;
             }
             ws = static_cast<char *>(k->workspace);
-            if (pl.seg_bytes > 0 && k->workspace_bytes >= pl.bytes + pl.seg_bytes) seg_ws = ws + pl.bytes;
+            given = GivenScratch{ws + pl.bytes, k->workspace_bytes - pl.bytes};
+            if (pl.seg_bytes > 0 && given.bytes >= pl.seg_bytes) seg_ws = ws + pl.bytes;
         } else {
             ws = static_cast<char *>(Workspace::reserve(pl.bytes, stream, WsUse::Scan1DBwd));
             if (!ws) return -1;
@@ -1266,20 +1289,12 @@ static int scan1d_bwd_run(const KMScan1DBwd *k, const BwdPlan &pl, bool bf, hipS
     a.dApart = reinterpret_cast<float *>(split ? seg_ws + pl.off_dAS : ws + pl.off_dA);
     if (pl.shared) a.slot = reinterpret_cast<float *>(ws + pl.off_slots);
     if (pl.need_ckpt || pl.need_hist) {
-        // Forward states from the same inputs (y not written).
-        KMScan1DFwd f{};
-        f.x = k->x; f.delta = k->delta; f.A = k->A; f.Bm = k->Bm; f.Cm = k->Cm; f.y = nullptr;
-        f.h0 = k->h0; f.B = k->B; f.L = k->L; f.D = k->D; f.N = k->N;
-        f.bc_sb = k->bc_sb; f.bc_st = k->bc_st; f.bc_sd = k->bc_sd;
-        f.dtype = k->dtype; f.clamp = k->clamp;
-        if (pl.need_ckpt) {
-            f.h_ckpt = reinterpret_cast<float *>(ws + pl.off_ckpt);
-            a.ckpt = f.h_ckpt;
-        } else {
-            f.h_hist = reinterpret_cast<float *>(ws + pl.off_hist);
-            a.hist = f.h_hist;
-        }
-        if (scan1d_fwd_launch(&f, stream, true) != 0) return -1;
+        float *const ckpt = pl.need_ckpt ? reinterpret_cast<float *>(ws + pl.off_ckpt) : nullptr;
+        float *const hist = pl.need_ckpt ? nullptr : reinterpret_cast<float *>(ws + pl.off_hist);
+        const KMScan1DFwd f = bwd_states_args(k, ckpt, hist);
+        if (pl.need_ckpt) a.ckpt = ckpt;
+        else a.hist = hist;
+        if (scan1d_fwd_launch(&f, stream, true, k->workspace ? &given : nullptr) != 0) return -1;
     }
     if (split) {
         // Adjoint maps of the parts after the first segment.

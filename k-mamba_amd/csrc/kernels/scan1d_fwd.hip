@@ -748,30 +748,50 @@ static bool split_always(const KMScan1DFwd *k) {
 // threads enqueue on it (they share the stream's scratch block).
 static std::mutex g_split_mu;
 
-// Segment workgroups have the unsplit kernel's shape: 8 waves of 8 steps
-// (64-step super-chunks). Returns 1 when the scratch is not to be had and
-// the call can run unsplit.
-template <typename T>
-static int launch_segmented(const KMScan1DFwd *k, const Scan1DFwdArgs &base, long Ls, hipStream_t s) {
-    constexpr int NPL = 8, NS = 2, DL = 32, WS = 8;
-    const long S = (k->L + Ls - 1) / Ls;
-    const long groups = (k->D + DL - 1) / DL;
-    const long r = map_parts(k->B, k->D, S - 1, Ls), nmap = (S - 1) * r;
-    const long grid = k->B * S * groups;
+// A split into S segments of Ls steps (r maps each, nmap in all) and its
+// scratch: maps, delta sums, clamp flags and, where h_final shares h0's memory,
+// a copy of h0.
+struct SplitPlan {
+    long S, groups, r, nmap;
+    size_t st, sd, sf, bytes;
+    bool alias;
+};
+static SplitPlan split_plan(const KMScan1DFwd *k, long Ls) {
+    SplitPlan q{};
+    q.S = (k->L + Ls - 1) / Ls;
+    q.groups = (k->D + 31) / 32;
+    q.r = map_parts(k->B, k->D, q.S - 1, Ls);
+    q.nmap = (q.S - 1) * q.r;
     const size_t nst = static_cast<size_t>(k->B) * k->D * k->N;
-    const size_t st = align_up(sizeof(float) * nst * nmap, 256);
-    const size_t sd = align_up(sizeof(float) * k->B * k->D * nmap, 256);
-    const size_t sf = align_up(4 * k->B * groups, 256);
+    q.st = align_up(sizeof(float) * nst * q.nmap, 256);
+    q.sd = align_up(sizeof(float) * k->B * k->D * q.nmap, 256);
+    q.sf = align_up(4 * k->B * q.groups, 256);
     const char *h0b = reinterpret_cast<const char *>(k->h0), *hfb = reinterpret_cast<const char *>(k->h_final);
-    const bool alias = h0b && hfb && h0b < hfb + 4 * nst && hfb < h0b + 4 * nst;
-    const size_t bytes = st + sd + sf + (alias ? align_up(4 * nst, 256) : 0);
+    q.alias = h0b && hfb && h0b < hfb + 4 * nst && hfb < h0b + 4 * nst;
+    q.bytes = q.st + q.sd + q.sf + (q.alias ? align_up(4 * nst, 256) : 0);
+    return q;
+}
+
+// Segment workgroups have the unsplit kernel's shape: 8 waves of 8 steps
+// (64-step super-chunks) on 32 channels. Returns 1 when the scratch is not to
+// be had and the call can run unsplit.
+template <typename T>
+static int launch_segmented(const KMScan1DFwd *k, const Scan1DFwdArgs &base, long Ls, hipStream_t s,
+                            const GivenScratch *given) {
+    constexpr int NPL = 8, NS = 2, WS = 8;
+    const SplitPlan pl = split_plan(k, Ls);
+    const long S = pl.S, groups = pl.groups, r = pl.r, nmap = pl.nmap, grid = k->B * S * groups;
+    const size_t st = pl.st, sd = pl.sd, sf = pl.sf;
+    const bool alias = pl.alias;
     std::lock_guard<std::mutex> guard(g_split_mu);
     char *ws;
-    if (split_always(k)) {
-        ws = static_cast<char *>(Workspace::reserve(bytes, s, WsUse::Scan1DSplit));
+    if (given && given->ptr && given->bytes >= pl.bytes) {
+        ws = static_cast<char *>(given->ptr);
+    } else if (split_always(k)) {
+        ws = static_cast<char *>(Workspace::reserve(pl.bytes, s, WsUse::Scan1DSplit));
         if (!ws) return -1;
     } else {
-        ws = static_cast<char *>(Workspace::try_reserve(bytes, s, WsUse::Scan1DSegments));
+        ws = given ? nullptr : static_cast<char *>(Workspace::try_reserve(pl.bytes, s, WsUse::Scan1DSegments));
         if (!ws) return 1;
     }
     const bool shared = (k->bc_sd == 0), hist = (k->h_hist != nullptr);
@@ -836,9 +856,24 @@ static int launch_serial(const Scan1DFwdArgs &a, bool hist, hipStream_t s) {
     return 0;
 }
 
+// The register-blocked kernel addresses each batch element's windows with
+// 32-bit byte offsets; larger problems take the sequential kernel.
+static bool small_windows(const KMScan1DFwd *k) {
+    const long es = (k->dtype == KM_BF16) ? 2 : 4;
+    const long lim = 0x3fffffffL;   // offsets reach (L + W*TC) rows
+    return k->L * k->D * es < lim && k->L * k->bc_st * es < lim &&
+           (!k->h_hist || k->L * k->D * k->N * 4 < lim) && k->bc_st >= 0 && k->bc_sd >= 0 && k->bc_sb >= 0;
+}
+
+// Scratch with which the call is split (0: it is not).
+size_t scan1d_fwd_scratch(const KMScan1DFwd *k) {
+    const long Ls = small_windows(k) ? segment_length(k, k->B * ((k->D + 31) / 32)) : 0;
+    return Ls ? split_plan(k, Ls).bytes : 0;
+}
+
 // allow_split = false keeps every shape on kernels that use no workspace
 // (the allocation-free ScanND entry point's 1D grids).
-int scan1d_fwd_launch(const KMScan1DFwd *k, hipStream_t stream, bool allow_split) {
+int scan1d_fwd_launch(const KMScan1DFwd *k, hipStream_t stream, bool allow_split, const GivenScratch *given) {
     if (!k) { set_error("km_scan1d_fwd: NULL arguments"); return -1; }
     // With no steps (L = 0) only A, h0 and h_final take part.
     if (!k->A || (k->L > 0 && (!k->x || !k->delta || !k->Bm || !k->Cm))) {
@@ -871,22 +906,16 @@ int scan1d_fwd_launch(const KMScan1DFwd *k, hipStream_t stream, bool allow_split
                     k->h_ckpt, (k->L + kCkptSteps - 1) / kCkptSteps, k->z, k->Dskip,
                     k->B, k->L, k->D, k->N, k->bc_sb, k->bc_st, k->bc_sd, k->clamp, 1,
                     static_cast<int>(std::min<long>(k->L, 0x7fffffffL)), nullptr, nullptr, nullptr, 0, 0};
-    // The register-blocked kernel addresses each batch element's windows with
-    // 32-bit byte offsets; larger problems take the sequential kernel.
-    const long es = (k->dtype == KM_BF16) ? 2 : 4;
-    const long lim = 0x3fffffffL;   // offsets reach (L + W*TC) rows
-    const bool small_windows = k->L * k->D * es < lim && k->L * k->bc_st * es < lim &&
-                               (!k->h_hist || k->L * k->D * k->N * 4 < lim) &&
-                               k->bc_st >= 0 && k->bc_sd >= 0 && k->bc_sb >= 0;
     const bool shared = (k->bc_sd == 0);
     const bool hist = (k->h_hist != nullptr);
     const bool bf = (k->dtype == KM_BF16);
-    if (!small_windows)
+    if (!small_windows(k))
         return bf ? launch_serial<bf16_t>(a, hist, stream) : launch_serial<f32_t>(a, hist, stream);
     // Few (batch, channel group) pairs and a long sequence: split the
     // sequence over workgroups.
     if (const long Ls = allow_split ? segment_length(k, k->B * ((k->D + 31) / 32)) : 0) {
-        const int rc = bf ? launch_segmented<bf16_t>(k, a, Ls, stream) : launch_segmented<f32_t>(k, a, Ls, stream);
+        const int rc = bf ? launch_segmented<bf16_t>(k, a, Ls, stream, given)
+                          : launch_segmented<f32_t>(k, a, Ls, stream, given);
         if (rc <= 0) return rc;
     }
     switch (k->N) {
@@ -919,7 +948,7 @@ extern "C" {
 
 int km_scan1d_fwd(const KMScan1DFwd *a, void *stream) {
     km::clear_error();
-    return km::scan1d_fwd_launch(a, static_cast<hipStream_t>(stream), true);
+    return km::scan1d_fwd_launch(a, static_cast<hipStream_t>(stream), true, nullptr);
 }
 
 // Reference cuda/scan1d.cu:258-310: B, C, h are [L, D, M]; h receives the
@@ -937,7 +966,7 @@ void om_scan1d_forward(const float *d_x, const float *d_A, const float *d_B, con
     a.B = 1; a.L = L; a.D = D; a.N = M;
     a.bc_sb = static_cast<long>(L) * D * M; a.bc_st = static_cast<long>(D) * M; a.bc_sd = M;
     a.dtype = KM_F32; a.clamp = 1;
-    if (km::scan1d_fwd_launch(&a, nullptr, true) != 0) return;
+    if (km::scan1d_fwd_launch(&a, nullptr, true, nullptr) != 0) return;
     if (hipStreamSynchronize(nullptr) != hipSuccess)
         km::set_error("om_scan1d_forward: %s", hipGetErrorString(hipGetLastError()));
 }
@@ -971,7 +1000,7 @@ void scan1d(ScanParams *p) {
     if (dev) {
         a.x = p->x; a.delta = p->delta; a.A = p->A; a.Bm = p->B; a.Cm = p->C; a.y = p->y;
         a.h0 = p->h; a.h_final = p->h;
-        if (km::scan1d_fwd_launch(&a, nullptr, true) == 0 && hipStreamSynchronize(nullptr) != hipSuccess)
+        if (km::scan1d_fwd_launch(&a, nullptr, true, nullptr) == 0 && hipStreamSynchronize(nullptr) != hipSuccess)
             km::set_error("scan1d: %s", hipGetErrorString(hipGetLastError()));
         return;
     }
@@ -993,7 +1022,7 @@ void scan1d(ScanParams *p) {
             km::set_error("scan1d: host-to-device copy failed");
         } else {
             a.x = x; a.delta = dt; a.A = A; a.Bm = Bm; a.Cm = Cm; a.y = y; a.h0 = h; a.h_final = h;
-            if (km::scan1d_fwd_launch(&a, nullptr, true) == 0) {
+            if (km::scan1d_fwd_launch(&a, nullptr, true, nullptr) == 0) {
                 if (km::copy_d2h(p->y, y, nLD * 4) != hipSuccess ||
                     km::copy_d2h(p->h, h, nDM * 4) != hipSuccess)
                     km::set_error("scan1d: device-to-host copy failed");

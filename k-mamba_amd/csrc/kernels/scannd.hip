@@ -45,7 +45,8 @@
 
 namespace km {
 
-int scan1d_fwd_launch(const KMScan1DFwd *k, hipStream_t stream, bool allow_split);
+int scan1d_fwd_launch(const KMScan1DFwd *k, hipStream_t stream, bool allow_split,
+                      const GivenScratch *given = nullptr);
 
 constexpr int kMaxNd = 8;
 

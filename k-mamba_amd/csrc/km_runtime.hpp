@@ -89,6 +89,14 @@ struct Workspace {
     static void *find(hipStream_t stream, WsUse use);
 };
 
+// Memory that an entry point was given and passes on to a launch that it
+// makes: the launch then takes its scratch there, if it fits, and not from the
+// library.
+struct GivenScratch {
+    void *ptr;
+    size_t bytes;
+};
+
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // Copies between pageable host memory and device memory through a ring of

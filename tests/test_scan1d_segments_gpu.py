@@ -244,3 +244,58 @@ def test_growing_decays_backward_of_masked_loss(L, kind, mode):
             assert_close(a, r, TOL_F32, n, np.abs(k))
         else:                                   # mixed signs of A: per tensor
             assert np.abs(a - r).max() <= TOL_F32 * np.abs(r).max(), n
+
+
+# --- scratch in the caller's workspace ------------------------------------------------
+
+def test_backward_with_workspace_takes_no_scratch():
+    # Without checkpoints the backward runs the forward first: split or not, a
+    # call that was given its workspace allocates nothing.
+    Bsz, L, D = 1, 1001, 64
+    x, dt, A, Bm, Cm = (T(a) for a in scan1d_inputs(Bsz, L, D, N, seed=61))
+    dy = T(rng_for("ws", L).standard_normal((Bsz, L, D)).astype(np.float32))
+    outs = [[torch.full_like(t, float("nan")) for t in (x, dt, A, Bm, Cm)] for _ in range(2)]
+    args = K.scan1d_bwd_args(x, dt, A, Bm, Cm, dy, *outs[0])
+    ws = torch.empty(K.km_scan1d_bwd_workspace_bytes(C.byref(args)), dtype=torch.uint8, device=DEV)
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    held = K.km_device_bytes_held()
+    K.scan1d_bwd(x, dt, A, Bm, Cm, dy, *outs[0], workspace=ws, stream=s)
+    s.synchronize()
+    assert K.km_device_bytes_held() == held
+    K.scan1d_bwd(x, dt, A, Bm, Cm, dy, *outs[1])          # the library's scratch: the same bits
+    torch.cuda.synchronize()
+    for a, b in zip(*outs):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("whole", [True, False])
+def test_mamba1_block_with_workspace_takes_no_scratch(whole):
+    # A workspace of the queried size, and one that holds the activations only.
+    Bsz, L, dim, R = 1, 1001, 64, 8
+    di = 2 * dim
+    g = torch.Generator().manual_seed(62)
+    rn = lambda *s, std=0.1: (torch.randn(s, generator=g) * std).to(DEV)   # noqa: E731
+    bf = torch.bfloat16
+    w = {"W_in": rn(2 * di, dim).to(bf), "conv_w": rn(4, di, std=0.5), "conv_b": rn(di),
+         "W_x": rn(R + 2 * N, di).to(bf), "W_dt": rn(di, R).to(bf), "dt_bias": rn(di) - 1,
+         "A": -torch.arange(1, N + 1, device=DEV, dtype=torch.float32).repeat(di, 1).contiguous(),
+         "Dskip": rn(di), "W_out": rn(dim, di).to(bf)}
+    x = rn(Bsz, L, dim, std=1.0).to(bf)
+    up = lambda v: (v + 255) // 256 * 256   # noqa: E731
+    nb = 5 * up(Bsz * L * di * 2) + up(Bsz * L * (R + 2 * N) * 2)
+    st = K.mamba1_weights(w)
+    if whole:
+        nb = K.km_mamba1_block_workspace_bytes(C.byref(st), Bsz, L)
+    ws = torch.empty(nb, dtype=torch.uint8, device=DEV)
+    out, want = torch.empty_like(x), torch.empty_like(x)
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    held = K.km_device_bytes_held()
+    K.mamba1_block_fwd(w, x, out, workspace=ws, stream=s)
+    s.synchronize()
+    assert K.km_device_bytes_held() == held
+    K.mamba1_block_fwd(w, x, want)
+    torch.cuda.synchronize()
+    # Split or not: the scan's fp32 sums in another order, rounded to bf16 once.
+    assert (out.float() - want.float()).norm() <= (1e-6 if whole else 4e-3) * want.float().norm()
