@@ -213,10 +213,11 @@ void ws_drop(int i) {
     }
     g_ws[i] = g_ws[--g_ws_n];
 }
-}  // namespace
 
-void *Workspace::reserve(size_t bytes, hipStream_t stream, WsUse use, bool *fresh, size_t *got) {
-    std::lock_guard<std::mutex> guard(g_ws_mu);
+// The block of (device, stream, use) with room for bytes, under g_ws_mu. With
+// `optional` another block is never dropped and a block that cannot grow stays
+// as it is. A failed allocation leaves no entry behind.
+void *ws_reserve(size_t bytes, hipStream_t stream, WsUse use, bool *fresh, size_t *got, bool optional) {
     if (fresh) *fresh = false;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0) {
@@ -231,7 +232,7 @@ void *Workspace::reserve(size_t bytes, hipStream_t stream, WsUse use, bool *fres
             // Evict the least recently used block of another (device, stream):
             // blocks of this stream may be in use by the calling entry point.
             int lru = -1;
-            for (int i = 0; i < g_ws_n; ++i)
+            for (int i = 0; i < g_ws_n && !optional; ++i)
                 if (!(g_ws[i].dev == dev && g_ws[i].stream == stream) &&
                     (lru < 0 || g_ws[i].last < g_ws[lru].last))
                     lru = i;
@@ -250,24 +251,35 @@ void *Workspace::reserve(size_t bytes, hipStream_t stream, WsUse use, bool *fres
         if (got) *got = e->size;
         return e->ptr;
     }
-    if (e->ptr) {
+    void *old = e->ptr;
+    if (old && !optional) {
         (void)hipStreamSynchronize(stream);   // earlier kernels on this stream may use the old block
-        (void)hipFree(e->ptr);
-        e->ptr = nullptr;
-        e->size = 0;
+        (void)hipFree(old);
+        old = nullptr;
     }
     const size_t want = align_up(bytes > 0 ? bytes : 1, size_t(1) << 20);
     void *p = nullptr;
     if (hipMalloc(&p, want) != hipSuccess) {
         (void)hipGetLastError();
         set_error("workspace: hipMalloc(%zu) failed", want);
+        if (!old) *e = g_ws[--g_ws_n];
         return nullptr;
+    }
+    if (old) {
+        (void)hipStreamSynchronize(stream);
+        (void)hipFree(old);
     }
     e->ptr = p;
     e->size = want;
     if (fresh) *fresh = true;
     if (got) *got = want;
     return p;
+}
+}  // namespace
+
+void *Workspace::reserve(size_t bytes, hipStream_t stream, WsUse use, bool *fresh, size_t *got) {
+    std::lock_guard<std::mutex> guard(g_ws_mu);
+    return ws_reserve(bytes, stream, use, fresh, got, false);
 }
 
 void *Workspace::try_reserve(size_t bytes, hipStream_t stream, WsUse use) {
@@ -278,22 +290,17 @@ void *Workspace::try_reserve(size_t bytes, hipStream_t stream, WsUse use) {
         return nullptr;
     }
     if (cap != hipStreamCaptureStatusNone) return nullptr;
-    {
-        std::lock_guard<std::mutex> guard(g_ws_mu);
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || dev < 0) return nullptr;
-        bool have = false;
-        for (int i = 0; i < g_ws_n; ++i)
-            have = have || (g_ws[i].dev == dev && g_ws[i].stream == stream && g_ws[i].use == use);
-        if (!have && g_ws_n == kMaxWs) return nullptr;
-    }
     // An allocation must not end a capture that some other stream is in.
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
-    void *p = reserve(bytes, stream, use);
+    void *p;
+    {
+        std::lock_guard<std::mutex> guard(g_ws_mu);
+        p = ws_reserve(bytes, stream, use, nullptr, nullptr, true);
+    }
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (!p) clear_error();
     return p;

@@ -77,7 +77,8 @@ struct Workspace {
     // disturbs nothing: nullptr without an error (the caller runs without)
     // while the stream is captured, on the per-thread stream (one handle,
     // several streams), where a full table would cost another stream its
-    // block, and when the device has no room.
+    // block, and when the device has no room (a block too small for this call
+    // then stays for those it is enough for).
     static void *try_reserve(size_t bytes, hipStream_t stream, WsUse use);
     // Frees every block of (current device, stream) after draining the
     // stream. Returns the bytes freed.
