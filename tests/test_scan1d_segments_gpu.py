@@ -120,21 +120,21 @@ def _bwd(x, dt, A, Bm, Cm, dy, *, mode, strides, h0=None, hist=None, workspace=N
     return [t.cpu().numpy() for t in out], need
 
 
-# Last segments of 1, 9, 31 and 64 steps; the fourth fills the chip only with
-# 16-wave workgroups, the last leaves most of its last wave of them empty.
-BWD = [(1, 1025, 64), (2, 1001, 40), (1, 799, 200), (2, 640, 1536), (1, 1024, 33), (9, 160, 1000)]
+def _unsplit_bytes(Bsz, L, D, *, shared, wide, mode):
+    """The workspace without a split: dB/dC slots, dA partials, checkpoints."""
+    up = lambda v: -(-v // 256) * 256   # noqa: E731
+    groups = -(-D // (32 if wide else 16))
+    return (up(8 * Bsz * groups * L * N) * shared + up(4 * Bsz * D * N) +
+            up(4 * Bsz * -(-L // 32) * D * N) * (mode == "recompute"))
 
 
-@pytest.mark.parametrize("Bsz,L,D", BWD)
-@pytest.mark.parametrize("mode", ["hist", "ckpt", "recompute"])
-def test_backward_segments_vs_oracle(Bsz, L, D, mode):
+def _check_backward(Bsz, L, D, *, mode, per_channel, wide):
     x, dt, A, Bm, Cm = scan1d_inputs(Bsz, L, D, N, seed=41)
     g = rng_for("segments-bwd", Bsz, L, D)
     if D == 40:
         A = (A * g.uniform(0.02, 1.0, size=A.shape)).astype(np.float32)   # generic, slow decays
     h0 = g.standard_normal((Bsz, D, N)).astype(np.float32)
     dy = g.standard_normal((Bsz, L, D)).astype(np.float32)
-    per_channel = D in (40, 33)
     strides = (L * N, N, 0)
     if per_channel:
         strides = (L * D * N, D * N, N)
@@ -144,12 +144,33 @@ def test_backward_segments_vs_oracle(Bsz, L, D, mode):
     ref = O.scan1d_batched_backward(x, dt, A, Bm, Cm, dy, hh, **kw)
     kap = scan1d_bwd_kappa(x, dt, A, Bm, Cm, dy, h0=h0, bc_strides=strides)
     got, need = _bwd(x, dt, A, Bm, Cm, dy, mode=mode, strides=strides, h0=h0, hist=hh)
+    assert need > _unsplit_bytes(Bsz, L, D, shared=not per_channel, wide=wide, mode=mode)
     for n, a, r, k in zip(("dx", "ddelta", "dA", "dB", "dC"), got, ref, kap):
         assert_close(a, r, TOL_F32, n, k)
     # The caller's own workspace of the queried size: the same bits.
     again, _ = _bwd(x, dt, A, Bm, Cm, dy, mode=mode, strides=strides, h0=h0, hist=hh, workspace="queried")
     for a, b in zip(got, again):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+# Last segments of 1, 41, 31 and 64 steps, two of them with per-channel B/C.
+@pytest.mark.parametrize("Bsz,L,D", [(1, 1025, 64), (2, 1001, 40), (1, 799, 200), (1, 1024, 33)])
+@pytest.mark.parametrize("mode", ["hist", "ckpt", "recompute"])
+def test_backward_segments_vs_oracle(Bsz, L, D, mode):
+    _check_backward(Bsz, L, D, mode=mode, per_channel=D in (40, 33), wide=False)
+
+
+# The same on 16-wave workgroups of 32 channels: forced on small shapes, and
+# where the rule takes them (260 groups, 3 segments of 384 steps).
+@pytest.mark.parametrize("Bsz,L,D", [(1, 1025, 64), (2, 1001, 40), (1, 799, 200)])
+@pytest.mark.parametrize("mode", ["hist", "ckpt"])
+def test_backward_segments_of_32_channels(Bsz, L, D, mode, monkeypatch):
+    monkeypatch.setenv("KM_SCAN1D_BWD_WIDE", "1")
+    _check_backward(Bsz, L, D, mode=mode, per_channel=False, wide=True)
+
+
+def test_backward_segments_where_32_channels_fill_the_chip():
+    _check_backward(5, 1123, 1664, mode="ckpt", per_channel=False, wide=True)
 
 
 def test_backward_segments_clamped_states():

@@ -13,9 +13,9 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 SMALL = [((2, 2, 8), 4, 16), ((3, 5, 9), 8, 8), ((1, 4, 17), 16, 4), ((5, 1, 8), 4, 16), ((4, 7, 1), 32, 2),
-         ((9, 3, 25), 20, 16), ((7, 8, 16), 2, 32)]
+         ((9, 3, 25), 20, 16), ((7, 8, 16), 2, 32), ((7, 5, 10), 1024, 16)]
 # Fronts of more than 768 waves: pencils (one channel group per 4 channels).
-LARGE = [((9, 6, 11), 832, 16), ((7, 5, 10), 1024, 16), ((5, 12, 9), 448, 32)]
+LARGE = [((9, 6, 11), 832, 16), ((7, 6, 10), 1024, 16), ((5, 12, 9), 448, 32)]
 # 2050 bands of 4 x 4 x 8 tiles (pencils: 1), whose 4101 of 2 x 2 x 8 would not
 # fit the host's tables; 801 and 778 bands of 2 x 2 x 8 tiles, more than the
 # dataflow schedule's table holds.
