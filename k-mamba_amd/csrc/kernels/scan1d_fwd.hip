@@ -271,41 +271,49 @@ __global__ void __launch_bounds__(64 * W, OCC) scan1d_fwd_chunked(Scan1DFwdArgs 
                      (p.A[dc * N + NS * j + ns] == static_cast<float>(NS * j + ns + 1) * p.A[dc * N]);
     const bool fast = __builtin_amdgcn_readfirstlane(__syncthreads_and(structured)) != 0;
 
-    // The state entering the workgroup's steps, state j by wave j (mod W): h0
-    // or, in a segment's replay, h0 carried through the maps before it,
-    // h <- exp(A * sum delta) h + h_end, in order. The loads of kFoldRun maps
-    // are in flight together.
-    for (int j = w; j < NPL; j += W) {
-        const long hi = (b * Dm + dc) * N + NS * j + ns;
-        float run = p.h0 ? p.h0[hi] : 0.f;
-        if constexpr (SEG) {
-            if (const int nm = seg * p.map_per) {
-                constexpr int kFoldRun = 8;
-                const float a2 = p.A[dc * N + NS * j + ns] * kLog2e, first = run;
-                const long m0 = b * p.nmap * Dm + dc;
-                for (int s0 = 0; s0 < nm; s0 += kFoldRun) {
-                    float ds[kFoldRun], hv[kFoldRun];
+    // The state entering the workgroup's steps: h0 or, in a segment's replay,
+    // h0 carried through the maps before it, h <- exp(A * sum delta) h + h_end,
+    // in order, the loads of kFoldRun maps in flight together. There the 512
+    // threads are the group's 32 channels x 16 states in memory order, so that a
+    // map costs each wave two coalesced loads: by the lanes' own states, 64
+    // maps of scattered loads took 8 us of the call (B1 L4096 D32 fp32: 30.6 -> 19.6
+    // us; by 4, 8, 16 and 32 maps in flight 21.1, 19.6, 19.1, 19.5, with fewer
+    // maps, as B1 L1024 D384 with 15, 18.3, 17.8, 18.0, 19.0).
+    if constexpr (SEG) {
+        static_assert(64 * W == DL * N, "a thread per channel and state");
+        const int fc = tid / N, fn = tid % N;
+        const long fd = min(static_cast<long>(grp) * DL + fc, p.D - 1);
+        const float first = p.h0 ? p.h0[(b * Dm + fd) * N + fn] : 0.f;
+        float run = first;
+        if (const int nm = seg * p.map_per) {
+            constexpr int kFoldRun = 8;
+            const float a2 = p.A[fd * N + fn] * kLog2e;
+            const long m0 = b * p.nmap * Dm + fd;
+            for (int s0 = 0; s0 < nm; s0 += kFoldRun) {
+                float ds[kFoldRun], hv[kFoldRun];
 #pragma unroll
-                    for (int i = 0; i < kFoldRun; ++i) {
-                        const long m = m0 + static_cast<long>(min(s0 + i, nm - 1)) * Dm;
-                        ds[i] = p.seg_dsum[m];
-                        hv[i] = p.seg_h[m * N + NS * j + ns];
-                    }
-#pragma unroll
-                    for (int i = 0; i < kFoldRun; ++i)
-                        if (s0 + i < nm) run = fmaf(exp2_fast(ds[i] * a2), run, hv[i]);
+                for (int i = 0; i < kFoldRun; ++i) {
+                    const long m = m0 + static_cast<long>(min(s0 + i, nm - 1)) * Dm;
+                    ds[i] = p.seg_dsum[m];
+                    hv[i] = p.seg_h[m * N + fn];
                 }
-                if (fold_overflowed(run)) {
-                    run = first;
+#pragma unroll
+                for (int i = 0; i < kFoldRun; ++i)
+                    if (s0 + i < nm) run = fmaf(exp2_fast(ds[i] * a2), run, hv[i]);
+            }
+            if (fold_overflowed(run)) {
+                run = first;
 #pragma unroll 1
-                    for (int i = 0; i < nm; ++i) {
-                        const long m = m0 + static_cast<long>(i) * Dm;
-                        run = decay_add(p.seg_dsum[m] * a2, run, p.seg_h[m * N + NS * j + ns]);
-                    }
+                for (int i = 0; i < nm; ++i) {
+                    const long m = m0 + static_cast<long>(i) * Dm;
+                    run = decay_add(p.seg_dsum[m] * a2, run, p.seg_h[m * N + fn]);
                 }
             }
         }
-        carry[0][j][lane] = run;
+        carry[0][fn / NS][fn % NS * DL + fc] = run;
+    } else {
+        for (int j = w; j < NPL; j += W)
+            carry[0][j][lane] = p.h0 ? p.h0[(b * Dm + dc) * N + NS * j + ns] : 0.f;
     }
 
     // B/C tile of super-chunk s: element e = (step, state) at row s*SC + e/N.
