@@ -1111,7 +1111,8 @@ static BwdPlan bwd_plan(const KMScan1DBwd *k) {
     const long es = (k->dtype == KM_BF16) ? 2 : 4;
     const long lim = 0x3fffffffL;
     const bool small_windows = k->L * k->D * es < lim && k->L * k->bc_st * es < lim &&
-                               (!k->h_hist || k->L * k->D * k->N * 4 < lim);
+                               (!k->h_hist || k->L * k->D * k->N * 4 < lim) &&
+                               rows_hold_channels(k->D, k->N, k->bc_st, k->bc_sd);
     const bool chunk_n = (k->N == 16 || k->N == 8 || k->N == 4 || k->N == 2 || k->N == 1);
     pl.serial = !(small_windows && chunk_n);
     pl.hist_in = (k->h_hist != nullptr);

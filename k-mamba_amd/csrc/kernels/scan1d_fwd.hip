@@ -865,12 +865,14 @@ static int launch_serial(const Scan1DFwdArgs &a, bool hist, hipStream_t s) {
 }
 
 // The register-blocked kernel addresses each batch element's windows with
-// 32-bit byte offsets; larger problems take the sequential kernel.
+// 32-bit byte offsets; larger problems, and strides whose rows do not hold every
+// channel, take the sequential kernel.
 static bool small_windows(const KMScan1DFwd *k) {
     const long es = (k->dtype == KM_BF16) ? 2 : 4;
     const long lim = 0x3fffffffL;   // offsets reach (L + W*TC) rows
     return k->L * k->D * es < lim && k->L * k->bc_st * es < lim &&
-           (!k->h_hist || k->L * k->D * k->N * 4 < lim) && k->bc_st >= 0 && k->bc_sd >= 0 && k->bc_sb >= 0;
+           (!k->h_hist || k->L * k->D * k->N * 4 < lim) && k->bc_st >= 0 && k->bc_sd >= 0 && k->bc_sb >= 0 &&
+           rows_hold_channels(k->D, k->N, k->bc_st, k->bc_sd);
 }
 
 // Scratch with which the call is split (0: it is not).

@@ -16,6 +16,12 @@
 
 namespace km {
 
+// The windowed kernels address B / C by rows of bc_st elements and read 0 past a
+// batch element's L rows, so a row must hold every channel's states. Other
+// strides (channel-major [D, L, N], B / C constant over time) go to the
+// sequential kernels.
+inline bool rows_hold_channels(long D, long N, long st, long sd) { return (D - 1) * sd + N <= st; }
+
 // A fold of maps takes h to 2^z h + add from map to map, z the exponent of the
 // decay over the map's steps, which may be out of range by itself: with 2^z =
 // inf a state of exactly 0 (padded x, masked dy) becomes NaN, with 2^z = 0 an

@@ -13,7 +13,7 @@ import pytest
 import kmamba as K
 import oracle as O
 from kmtest import (TOL_BF16, TOL_F32, assert_close, bf16_round, rel_err, rel_err_cond, rng_for,
-                    scan1d_inputs, scan1d_kappa, silu_ref)
+                    scan1d_bwd_kappa, scan1d_inputs, scan1d_kappa, silu_ref)
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -341,3 +341,32 @@ def test_config1_bf16_full_size_sampled_parity():
     ky, kh, _ = scan1d_kappa(*args)
     assert_close(y[:, :, sel], yr, TOL_BF16, "bf16 y", ky)
     assert_close(hf[:, sel], hr, TOL_BF16, "bf16 h_final", kh)
+
+
+# B / C whose rows (bc_st) do not hold every channel: channel-major, and
+# constant over time; a single step with any row stride.
+@pytest.mark.parametrize("N", [16, 4])
+@pytest.mark.parametrize("Bsz,L,D", [(1, 70, 40), (2, 300, 33), (1, 1, 20)])
+def test_strides_whose_rows_do_not_hold_the_channels(Bsz, L, D, N):
+    x, dt, A, Bs, Cs = scan1d_inputs(Bsz, L, D, N, seed=71)
+    g = rng_for("strides", Bsz, L, D, N)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda")   # noqa: E731
+    h0 = g.standard_normal((Bsz, D, N)).astype(np.float32)
+    dy = g.standard_normal((Bsz, L, D)).astype(np.float32)
+    major = tuple((g.standard_normal((Bsz, D, L, N)) * 0.25).astype(np.float32) for _ in range(2))
+    for (Bm, Cm), st in ((major, (D * L * N, N, L * N)), ((Bs[:, :1], Cs[:, :1]), (N, 0, 0))):
+        yr, hr, hh = O.scan1d_batched(x, dt, A, Bm, Cm, h0=h0, bc_strides=st, hist=True)
+        ky, kh, _ = scan1d_kappa(x, dt, A, Bm, Cm, h0=h0, bc_strides=st)
+        ins = [dev(a) for a in (x, dt, A, Bm, Cm)]
+        y, hf = torch.empty_like(ins[0]), torch.empty((Bsz, D, N), device="cuda")
+        K.scan1d_fwd(*ins, y, h0=dev(h0), h_final=hf, bc_strides=st)
+        assert_close(y.cpu().numpy(), yr, TOL_F32, "y", ky)
+        assert_close(hf.cpu().numpy(), hr, TOL_F32, "h_final", kh)
+        if st[1] == 0 and L > 1:
+            continue                            # the backward refuses gradients that alias over time
+        ref = O.scan1d_batched_backward(x, dt, A, Bm, Cm, dy, hh, h0=h0, bc_strides=st)
+        kap = scan1d_bwd_kappa(x, dt, A, Bm, Cm, dy, h0=h0, bc_strides=st)
+        outs = [torch.full_like(ins[i], float("nan")) for i in (0, 0, 2, 3, 4)]
+        K.scan1d_bwd(*ins, dev(dy), *outs, h0=dev(h0), bc_strides=st)
+        for n, a, r, k in zip(("dx", "ddelta", "dA", "dB", "dC"), outs, ref, kap):
+            assert_close(a.cpu().numpy(), r, TOL_F32, n, k)
