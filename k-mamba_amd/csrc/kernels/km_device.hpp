@@ -193,6 +193,16 @@ template <> struct bio<f32_t> {
     static __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, int voff, int soff, float v) {
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, voff, soff, 0);
     }
+    // 16 consecutive elements, 4-byte aligned (each dword is range-checked).
+    static __device__ __forceinline__ void ld16(__amdgpu_buffer_rsrc_t r, int voff, float (&v)[16]) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            using f32x4 = float __attribute__((ext_vector_type(4)));
+            const f32x4 w = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff + 16 * q, 0, 0));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[4 * q + i] = w[i];
+        }
+    }
     // Agent-coherent load (cache policy sc1): misses the CU's L1 and reads
     // the XCD's L2, so it sees stores another CU of the same XCD completed.
     static __device__ __forceinline__ float ld_agent(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
@@ -206,6 +216,18 @@ template <> struct bio<bf16_t> {
     }
     static __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, int voff, int soff, float v) {
         __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(v), r, voff, soff, 0);
+    }
+    static __device__ __forceinline__ void ld16(__amdgpu_buffer_rsrc_t r, int voff, float (&v)[16]) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            using u32x4 = unsigned __attribute__((ext_vector_type(4)));
+            const u32x4 w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff + 16 * q, 0, 0));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                v[8 * q + 2 * i] = bf16_to_f32(static_cast<uint16_t>(w[i] & 0xffffu));
+                v[8 * q + 2 * i + 1] = bf16_to_f32(static_cast<uint16_t>(w[i] >> 16));
+            }
+        }
     }
 };
 

@@ -67,7 +67,10 @@ struct MapArgs {
 // delta and M are in flight ahead of the arithmetic; the wave's M rows go
 // through its own LDS rows, from which every lane reads the same 16 values.
 constexpr int kMapWaves = 8, kMapBlock = 8;
-template <typename T, bool SHARED, bool ADJ>
+// VEC (per-channel M, whose loads bound the pass): a lane's 16 states in 16-byte
+// loads. B1 L16384 D64 bf16, whole call: 145 us, with 16 loads of 2 bytes 250,
+// with the output kernel as the map pass 194.
+template <typename T, bool SHARED, bool ADJ, bool VEC>
 __global__ void __launch_bounds__(64 * kMapWaves, 4) scan1d_segment_map(MapArgs p) {
     using IO = bio<T>;
     constexpr int N = 16, TS = IO::size, MB = kMapBlock, W = kMapWaves, PADC = 65;
@@ -159,9 +162,13 @@ __global__ void __launch_bounds__(64 * kMapWaves, 4) scan1d_segment_map(MapArgs 
 #pragma unroll
             for (int k = 0; k < MB; ++k) {
                 float mv[N];
+                if constexpr (VEC) {
+                    IO::ld16(rM, vm + row(t + k) * rowm, mv);
+                } else {
 #pragma unroll
-                for (int n = 0; n < N; ++n)
-                    mv[n] = SHARED ? tile[k * N + n] : IO::ld(rM, vm + n * TS + row(t + k) * rowm, 0);
+                    for (int n = 0; n < N; ++n)
+                        mv[n] = SHARED ? tile[k * N + n] : IO::ld(rM, vm + n * TS + row(t + k) * rowm, 0);
+                }
                 const float u = ADJ ? xs[k] : ds[k] * xs[k];
                 dsum += ds[k];
                 float e[N];
@@ -235,8 +242,12 @@ inline long map_parts(long B, long D, long nsegs, long Ls) {
 template <typename T, bool ADJ>
 static int launch_maps(const MapArgs &m, long B, hipStream_t s) {
     const dim3 grid(static_cast<unsigned>(B * m.nmap * ((m.D + 63) / 64))), blk(64 * kMapWaves);
-    if (m.sd == 0) hipLaunchKernelGGL((scan1d_segment_map<T, true, ADJ>), grid, blk, 0, s, m);
-    else           hipLaunchKernelGGL((scan1d_segment_map<T, false, ADJ>), grid, blk, 0, s, m);
+    // The loads' dwords have to be aligned, which 4-byte elements are.
+    constexpr uintptr_t es = bio<T>::size;
+    const bool dwords = ((reinterpret_cast<uintptr_t>(m.M) | m.sb * es | m.st * es | m.sd * es) & 3) == 0;
+    if (m.sd == 0)   hipLaunchKernelGGL((scan1d_segment_map<T, true, ADJ, false>), grid, blk, 0, s, m);
+    else if (dwords) hipLaunchKernelGGL((scan1d_segment_map<T, false, ADJ, true>), grid, blk, 0, s, m);
+    else             hipLaunchKernelGGL((scan1d_segment_map<T, false, ADJ, false>), grid, blk, 0, s, m);
     KM_HIP_TRY(hipGetLastError());
     return 0;
 }

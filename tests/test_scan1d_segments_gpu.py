@@ -194,6 +194,40 @@ def test_backward_segments_clamped_states():
         assert_close(a, r, TOL_F32, n, k)
 
 
+# --- per-channel B / C read in 16-byte loads --------------------------------------
+
+@pytest.mark.parametrize("io,tol", [(torch.float32, TOL_F32), (torch.bfloat16, 2e-2)])
+def test_per_channel_rows_of_any_alignment(io, tol):
+    # Whole rows; from an odd element on; channels 17 elements apart: the same
+    # values, so the same bits, and the oracle's to rounding.
+    Bsz, L, D = 2, 1001, 40
+    x, dt, A, _, _ = scan1d_inputs(Bsz, L, D, N, seed=34)
+    g = rng_for("alignment", L)
+    Bm, Cm = ((g.standard_normal((Bsz, L, D, N)) * 0.25).astype(np.float32) for _ in range(2))
+    dy = g.standard_normal((Bsz, L, D)).astype(np.float32)
+    st = (L * D * N, D * N, N)
+    xd, dtd, dyd = (T(a, io) for a in (x, dt, dy))
+    runs = []
+    for first, gap in ((0, N), (1, N), (0, N + 1)):
+        flat = [torch.zeros(first + Bsz * L * D * gap, dtype=io, device=DEV) for _ in range(4)]
+        M = [f[first:] for f in flat]
+        for m, a in zip(M, (Bm, Cm)):
+            m.view(Bsz, L, D, gap)[..., :N] = T(a, io)
+        stg = (L * D * gap, D * gap, gap)
+        y, hf = torch.empty_like(xd), torch.empty((Bsz, D, N), device=DEV)
+        K.scan1d_fwd(xd, dtd, T(A), M[0], M[1], y, h_final=hf, bc_strides=stg)
+        dx, ddt, dA = torch.empty_like(xd), torch.empty_like(xd), torch.empty((D, N), device=DEV)
+        K.scan1d_bwd(xd, dtd, T(A), M[0], M[1], dyd, dx, ddt, dA, M[2], M[3], bc_strides=stg)
+        runs.append([y, hf, dx, ddt, dA] + [m.view(Bsz, L, D, gap)[..., :N].clone() for m in M[2:]])
+    for other in runs[1:]:
+        for a, b in zip(runs[0], other):
+            assert torch.equal(a, b)
+    yr, hr, _ = O.scan1d_batched(x, dt, A, Bm, Cm, bc_strides=st)
+    ky, kh, _ = scan1d_kappa(x, dt, A, Bm, Cm, bc_strides=st)
+    assert_close(runs[0][0].float().cpu().numpy(), yr, tol, "y", ky)
+    assert_close(runs[0][1].cpu().numpy(), hr, tol, "h_final", kh)
+
+
 # --- decays over a whole segment that are out of range -----------------------------
 
 def _growing(Bsz, L, D, kind):
