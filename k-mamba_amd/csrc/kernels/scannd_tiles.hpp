@@ -70,9 +70,11 @@ constexpr long kSmallFront = 768;
 // The critical path of a tiling (us): its fronts, each a hand-over and the
 // tile's rows of 8 points one after the other. Smaller tiles shorten it where
 // they split a plane, not where they only split axis 0 (an axis of 3 or 7 rows
-// is one tile, or two of 4, either way). M = 16, D64, pencils / small tiles:
+// is one tile, or two of 4, either way), and not on a grid of one column of
+// tiles, whose pencil hands nothing over. M = 16, D64, pencils / small tiles:
 // 700x8x8 3270 / 2035, 8x8x600 1490 / 520, but 400x7x8 1850 / 2005, 100x3x3 320
-// / 357, 60x7x7 296 / 312.
+// / 357, 60x7x7 296 / 312; 9x3x4 D320 M = 1 36.5 / 39.2. (By 5 %: the model's
+// error; 30x3x16 D64, 2 % shorter by it, 119 / 129.)
 inline double nd_path_us(long nbands, const int *tile) { return nbands * (1.6 + 1.05 * tile[0] * tile[1]); }
 // Sets tile and ntile to the 2 x 2 x `row` tiles (axis 1 may have more rows,
 // see nd_tiles) and returns true where they are the faster ones for ncg channel
@@ -85,8 +87,8 @@ inline bool nd_small_tiles(const int *dims, int row, long ncg, size_t max_flags,
     const double path4 = nd_path_us(nd_tiles(3, dims, row, 4, tile4, ntile4), tile4);
     const long nbands = nd_tiles(3, dims, row, 2, tile, ntile);
     const long n = static_cast<long>(ntile[0]) * ntile[1] * ntile[2] * ncg;
-    return nbands <= kMaxFlowBands && n <= kSmallFront * nbands && nd_path_us(nbands, tile) < path4 &&
-           static_cast<size_t>(n) <= max_flags;
+    return nbands <= kMaxFlowBands && n <= kSmallFront * nbands && nd_path_us(nbands, tile) < 0.95 * path4 &&
+           ntile[1] * ntile[2] > 1 && static_cast<size_t>(n) <= max_flags;
 }
 
 }  // namespace km

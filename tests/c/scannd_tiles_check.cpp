@@ -46,7 +46,7 @@ int main() {
                 }
     // Both sides of the rule, as they measured.
     const int faster[][3] = {{700, 8, 8}, {8, 8, 600}, {7, 7, 60}, {100, 9, 8}, {32, 32, 32}, {20, 19, 23}};
-    const int slower[][3] = {{400, 7, 8}, {60, 7, 7}, {100, 7, 16}, {3, 4, 5}, {100, 3, 3}, {2000, 8, 8}};
+    const int slower[][3] = {{400, 7, 8}, {60, 7, 7}, {100, 7, 16}, {3, 4, 5}, {100, 3, 3}, {2000, 8, 8}, {9, 3, 4}, {6, 2, 2}, {30, 3, 16}};
     int tile[3], ntile[3];
     for (const auto &d : faster)
         if (!km::nd_small_tiles(d, 8, 16, SIZE_MAX, tile, ntile)) return std::printf("%dx%dx%d\n", d[0], d[1], d[2]);
