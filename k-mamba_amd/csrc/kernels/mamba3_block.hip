@@ -65,7 +65,7 @@ __global__ void __launch_bounds__(256) m3_proj(M3Args p) {
     __shared__ float sx[2][kPK][kPT + kPPad];
     __shared__ float sw[2][kPK][kPJ + kPPad];
     const int tid = threadIdx.x;
-    const int ty = tid / 16, tx = tid % 16;            // 4 tokens x 4 rows each
+    const int ty = tid / 16, tx = tid % 16;            // tokens 4 tx .. + 3, rows 4 ty .. + 3
     const long t0 = static_cast<long>(blockIdx.x) * kPT;
     const long j0 = static_cast<long>(blockIdx.y) * kPJ;
     const bool vec = (p.D % 4) == 0;
@@ -114,8 +114,8 @@ __global__ void __launch_bounds__(256) m3_proj(M3Args p) {
         if (ks + 1 < nk) gload((ks + 1) * kPK);
 #pragma unroll 8
         for (int kk = 0; kk < kPK; ++kk) {
-            const float4 xv = *reinterpret_cast<const float4 *>(&sx[buf][kk][ty * 4]);
-            const float4 wv = *reinterpret_cast<const float4 *>(&sw[buf][kk][tx * 4]);
+            const float4 xv = *reinterpret_cast<const float4 *>(&sx[buf][kk][tx * 4]);
+            const float4 wv = *reinterpret_cast<const float4 *>(&sw[buf][kk][ty * 4]);
             const float xa[4] = {xv.x, xv.y, xv.z, xv.w}, wa[4] = {wv.x, wv.y, wv.z, wv.w};
 #pragma unroll
             for (int i = 0; i < 4; ++i)
@@ -126,14 +126,12 @@ __global__ void __launch_bounds__(256) m3_proj(M3Args p) {
         __syncthreads();
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const long t = t0 + ty * 4 + i;
-        if (t >= p.T) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const long jj = j0 + tx * 4 + j;
-            if (jj < p.J) p.P[jj * p.Tp + t] = acc[i][j];
-        }
+    for (int j = 0; j < 4; ++j) {
+        // Four steps of a row at once (Tp holds whole tiles of 64 tokens).
+        const long jj = j0 + ty * 4 + j;
+        if (jj < p.J)
+            *reinterpret_cast<float4 *>(p.P + jj * p.Tp + t0 + tx * 4) =
+                make_float4(acc[0][j], acc[1][j], acc[2][j], acc[3][j]);
     }
 }
 
@@ -240,12 +238,31 @@ __device__ __forceinline__ void m3_ctrl(const M3Args &p, float rd, float rl, flo
     lam = p.has_lambda ? 1.f / (1.f + expf(-rl)) : 0.5f;
 }
 
-// Bu_t[n] = sum_r (W_B x_t + b_B)[r, n] * SiLU(W_in x_t)[r].
-__device__ __forceinline__ float m3_bu(const M3Args &p, long t, long n) {
-    float s = 0.f;
-    for (long r = 0; r < p.R; ++r)
-        s += (p.P[(p.R + 2 + r * p.N + n) * p.Tp + t] + p.bB[r * p.N + n]) * silu_f(p.P[r * p.Tp + t]);
-    return s;
+// Bu_t[n] = sum_r (W_B x_t + b_B)[r, n] * SiLU(W_in x_t)[r] of the steps t and tp,
+// four ranks' loads together (each is a line of its own).
+__device__ __forceinline__ void m3_bu(const M3Args &p, long t, long tp, long n, float &bu, float &bp) {
+    constexpr int RB = 4;
+    bu = bp = 0.f;
+    for (long r0 = 0; r0 < p.R; r0 += RB) {
+        float z[RB], zp[RB], x[RB], xp[RB], c[RB];
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            const long r = min(r0 + i, p.R - 1);
+            const float *const row = p.P + (p.R + 2 + r * p.N + n) * p.Tp;
+            z[i] = p.P[r * p.Tp + t];
+            zp[i] = p.P[r * p.Tp + tp];
+            x[i] = row[t];
+            xp[i] = row[tp];
+            c[i] = p.bB[r * p.N + n];
+        }
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            if (r0 + i < p.R) {
+                bu += (x[i] + c[i]) * silu_f(z[i]);
+                bp += (xp[i] + c[i]) * silu_f(zp[i]);
+            }
+        }
+    }
 }
 
 // Both of every step and state, for m3_scan<PREP>: whole chip, time along the
@@ -257,8 +274,10 @@ __global__ void __launch_bounds__(256) m3_prep(M3Args p) {
     float dt, lam;
     m3_ctrl(p, p.P[p.R * p.Tp + t], p.P[(p.R + 1) * p.Tp + t], dt, lam);
     const float alpha = expf(dt * p.A[n]);
-    const float bu = m3_bu(p, t, n);
-    const float pbu = t % p.L > 0 ? m3_bu(p, t - 1, n) : 0.f;
+    const bool prev = t % p.L > 0;
+    float bu, pbu;
+    m3_bu(p, t, prev ? t - 1 : t, n, bu, pbu);
+    if (!prev) pbu = 0.f;
     p.a[i] = alpha;
     p.c[i] = (1.f - lam) * dt * alpha * pbu + lam * dt * bu;
 }
@@ -444,8 +463,22 @@ __global__ void __launch_bounds__(256) m3_readout(M3Args p) {
     const long r = i / p.Tp, t = i - r * p.Tp;
     if (r >= p.R || t >= p.T) return;
     const float *C = p.P + (p.R + 2 + p.N * p.R + r * p.N) * p.Tp + t;
+    // Eight states' loads together (each is a line of its own).
+    constexpr int NB = 8;
     float s = 0.f;
-    for (long n = 0; n < p.N; ++n) s = fmaf(C[n * p.Tp] + p.bC[r * p.N + n], p.H[n * p.Tp + t], s);
+    for (long n0 = 0; n0 < p.N; n0 += NB) {
+        float c[NB], h[NB], b[NB];
+#pragma unroll
+        for (int k = 0; k < NB; ++k) {
+            const long n = min(n0 + k, p.N - 1);
+            c[k] = C[n * p.Tp];
+            h[k] = p.H[n * p.Tp + t];
+            b[k] = p.bC[r * p.N + n];
+        }
+#pragma unroll
+        for (int k = 0; k < NB; ++k)
+            if (n0 + k < p.N) s = fmaf(c[k] + b[k], h[k], s);
+    }
     p.Y[i] = s;
 }
 
@@ -454,6 +487,7 @@ __global__ void __launch_bounds__(256) m3_out(M3Args p) {
     if (i >= p.T * p.D) return;
     const long t = i / p.D, d = i % p.D;
     float s = 0.f;
+#pragma unroll 4
     for (long r = 0; r < p.R; ++r) s = fmaf(p.W_out[d * p.R + r], p.Y[r * p.Tp + t], s);
     p.out[i] = p.x[i] + s;
 }
