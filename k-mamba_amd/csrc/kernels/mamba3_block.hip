@@ -837,7 +837,8 @@ void mamba_block_forward(MambaBlock *b, float *output, const float *input, size_
         float *x = dev_io ? const_cast<float *>(input) : cv.take<float>(T * D);
         float *o = dev_io ? output : cv.take<float>(T * D);
         // Parameters live in host memory (the reference layout): pack them
-        // into one pinned block and upload it with a single copy.
+        // into one pinned block, from which a kernel (large blocks: a DMA copy)
+        // brings them to the device.
         const size_t nW = static_cast<size_t>(J * D), nO = static_cast<size_t>(D * R);
         const size_t nP = nW + nO + N + 2 * NR + TS;
         float *dpar = cv.take<float>(nP);

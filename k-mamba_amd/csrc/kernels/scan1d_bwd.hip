@@ -326,9 +326,8 @@ __global__ void __launch_bounds__(HWT == 2 ? 1024 : 512, 4) scan1d_bwd_chunked(S
     };
 
     // The adjoint entering the workgroup's last step, state w by wave w (the
-    // clamped re-run finds it again in the dA partial, which is written
-    // last): zero,
-    // or the fold of the maps after a segment, last first,
+    // clamped re-run finds it again in the dA partial, which is written last):
+    // zero, or the fold of the maps after a segment, last first,
     // g <- exp(A * sum delta) g + g_end. kFoldRun maps' loads are in flight
     // together.
     if constexpr (SEG) {

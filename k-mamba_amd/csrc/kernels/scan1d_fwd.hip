@@ -56,9 +56,9 @@ struct Scan1DFwdArgs {
     long B, L, D, N;
     long sb, st, sd;
     int clamp;
-    // Segmented launches (the sequence split over workgroups): the grid holds
-    // nseg workgroups per (batch, group), workgroup sg on steps [sg * Ls,
-    // min(L, (sg + 1) * Ls)). nseg = 1 with Ls = L otherwise.
+    // Segmented launches (the sequence split over workgroups, the kernel built
+    // with SEG): the grid holds nseg workgroups per (batch, group), workgroup sg
+    // on steps [sg * Ls, min(L, (sg + 1) * Ls)).
     int nseg, Ls;
     // A workgroup of a segmented launch whose states leave [-1000, 1000] sets
     // clamp_flag[b * groups + group] and leaves the sequential re-run to
@@ -713,11 +713,14 @@ constexpr int kMaxSegments = 64;
 // split launch, or 0 to run unsplit. Only N = 16, and only when the unsplit
 // grid leaves CUs idle. The model, from gfx950 timings of the 8-wave kernel
 // with one workgroup per CU: a launch of n workgroups over c 64-step chunks
-// takes (4 + 2.1 c) ceil(n / 256) us, and a split runs two of them, plus
-// ~6 us for the clamp check and the launches; it is taken when it wins 15 %.
-// B1 L5003 D1536 bf16 gated (48 groups): 72.4 us in 5 segments, 195.7 us
-// unsplit; B1 L1920 D768 fp32 (24): 29.5 in 10, 68.8; B2 L1920 D1536 fp32
-// (96): 71.7 in 5 against 69.6 unsplit, which the model keeps.
+// takes (4 + 2.1 c) ceil(n / 256) us. A split is priced as two of them plus
+// ~6 us for the clamp check and the launches, and taken when it wins 15 %. That
+// is dear: the map pass takes 0.35 to 0.45 of the replay (B1 L5003 D1536 bf16
+// gated 22 and 54 us), so a split that is taken wins by more than the model says
+// and some that would win are not. B1 L5003 D1536 bf16 gated (48 groups): 69.2
+// us in 5 segments, 196 unsplit; B1 L1920 D768 fp32 (24): 25.1 in 10, 69.0; but
+// B2 L1920 D1536 fp32 (96) stays at 69.5, with 53.0 in 2, and B3 L4096 D1000 (96)
+// at 139, with 98.8 in 8.
 static long segment_length(const KMScan1DFwd *k, long groups_total) {
     if (k->N != 16 || groups_total >= 128 || k->L < 128) return 0;
     const long ov = scan1d_split_override();

@@ -33,7 +33,7 @@
 // chain), 17x19 D16 34.5 -> 17.4, 200x190 D48 399 -> 285; 256x256 D256, which
 // fills the chip either way, 949 -> 870 (4.0 TB/s). Blocks in flight on the
 // last two: 3: 300, 965; 4: 285, 870; 5: 287, 866; 6 (spills): 286, 877.
-// Forward and backward, tiles in both -> strips in both: 45x61 D96 401 -> 144
+// Forward and backward, tiles in both -> strips in both: 45x61 D96 401 -> 150
 // (221 with the forward's alone), 12x250 D48 719 -> 126, 30x24 D32 153 -> 80,
 // 250x12 D48 381 -> 292, one row of 600 802 -> 102, one column of 600 568 -> 97.
 #pragma once
