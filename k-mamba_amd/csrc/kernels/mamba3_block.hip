@@ -493,10 +493,10 @@ __global__ void __launch_bounds__(256) m3_out(M3Args p) {
 }
 
 // Tokens of an output workgroup, and the ranks up to which it forms Y itself:
-// its ranks' sums come one after the other, which from 16 ranks on costs more
-// than a launch. D 256, N 16, whole call (us), Y here / in m3_readout: T 2048 R8
-// 54.7 / 57.1, R16 80.8 / 78.3, R24 106.8 / 99.9, R64 241 / 214; T 65536 R12
-// 312 / 321, R32 829 / 776.
+// its ranks' sums come one after the other, which costs more than a launch from
+// 8 ranks on for few tokens, from 16 on for many. D 256, N 16, whole call (us), Y
+// here / in m3_readout: T 2048 R8 54.5 / 53.2, R16 76.1 / 70.6, R24 99.5 / 90.3,
+// R64 225 / 196; T 65536 R8 231 / 236, R12 309 / 316, R16 396 / 394, R32 806 / 740.
 constexpr int kM3OutT = 16, kM3OutR = 16;
 // The token group of a workgroup: the grid's y, and z past its 65535.
 __device__ __forceinline__ long m3_out_t0() {
@@ -624,11 +624,11 @@ static long grid256(long n) { return (n + 255) / 256; }
 // the scan's own threads (twice the states, not the steps, apart). Few scan
 // workgroups (one per batch element and pair): their time is R loads and drives
 // for every chunk of a thread in turn, against one more launch. Scan / m3_prep,
-// N 16, whole call (us): B1 R1 L1000 34.3 / 35.3, L4096 49.0 / 45.4, L16384 114
-// / 90; B1 L2048 R4 53.4 / 46.9, R16 120 / 87. Enough of them to fill the chip:
-// the scan's own, B64 L2048 R1 128 / 139, R2 203 / 213, unless there are many
-// ranks (B64 L256 R8 93.1 / 88.6) or sequences so short that most of a
-// workgroup idles (B4000 L16 R1 226 / 143).
+// dim 256, N 16, whole call (us): B1 R1 L1000 33.7 / 34.6, L4096 48.4 / 44.9,
+// L16384 113 / 90; B1 L2048 R4 53.0 / 44.7, R16 120 / 81. Enough of them to fill
+// the chip: the scan's own, B64 L2048 R1 126 / 143, R2 202 / 213, unless there
+// are many ranks (B64 L256 R8 91.8 / 87.1) or sequences so short that most of a
+// workgroup idles (B4000 L16 R1 308 / 143).
 static bool m3_prep_wanted(long B, long L, long N, long R) {
     const long wgs = B * ((N + 1) / 2);
     if (wgs < 256) return R * ((L + 255) / 256) > 8;

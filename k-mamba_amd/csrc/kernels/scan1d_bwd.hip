@@ -1049,8 +1049,8 @@ static bool bwd_wide(long B, long D) {
 // 14) of prologue and uneven ends; the finalize reads the slots at 4.7 TB/s; a
 // split adds the map pass (3.8 VALU instructions per state update) and ~12 of
 // launch, fold and partials. Taken when it wins 10 %. Training step (forward
-// and backward): B1 L4096 D1024 fp32 461 -> 145 us (8 segments), B2 L1999 D768
-// bf16 249 -> 126, B4 L4096 D1024 fp32 479 -> 437, B9 L2000 D1024 fp32 (288
+// and backward): B1 L4096 D1024 fp32 461 -> 138 us (8 segments), B2 L1999 D768
+// bf16 249 -> 126, B4 L4096 D1024 fp32 479 -> 428, B9 L2000 D1024 fp32 (288
 // workgroups, 1.1 rounds) 656 -> 567.
 constexpr long kMaxBwdSegments = 64;
 static void bwd_segments(const KMScan1DBwd *k, BwdPlan &pl) {
