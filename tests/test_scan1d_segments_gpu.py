@@ -354,3 +354,30 @@ def test_mamba1_block_with_workspace_takes_no_scratch(whole):
     torch.cuda.synchronize()
     # Split or not: the scan's fp32 sums in another order, rounded to bf16 once.
     assert (out.float() - want.float()).norm() <= (1e-6 if whole else 4e-3) * want.float().norm()
+
+
+def test_captured_backward_with_workspace():
+    # The split's scratch is the caller's: forward (states again) and backward are
+    # split inside a capture too, and each replay equals an eager call.
+    Bsz, L, D = 1, 1001, 64
+    x, dt, A, Bm, Cm = (T(a) for a in scan1d_inputs(Bsz, L, D, N, seed=63))
+    dy = T(rng_for("graph-ws", L).standard_normal((Bsz, L, D)).astype(np.float32))
+    outs, want = ([torch.zeros_like(t) for t in (x, x, A, Bm, Cm)] for _ in range(2))
+    args = K.scan1d_bwd_args(x, dt, A, Bm, Cm, dy, *outs)
+    ws = torch.empty(K.km_scan1d_bwd_workspace_bytes(C.byref(args)), dtype=torch.uint8, device=DEV)
+    args = K.scan1d_bwd_args(x, dt, A, Bm, Cm, dy, *outs, workspace=ws)
+    s = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    held = K.km_device_bytes_held()
+    with torch.cuda.graph(g, stream=s):
+        assert K.km_scan1d_bwd_c(C.byref(args), C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    assert K.km_device_bytes_held() == held
+    for i in range(3):
+        x.copy_(T(rng_for("graph-ws-x", i).standard_normal((Bsz, L, D)).astype(np.float32)))
+        g.replay()
+        torch.cuda.synchronize()
+        K.scan1d_bwd(x, dt, A, Bm, Cm, dy, *want)
+        torch.cuda.synchronize()
+        for a, b in zip(outs, want):
+            assert torch.isfinite(a).all() and torch.equal(a, b)
